@@ -1,5 +1,7 @@
 // Store build: 4-bit quantiser, bit-plane packers and the channel-major
-// nibble store of the chan4 baseline (lane = channel layout).
+// nibble store of the chan4 baseline (lane = channel layout).  Rows of D = 128
+// take quantise.hip's kernels; those here serve other D, unaligned buffers and
+// the nibble store.
 //
 // A wave owns 64 consecutive channels of one 64-token block: every key load is
 // a coalesced row segment, each lane keeps its channel's 64 values in
@@ -7,7 +9,7 @@
 // plane words in registers (bit i = token 64b+i).  A workgroup of 4 waves
 // walks 16 consecutive blocks so each (channel, plane) 128-byte superblock unit
 // is written by one workgroup (one XCD's L2).
-#include "common.hpp"
+#include "pack_internal.hpp"
 
 namespace fathom {
 namespace {
@@ -311,6 +313,8 @@ extern "C" int fathom_quantise_pack(const void *K, int k_dtype, int64_t lead, in
   int rc = check_grid(lead, D, cover, "quantise_pack");
   if (rc) return rc;
   if (!code && !scales_blk && !planes_log && !planes_sb) return FATHOM_OK;
+  const pack::QuantArgs qa{K, n, nblk, cover, sub, nsb, scale_dtype, code, scales_blk, planes_log, planes_sb, scales_sb};
+  if (pack::quantise128_accepts(qa, k_dtype, D)) return pack::quantise128(qa, k_dtype, lead, (hipStream_t)stream);
   return quantise_dispatch<false>(K, k_dtype, lead, n, D, scale_dtype, nblk, cover, sub, nsb, code, scales_blk,
                                   planes_log, planes_sb, scales_sb, nullptr, (hipStream_t)stream);
 }
@@ -350,6 +354,7 @@ extern "C" int fathom_pack_planes(const uint8_t *code, int64_t lead, int64_t n, 
   const int64_t nblk = cdiv(n, kBlk);
   int rc = check_grid(lead, D, nblk, "pack_planes");
   if (rc) return rc;
+  if (pack::pack128_accepts(code, D, planes)) return pack::pack128(code, lead, n, planes, (hipStream_t)stream);
   dim3 grid((unsigned)cdiv(nblk, kBlocksPerWG), (unsigned)cdiv(D, 64), (unsigned)lead);
   pack_planes_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(code, n, D, nblk, planes);
   return launch_status("pack_planes_kernel");

@@ -1,0 +1,64 @@
+"""Store builders of D = 128 rows at the edges of their tiles: codes, scales and plane words equal the oracle's bit for
+bit, whichever of the workgroup shapes the size picks."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from fathom_amd import bitplane as bp
+from oracle import fathom_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+SDT = {"f16": torch.float16, "f32": torch.float32, "bf16": torch.bfloat16}
+
+
+def _edge_keys(BH, n, dtype, seed):
+    """Random keys, and per channel the quotient's edges: multiples of the block's scale step and the representable
+    values next to them, both signs."""
+    g = torch.Generator().manual_seed(seed)
+    K = torch.randn(BH, n, 128, generator=g) * torch.exp(2 * torch.randn(BH, 1, 128, generator=g))
+    K = K.to(dtype)
+    a = K.float().abs().reshape(BH, n, 128)[:, :64].amax(1)          # the first block's absmax
+    step = a.half().float() / 8
+    m = torch.arange(-8, 9, dtype=torch.float32)
+    at = (m[None, :, None] * step[:, None, :]).to(dtype)
+    near = [at, torch.nextafter(at, torch.full_like(at, math.inf)), torch.nextafter(at, torch.full_like(at, -math.inf))]
+    rows = torch.cat(near, 1)                                        # [BH, 51, 128]
+    rows = torch.where(rows.float().abs() <= a[:, None], rows, torch.zeros((), dtype=dtype))
+    K[:, 5:56] = rows[:, :min(51, n - 5)]
+    return K
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("sdt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("BH,n,sub", [(1, 64, 16), (2, 1000, 3), (3, 65536 + 33, 16), (9, 7777, 64), (1, 1049000, 0),
+                                      (2, 530000, 5)])
+def test_build_equals_oracle_at_tile_edges(BH, n, sub, sdt, dtype, monkeypatch):
+    print(f"[build] {BH}x{n} sub={sub} {sdt} {dtype}", flush=True)
+    nb = -(-n // 64)
+    monkeypatch.setattr(bp, "SUB", sub or nb)
+    K = _edge_keys(BH, n, dtype, n)
+    if n > 500000:                          # the large shapes' rows repeat their head: the oracle is slow
+        K[:, 8192:] = K[:, :8192].repeat(1, -(-n // 8192), 1)[:, 8192:n]
+    st = bp.PlaneStore(K.to(DEV), scale_dtype=SDT[sdt])
+    lean = bp.PlaneStore(K.to(DEV), scale_dtype=SDT[sdt], keep_code=False)
+    torch.cuda.synchronize()
+    assert torch.equal(st.planes_k, lean.planes_k) and torch.equal(st.scales_k, lean.scales_k)
+    assert torch.equal(bp.unpack_planes(bp.pack_planes(st.code), n), st.code)
+    pl, sc = bp.to_superblocks(bp.pack_planes(st.code), st.scales_blk)
+    assert torch.equal(pl, st.planes_k)
+    if sdt == "f16":
+        assert torch.equal(sc, st.scales_k)
+    keep = min(n, 8192 if n > 500000 else n)
+    head = K[:, :keep].float().numpy()
+    code_r, sc_r = O.quantise_u4(head, sdt)
+    np.testing.assert_array_equal(st.code[:, :keep].cpu().numpy(), code_r)
+    np.testing.assert_array_equal(st.scales_blk[:, :-(-keep // 64)].float().cpu().numpy(), sc_r)
+    tail = (n - 1) // 64 * 64               # the last, ragged block
+    code_t, sc_t = O.quantise_u4(K[:, tail:].float().numpy(), sdt)
+    np.testing.assert_array_equal(st.code[:, tail:].cpu().numpy(), code_t)
+    np.testing.assert_array_equal(st.scales_blk[:, -1:].float().cpu().numpy(), sc_t)
+    planes = bp.pack_planes(st.code[:, tail:].contiguous())
+    np.testing.assert_array_equal(planes.cpu().numpy().view(np.uint64), O.pack_planes(code_t))
