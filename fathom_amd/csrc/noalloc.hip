@@ -2,7 +2,8 @@
 // under graph capture, tight serving loops, harnesses that forbid hipMalloc).
 //
 // Its workspace is `scratch`, a static device array of this library of
-// FATHOM_NOALLOC_SCRATCH_BYTES: each device holds its own copy from the first
+// FATHOM_NOALLOC_SCRATCH_BYTES (and room to pad short rows to whole blocks, which
+// the limit does not count): each device holds its own copy from the first
 // call on that device until the process ends.  Host code never passes the
 // array's name to a kernel (on the host it is a stand-in, not a device
 // address): the first call on a device looks its address up with
@@ -23,7 +24,9 @@
 namespace fathom {
 namespace {
 
-constexpr size_t kScratchBytes = (size_t)FATHOM_NOALLOC_SCRATCH_BYTES;
+constexpr size_t kScratchLimit = (size_t)FATHOM_NOALLOC_SCRATCH_BYTES;
+constexpr size_t kScratchBytes = kScratchLimit + (17u << 20);
+static_assert(kScratchBytes - kScratchLimit >= 65535u * (kBlk - 1) * 4u + 256u, "the padding of 65535 rows");
 static_assert(kScratchBytes % 256 == 0, "scratch is a whole number of 256-byte sections");
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -72,12 +75,12 @@ extern "C" int fathom_scan_topk_noalloc(const float *q, int64_t BH, int64_t G, i
   if (k - sink - local == 0)
     return scan_topk_run(q, BH, G, D, cls, clsn, bmax, units_max, planes_sb, scales_sb, n, nsb, sub, m, k, sink,
                          local, idx, nullptr, 0, FATHOM_STAGE_ALL, stream);
-  const size_t need = scan_topk_ws(BH * G, n, k, k - sink - local);
-  if (need > kScratchBytes)
+  const size_t need = scan_topk_ws(BH * G, n, k, k - sink - local, false);
+  if (need > kScratchLimit)
     return fail(FATHOM_ERR_WORKSPACE,
                 "scan_topk_noalloc: BH=%lld G=%lld n=%lld k=%lld needs %zu bytes of scratch, the static array holds "
                 "%zu (use fathom_scan_topk with a caller workspace)",
-                (long long)BH, (long long)G, (long long)n, (long long)k, need, kScratchBytes);
+                (long long)BH, (long long)G, (long long)n, (long long)k, need, kScratchLimit);
   void *ws = nullptr;
   rc = scratch_on_current_device(&ws);
   if (rc) return rc;

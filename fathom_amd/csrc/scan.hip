@@ -22,8 +22,8 @@ using namespace sc;
 // larger plan keeps over its register groups (4: fewer reloads, more
 // registers).  The scores are the same for any
 // choice; the launch picks them from the plan's units bound.  HOST (the
-// candidate pass over a store in mapped host memory, superblocks of a
-// multiple of 64 blocks): workgroups stage groups of four wave-tiles in LDS
+// candidate pass and the scores with group maxima over a store in mapped host
+// memory, superblocks of a multiple of 64 blocks): workgroups stage groups of four wave-tiles in LDS
 // (two workgroups per CU).
 template <int MODE, int NSMAX, int ACC, bool HOST = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(
@@ -55,7 +55,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(
     constexpr bool kCand = MODE == kEmitFilter;
     const int64_t nlist = kCand && em.sel.nreg > a.nwt ? em.sel.nreg : a.nwt;
     if constexpr (HOST) {
-      static_assert(kCand, "staged host tiles in the candidate pass");
       const int nsl = __builtin_amdgcn_readfirstlane(sh.U) / kSlice;
       const int ureal = __builtin_amdgcn_readfirstlane(sh.ureal);
       if (nsl <= NSMAX) {  // uniform; larger plans read the store directly
@@ -94,21 +93,22 @@ int launch_scan(const ScanArgs &a0, int64_t nwt, int64_t BH, const Emit &em, int
     wgs = cdiv(cdiv(nwt, per), kWaves);
   }
   // the layout of stores in mapped host memory (superblocks of a multiple of
-  // 64 blocks, shorter than the row; 16-byte aligned): the candidate pass
-  // stages its tiles, two workgroups per CU.  The whole-row layout of the
+  // 64 blocks, shorter than the row; 16-byte aligned): the passes over
+  // long rows stage their tiles, two workgroups per CU.  The whole-row layout of the
   // copy-index staging store (in HBM) reads directly.
-  const bool host = MODE == kEmitFilter && nsl <= kGS && a.sub % kHostBlk == 0 && a.sub < cdiv(a.n, kBlk) &&
+  constexpr bool kStaged = MODE == kEmitFilter || emits_max(MODE);
+  const bool host = kStaged && a.n > kRowSelectMax && nsl <= kGS && a.sub % kHostBlk == 0 && a.sub < cdiv(a.n, kBlk) &&
                     (reinterpret_cast<uintptr_t>(a.planes) & 15) == 0 && (reinterpret_cast<uintptr_t>(a.scales) & 15) == 0;
   if (host) {
     const int64_t per = cdiv(nwt * BH, kTargetWaves / 2);
     const dim3 hgrid((unsigned)cdiv(cdiv(nwt, per), kWaves), (unsigned)BH);
-    if (MODE == kEmitFilter) {
+    if constexpr (kStaged) {
       if (nsl == 4)
-        scan_wave_kernel<kEmitFilter, 4, 1, true><<<hgrid, kThreads, 0, st>>>(a, em, split);
+        scan_wave_kernel<MODE, 4, 1, true><<<hgrid, kThreads, 0, st>>>(a, em, 0);
       else if (nsl == 3)
-        scan_wave_kernel<kEmitFilter, 3, 1, true><<<hgrid, kThreads, 0, st>>>(a, em, split);
+        scan_wave_kernel<MODE, 3, 1, true><<<hgrid, kThreads, 0, st>>>(a, em, 0);
       else
-        scan_wave_kernel<kEmitFilter, 2, 1, true><<<hgrid, kThreads, 0, st>>>(a, em, split);
+        scan_wave_kernel<MODE, 2, 1, true><<<hgrid, kThreads, 0, st>>>(a, em, 0);
     }
     return launch_status("scan_wave_kernel");
   }
@@ -122,6 +122,24 @@ int launch_scan(const ScanArgs &a0, int64_t nwt, int64_t BH, const Emit &em, int
   else
     scan_wave_kernel<MODE, 2, 1><<<grid, kThreads, 0, st>>>(a, em, split);
   return launch_status("scan_wave_kernel");
+}
+
+// The scores with group maxima, in the order the selection reads (quad_order).
+int launch_scores_max(const ScanArgs &a, int64_t nwt, int64_t BH, const Emit &em, int64_t units_max, hipStream_t st) {
+  return quad_order(a.G, a.n) ? launch_scan<kEmitQuadsMax>(a, nwt, BH, em, units_max, st)
+                              : launch_scan<kEmitScoresMax>(a, nwt, BH, em, units_max, st);
+}
+
+// Its emission into a workspace of scan_topk_ws bytes.
+Emit group_max_emit(int64_t rows, int64_t n, int64_t m, int64_t sink, int64_t local, void *workspace) {
+  Emit es{};
+  es.out = static_cast<float *>(workspace);
+  es.ostride = tile_score_floats(n);
+  es.gmax = reinterpret_cast<uint32_t *>(static_cast<char *>(workspace) +
+                                         ws_align((size_t)rows * (size_t)tile_score_floats(n) * 4));
+  es.sink = sink;
+  es.lstart = (m - local) > 0 ? (m - local) : 0;
+  return es;
 }
 
 // The plan's units bound: the caller's, else every channel at full depth.
@@ -196,19 +214,23 @@ extern "C" int fathom_scan_planes(const float *q, int64_t BH, int64_t G, int64_t
   a.wt0 = blk0 / kWB;
   Emit em{};
   em.out = out;
+  em.ostride = n;
   return launch_scan<kEmitScores>(a, cdiv(blk_end, kWB) - a.wt0, BH, em, units_bound(units_max, D, bmax),
                                   (hipStream_t)stream);
 }
 
 namespace fathom {
-// Workspace of the fused scan + top-k: rows up to kRowSelectMax keep their
-// scores ([rows, n] fp32) for one row-select launch; longer rows the sampled
+// Workspace of the fused scan + top-k: rows up to kGmaxSelectMax keep their
+// scores and group maxima for one selection launch; longer rows the sampled
 // keys, the candidate regions and the plan tables (one per row: at least one
-// per (batch, KV head)).  kk above kSelMaxK: the scores and the wide path's
+// per (batch, KV head); rows between kRowSelectMax and kGmaxSelectMax are given
+// this larger size too).  kk above kSelMaxK: the scores and the wide path's
 // selection state.
-size_t scan_topk_ws(int64_t rows, int64_t n, int64_t k, int64_t kk) {
+size_t scan_topk_ws(int64_t rows, int64_t n, int64_t k, int64_t kk, bool whole_blocks) {
   if (kk > kSelMaxK) return ws_align((size_t)rows * (size_t)n * 4) + wide_topk_bytes(rows, n, k);
-  if (n <= kRowSelectMax) return ws_align((size_t)rows * (size_t)n * 4) + ws_align((size_t)rows * cdiv(n, kGroupTok) * 4);
+  if (n <= kRowSelectMax)
+    return ws_align((size_t)rows * (size_t)(whole_blocks ? tile_score_floats(n) : n) * 4) +
+           ws_align((size_t)rows * cdiv(n, kGroupTok) * 4);
   return topk_layout(rows, n, k, true, nullptr, nullptr, nullptr, nullptr, nullptr) +
          ws_align((size_t)rows * sizeof(sc::PlanTab));
 }
@@ -252,6 +274,7 @@ int scan_topk_run(const float *q, int64_t BH, int64_t G, int64_t D, const int32_
     // its candidate lists (the finalize stage)
     Emit es{};
     es.out = static_cast<float *>(workspace);
+    es.ostride = n;
     const size_t sb = ws_align((size_t)rows * (size_t)n * 4);
     if (stages & FATHOM_STAGE_CANDIDATES) {
       rc = launch_scan<kEmitScores>(a, nwt, BH, es, um, st);
@@ -262,20 +285,16 @@ int scan_topk_run(const float *q, int64_t BH, int64_t G, int64_t D, const int32_
                                workspace_bytes - sb, st)
                : FATHOM_OK;
   }
-  if (n <= kRowSelectMax) {
-    // short rows: the scores and their 16-token group maxima in the workspace
-    // (the candidate stage), then the rows selected in one launch from the
-    // groups that can hold a top-kk key (the finalize stage)
-    Emit es{};
-    es.out = static_cast<float *>(workspace);
-    es.gmax = reinterpret_cast<uint32_t *>(static_cast<char *>(workspace) + ws_align((size_t)rows * (size_t)n * 4));
-    es.sink = sink;
-    es.lstart = (m - local) > 0 ? (m - local) : 0;
+  if (n <= kGmaxSelectMax) {
+    // the scores and their 16-token group maxima in the workspace (the
+    // candidate stage), then the rows selected in one launch from the groups
+    // that can hold a top-kk key (the finalize stage)
+    const Emit es = group_max_emit(rows, n, m, sink, local, workspace);
     if (stages & FATHOM_STAGE_CANDIDATES) {
-      rc = launch_scan<kEmitScoresMax>(a, nwt, BH, es, um, st);
+      rc = launch_scores_max(a, nwt, BH, es, um, st);
       if (rc) return rc;
     }
-    return (stages & FATHOM_STAGE_FINALIZE) ? launch_rowselect_gmax(es.out, es.gmax, rows, n, m, k, sink, local, idx, st)
+    return (stages & FATHOM_STAGE_FINALIZE) ? launch_rowselect_gmax(es.out, es.gmax, rows, G, n, m, k, sink, local, idx, st)
                                             : FATHOM_OK;
   }
   Emit em{};
@@ -372,7 +391,7 @@ int plan_scan_topk_run(const float *q, const float *g, const float *budget, floa
   hipStream_t st = (hipStream_t)stream;
   const int64_t kk = k - sink - local;
   const size_t sws = scan_topk_ws(rows, n, k, kk);
-  if (n > kRowSelectMax || kk == 0 || kk > kSelMaxK) {
+  if (n > kGmaxSelectMax || kk == 0 || kk > kSelMaxK) {
     // make_plan into the workspace, then the fused scan + top-k
     char *p = static_cast<char *>(workspace) + sws;
     int8_t *t = t_out ? t_out : reinterpret_cast<int8_t *>(p);
@@ -393,7 +412,7 @@ int plan_scan_topk_run(const float *q, const float *g, const float *budget, floa
     return scan_topk_run(q, BH, G, D, cls, clsn, bmax, units_max, planes_sb, scales_sb, n, nsb, sub, m, k, sink, local,
                          idx, workspace, sws, FATHOM_STAGE_ALL, stream);
   }
-  // short rows: every workgroup of the scan plans its row in the prologue
+  // every workgroup of the scan plans its row in the prologue
   // (the plan kernel's arithmetic), then the rows are selected as in scan_topk
   const int64_t nblk = cdiv(n, kBlk);
   ScanArgs a = make_args(q, G, D, nullptr, nullptr, bmax, planes_sb, scales_sb, n, nsb, sub);
@@ -405,17 +424,13 @@ int plan_scan_topk_run(const float *q, const float *g, const float *budget, floa
   a.budget_value = budget_value;
   a.iters = iters;
   a.t_out = t_out;
-  Emit es{};
-  es.out = static_cast<float *>(workspace);
-  es.gmax = reinterpret_cast<uint32_t *>(static_cast<char *>(workspace) + ws_align((size_t)rows * (size_t)n * 4));
-  es.sink = sink;
-  es.lstart = (m - local) > 0 ? (m - local) : 0;
-  rc = launch_scan<kEmitScoresMax>(a, cdiv(nblk, kWB), BH, es, units_bound(units_max, D, bmax), st);
+  const Emit es = group_max_emit(rows, n, m, sink, local, workspace);
+  rc = launch_scores_max(a, cdiv(nblk, kWB), BH, es, units_bound(units_max, D, bmax), st);
   if (rc) return rc;
   if (att)  // the selection's workgroups go on to their head's attention
     return launch_rowselect_gmax_attn(es.out, es.gmax, rows, n, m, k, sink, local, idx, q, G, att->K, att->V, att->cap,
                                       att->scale, att->out, st);
-  return launch_rowselect_gmax(es.out, es.gmax, rows, n, m, k, sink, local, idx, st);
+  return launch_rowselect_gmax(es.out, es.gmax, rows, G, n, m, k, sink, local, idx, st);
 }
 }  // namespace
 }  // namespace fathom
@@ -452,7 +467,7 @@ extern "C" int fathom_plan_scan_topk_attention(const float *q, const float *g, c
   const int64_t kk = k - sink - local;
   // fused where gather_attention would take one 16-wave split per head, so
   // the outputs are the two calls' bit for bit
-  const bool fused = n <= kRowSelectMax && kk > 0 && k <= 512 && attn::attn_wide(BH, G, k) &&
+  const bool fused = n <= kGmaxSelectMax && kk > 0 && k <= 512 && attn::attn_wide(BH, G, k) &&
                      ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(Ksrc) |
                        reinterpret_cast<uintptr_t>(Vsrc)) & 7) == 0;
   if (fused) {

@@ -66,7 +66,9 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-enum : int { kEmitScores = 0, kEmitSample = 1, kEmitFilter = 2, kEmitScoresMax = 3 };
+enum : int { kEmitScores = 0, kEmitSample = 1, kEmitFilter = 2, kEmitScoresMax = 3, kEmitQuadsMax = 4 };
+// the modes that write group maxima beside the scores (kEmitQuadsMax: in quad order)
+constexpr bool emits_max(int mode) { return mode == kEmitScoresMax || mode == kEmitQuadsMax; }
 
 struct ScanArgs {
   const float *q;          // [BH, G, D]
@@ -93,8 +95,9 @@ struct ScanArgs {
 struct PlanTab;
 
 struct Emit {
-  float *out;        // scores [BH, G, n]
-  uint32_t *gmax;    // kEmitScoresMax: [BH * G, ceil(n / 16)] each 16-token group's largest masked key
+  float *out;        // scores [BH, G] rows of ostride floats (kEmitQuadsMax: quad order)
+  int64_t ostride;   // n, or whole blocks (kEmitScoresMax)
+  uint32_t *gmax;    // kEmitScoresMax, kEmitQuadsMax: [BH * G, ceil(n / 16)] each 16-token group's largest masked key
   uint32_t *samp;    // sampled keys [BH * G, samp_cap]: list entry L at L * kWTok
   int64_t samp_cap;
   TopkSel sel;       // thresholds + candidate regions
@@ -813,7 +816,7 @@ __device__ __forceinline__ void emit_filter_w(const Emit &em, const ScanArgs &a,
 // s4[slot][w]: each lane stores its block's four consecutive tokens per head
 // (and, GMAX, folds them into the quarter's group maximum, written once the
 // quarter ends).
-template <bool GMAX>
+template <bool GMAX, bool QUADS>
 __device__ __forceinline__ void store_scores(const Emit &em, const ScanArgs &a, const float (&s4)[2][4], EmitState &es,
                                              int64_t bh, int64_t beta0, int qs, int V, int lane) {
   const int c = lane & 15, gp = lane >> 4;
@@ -826,8 +829,8 @@ __device__ __forceinline__ void store_scores(const Emit &em, const ScanArgs &a, 
     const int h = 2 * gp + i;
     if (h >= a.G || !inr || tq >= a.n) continue;
     const float *s = s4[i];
-    float *dst = em.out + (bh * a.G + h) * a.n + t4;
-    if (t4 + 4 <= a.n && (a.n & 3) == 0) {
+    float *dst = em.out + (QUADS ? quad_score_at(a.n, a.G, bh, h, beta0, c, 4 * qs + V) : (bh * a.G + h) * em.ostride + t4);
+    if (GMAX || (t4 + 4 <= a.n && (a.n & 3) == 0)) {
       *reinterpret_cast<f4 *>(dst) = f4{s[0], s[1], s[2], s[3]};
     } else {
 #pragma unroll
@@ -903,8 +906,8 @@ __device__ __forceinline__ void emit_w(const Emit &em, const ScanArgs &a, const 
 template <int MODE>
 __device__ __forceinline__ void emit_flush(const Emit &em, const ScanArgs &a, EmitState &es, const StepOut &o,
                                            int64_t bh, int64_t beta0, int64_t L, int qs, int V, int lane) {
-  if constexpr (MODE == kEmitScores) store_scores<false>(em, a, o.s4, es, bh, beta0, qs, V, lane);
-  if constexpr (MODE == kEmitScoresMax) store_scores<true>(em, a, o.s4, es, bh, beta0, qs, V, lane);
+  if constexpr (MODE == kEmitScores) store_scores<false, false>(em, a, o.s4, es, bh, beta0, qs, V, lane);
+  if constexpr (emits_max(MODE)) store_scores<true, MODE == kEmitQuadsMax>(em, a, o.s4, es, bh, beta0, qs, V, lane);
   if constexpr (MODE == kEmitSample) store_sample(em, a, o.s4, es, bh, beta0, L, qs, V, lane);
 }
 
@@ -1205,8 +1208,8 @@ __device__ __forceinline__ void store_scores_stk(const Emit &em, const ScanArgs 
     const int h = 2 * gh + i;
     const bool on = h < a.G && inr && tq < a.n;
     if (on) {
-      float *dst = em.out + (bh * a.G + h) * a.n + t2;
-      if (t2 + 2 <= a.n && (a.n & 1) == 0) {
+      float *dst = em.out + (bh * a.G + h) * em.ostride + t2;
+      if (GMAX || (t2 + 2 <= a.n && (a.n & 1) == 0)) {
         *reinterpret_cast<f2 *>(dst) = f2{s2[i][0], s2[i][1]};
       } else {
         if (t2 < a.n) dst[0] = s2[i][0];
@@ -1288,7 +1291,7 @@ __device__ __forceinline__ void step_group_stk(const uint32_t (&qlo)[NS][2], con
   __builtin_amdgcn_sched_barrier(0);
   emit_pair<MODE, 1>(em, a, p1, k, es, o, bh, beta0, qs, V, lane);
   if constexpr (MODE == kEmitScores) store_scores_stk<false>(em, a, o.s, es, bh, beta0, qs, V, lane);
-  if constexpr (MODE == kEmitScoresMax) store_scores_stk<true>(em, a, o.s, es, bh, beta0, qs, V, lane);
+  if constexpr (emits_max(MODE)) store_scores_stk<true>(em, a, o.s, es, bh, beta0, qs, V, lane);
   if constexpr (MODE == kEmitSample) store_sample_stk(em, a, o.s, es, bh, beta0, L, qs, V, lane);
 }
 
@@ -1603,7 +1606,7 @@ template <int MODE, int NSK, bool FB, bool STK>
 __device__ __forceinline__ void host_tile_loop(const ScanArgs &a, const Emit &em, const Shared &sh, HostStage &hs,
                                                int64_t bh, int lane, int wave, int64_t nlist, uint32_t skipm, int nsl,
                                                int ureal) {
-  static_assert(MODE == kEmitFilter && NSK > 0 && NSK * kSlice <= kHostUnits, "staged candidate pass");
+  static_assert((MODE == kEmitFilter || emits_max(MODE)) && NSK > 0 && NSK * kSlice <= kHostUnits, "staged passes");
   uint32_t *rcp = FB ? em.sel.rc2 : em.sel.rc1;
   host_slots(hs, sh, ureal);
   __syncthreads();
@@ -1611,14 +1614,15 @@ __device__ __forceinline__ void host_tile_loop(const ScanArgs &a, const Emit &em
   uint32_t qreg[NSK][2], qhi[NSK][2];
   load_arows<NSK>(qreg, sh.qa, 0, lane & 15, lane >> 4);
   if constexpr (STK) load_arows_hi<NSK>(qhi, sh.qa, 0, lane);
-  const RowK rk = row_consts(em, a, bh, lane, FB, skipm, STK);
+  RowK rk{};
+  if constexpr (MODE == kEmitFilter) rk = row_consts(em, a, bh, lane, FB, skipm, STK);
   const int64_t step = (int64_t)gridDim.x * kWaves;
 #pragma unroll 1
   for (int64_t L4 = (int64_t)blockIdx.x * kWaves; L4 < nlist; L4 += step) {
     const int64_t L = L4 + wave;
     if (L4 < a.nwt) host_stage(hs, a, sh, bh, L4, nsl * kSlice, nch);  // uniform
     __syncthreads();
-    if (L < nlist && L >= a.nwt) {
+    if (L < nlist && L >= a.nwt) {  // the candidate pass only: its lists go on past the row
       if (lane < a.G && !((skipm >> lane) & 1u)) rcp[(bh * a.G + lane) * em.sel.nreg + L] = 0u;
     } else if (L < nlist) {
       TileJob j{bh, L * kWB, L, 0, kQS, lane, ureal, FB, skipm, rk};

@@ -5,8 +5,10 @@
 namespace fathom {
 
 // Workspace bytes of the fused scan + top-k over rows = BH * G score rows of n
-// tokens, kk = k - sink - local.
-size_t scan_topk_ws(int64_t rows, int64_t n, int64_t k, int64_t kk);
+// tokens, kk = k - sink - local.  whole_blocks = false: without the padding of
+// short rows to whole 64-token blocks (the size the scratch-free entry point's
+// limit is stated in).
+size_t scan_topk_ws(int64_t rows, int64_t n, int64_t k, int64_t kk, bool whole_blocks = true);
 
 // The fused scan + top-k (stages: FATHOM_STAGE_* mask) on a caller-provided workspace.
 int scan_topk_run(const float *q, int64_t BH, int64_t G, int64_t D, const int32_t *cls, const int32_t *clsn, int bmax,

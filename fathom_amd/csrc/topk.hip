@@ -550,7 +550,8 @@ __device__ __forceinline__ uint64_t range_select(const Src &src, int64_t cnt, ui
   return sh.thr;
 }
 
-__device__ __forceinline__ uint32_t masked_key(const float *row, int64_t i, int64_t sink, int64_t lstart) {
+template <typename Scores>
+__device__ __forceinline__ uint32_t masked_key(const Scores &row, int64_t i, int64_t sink, int64_t lstart) {
   return (i < sink || i >= lstart) ? kKeyNegInf : score_key(row[i]);
 }
 
@@ -1158,6 +1159,63 @@ __global__ __launch_bounds__(kSelThreads) void select_groups_kernel(const uint32
   }
 }
 
+// A group's 16 scores from four quads `step` apart.
+__device__ __forceinline__ void load_quads(const float *q, int64_t step, float (&v)[kGroupTok]) {
+  float4 f[kGroupTok / 4];
+#pragma unroll
+  for (int r = 0; r < kGroupTok / 4; ++r) f[r] = *reinterpret_cast<const float4 *>(q + r * step);
+#pragma unroll
+  for (int r = 0; r < kGroupTok / 4; ++r) {
+    v[4 * r] = f[r].x;
+    v[4 * r + 1] = f[r].y;
+    v[4 * r + 2] = f[r].z;
+    v[4 * r + 3] = f[r].w;
+  }
+}
+
+// Where a row's scores are: RowScores in the drop-in order, TileScores and
+// QuadScores in the fused scan's.  group: the 16 scores of the
+// group at t0 (past n: anything, and none where t0 is).
+struct RowScores {
+  const float *p;
+  int64_t n;
+  __device__ __forceinline__ RowScores(const float *scores, int64_t n_, int64_t) : p(scores + blockIdx.x * n_), n(n_) {}
+  __device__ __forceinline__ float operator[](int64_t i) const { return p[i]; }
+  __device__ __forceinline__ void group(int64_t t0, float (&v)[kGroupTok]) const {
+#pragma unroll
+    for (int r = 0; r < kGroupTok; ++r) v[r] = t0 + r < n ? p[t0 + r] : 0.0f;
+  }
+};
+struct TileScores {  // quad_order(G, n) false
+  const float *p;
+  int64_t n;
+  __device__ __forceinline__ TileScores(const float *scores, int64_t n_, int64_t)
+      : p(scores + blockIdx.x * tile_score_floats(n_)), n(n_) {}
+  __device__ __forceinline__ float operator[](int64_t i) const { return p[i]; }
+  __device__ __forceinline__ void group(int64_t t0, float (&v)[kGroupTok]) const {
+    if (t0 < n) load_quads(p + t0, 4, v);  // rows end on a whole block
+  }
+};
+struct QuadScores {  // quad_order(G, n) true
+  const float *p;    // the (batch, KV head) row's tiles
+  int64_t n;
+  int G, h;
+  __device__ __forceinline__ QuadScores(const float *scores, int64_t n_, int64_t G_)
+      : p(scores + (int64_t)(blockIdx.x / (uint32_t)G_) * G_ * tile_score_floats(n_)),
+        n(n_), G((int)G_), h((int)(blockIdx.x % (uint32_t)G_)) {}
+  __device__ __forceinline__ int64_t quad_at(int64_t i) const {  // the quad that holds token i
+    const int64_t beta0 = i / kRegTok * (kRegTok / kBlk);
+    const int t = (int)(i - beta0 * kBlk);
+    return quad_score_at(n, G, 0, h, beta0, t / kBlk, (t % kBlk) / 4);
+  }
+  __device__ __forceinline__ float operator[](int64_t i) const { return p[quad_at(i) + (i & 3)]; }
+  __device__ __forceinline__ void group(int64_t t0, float (&v)[kGroupTok]) const {
+    if (t0 >= n) return;
+    const int64_t q0 = quad_at(t0);
+    load_quads(p + q0, quad_at(t0 + 4) - q0, v);
+  }
+};
+
 // Exact top kk of short score rows whose 16-token group maxima the scan
 // wrote beside them (gmax [rows, ceil(n / 16)]: the largest masked key of each
 // group).  T, a lower bound of the kk-th largest group maximum, bounds the
@@ -1167,19 +1225,19 @@ __global__ __launch_bounds__(kSelThreads) void select_groups_kernel(const uint32
 // for spread scores).  Up to 2048 candidates are ranked by one sort; more are
 // selected first; rows whose candidates outgrow the LDS list (ties around T)
 // are selected from the whole row.
-constexpr int kGmaxGroups = (int)(kRowSelectMax / kGroupTok);
+constexpr int kGroupList = (int)(sizeof(uint64_t) * kMaxK / sizeof(uint16_t));  // listed groups (in ss)
+static_assert(kGmaxSelectMax / kGroupTok <= 65536, "group numbers fit 16 bits");
 // ranked (LDS of k int32, past the sort's scratch in cl; null: none): rows of
 // at most 2048 candidates also leave their k output tokens there, and the
 // call returns true.
-__device__ __forceinline__ bool rowselect_gmax_row(const float *__restrict__ scores, const uint32_t *__restrict__ gmax,
-                                                   int64_t n, int64_t m, int64_t k, int64_t sink, int64_t local,
+template <int kPer, typename Scores>
+__device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint32_t *__restrict__ gmax, int64_t n,
+                                                   int64_t m, int64_t k, int64_t sink, int64_t local,
                                                    int64_t *__restrict__ idx, uint64_t *cl, uint64_t *ss,
-                                                   RangeShared &sh, uint16_t *glist, uint32_t &s_cnt,
-                                                   int32_t *ranked = nullptr) {
-  constexpr int kPer = kGmaxGroups / kFinThreads;
+                                                   RangeShared &sh, uint32_t &s_cnt, int32_t *ranked = nullptr) {
+  uint16_t *glist = reinterpret_cast<uint16_t *>(ss);  // ss holds the survivors only after the groups are read
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = kFinThreads >> 6;
   const int64_t row = blockIdx.x;
-  const float *rs = scores + row * n;
   const int64_t lstart = (m - local) > 0 ? (m - local) : 0;
   const int64_t kk = k - sink - local;
   const int ngrp = (int)cdiv(n, kGroupTok);
@@ -1209,29 +1267,25 @@ __device__ __forceinline__ bool rowselect_gmax_row(const float *__restrict__ sco
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
       const int g = tid + u * kFinThreads;
-      if (g < ngrp && gm[u] >= T) glist[off++] = (uint16_t)g;
+      if (g < ngrp && gm[u] >= T) {
+        if (off < (uint32_t)kGroupList) glist[off] = (uint16_t)g;
+        ++off;
+      }
     }
     __syncthreads();
+  }
+  if (ngr > (uint32_t)kGroupList) {  // uniform: ties around T
+    const auto src = index_src([&](int64_t i) { return k64_of(masked_key(rs, i, sink, lstart), i); }, n);
+    select_sorted(src, n, kk, m, sink, local, out, cl, ss, sh, s_cnt, true);
+    return false;
   }
   // their keys >= T, one group per thread, placed by a workgroup prefix sum
   uint32_t cnt = 0u;
   for (uint32_t e0 = 0; e0 < ngr; e0 += kFinThreads) {  // uniform
     const uint32_t e = e0 + tid;
     const int64_t t0 = e < ngr ? (int64_t)glist[e] * kGroupTok : n;
-    float v[kGroupTok];
-    if (t0 + kGroupTok <= n && (n & 3) == 0) {
-#pragma unroll
-      for (int r = 0; r < kGroupTok; r += 4) {
-        const float4 f = *reinterpret_cast<const float4 *>(rs + t0 + r);
-        v[r] = f.x;
-        v[r + 1] = f.y;
-        v[r + 2] = f.z;
-        v[r + 3] = f.w;
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < kGroupTok; ++r) v[r] = t0 + r < n ? rs[t0 + r] : 0.0f;
-    }
+    float v[kGroupTok] = {};
+    rs.group(t0, v);
     uint32_t key[kGroupTok], c = 0u;
 #pragma unroll
     for (int r = 0; r < kGroupTok; ++r) {
@@ -1303,22 +1357,22 @@ struct RowAttn {
   float scale;
   float *out;      // [rows, D] fp32
 };
-template <bool ATTN>
-__global__ __launch_bounds__(kFinThreads) void rowselect_gmax_kernel(const float *__restrict__ scores,
+template <typename Scores, bool ATTN, int kPer>
+__global__ __launch_bounds__(kFinThreads) void rowselect_gmax_kernel(const float *__restrict__ scores, int64_t G,
                                                                      const uint32_t *__restrict__ gmax, int64_t n,
                                                                      int64_t m, int64_t k, int64_t sink, int64_t local,
                                                                      int64_t *__restrict__ idx, RowAttn ra) {
   __shared__ uint64_t cl[kCandLds];
   __shared__ uint64_t ss[kMaxK];
   __shared__ RangeShared sh;
-  __shared__ uint16_t glist[kGmaxGroups];
   __shared__ uint32_t s_cnt;
   // ATTN: the ranked tokens also in LDS, in cl's upper half (past the sort's
   // scratch and the attention's triples)
   int32_t *ranked = ATTN ? reinterpret_cast<int32_t *>(cl + kCandLds / 2) : nullptr;
   static_assert(kCandLds / 2 >= 2 * 2 * kFinThreads + kBins && 2 * (kCandLds / 2) >= kMaxK + kFinThreads,
                 "the ranked tokens lie past the sort's scratch and hold k of them");
-  const bool in_lds = rowselect_gmax_row(scores, gmax, n, m, k, sink, local, idx, cl, ss, sh, glist, s_cnt, ranked);
+  const bool in_lds = rowselect_gmax_row<kPer>(Scores(scores, n, G), gmax, n, m, k, sink, local, idx, cl, ss, sh,
+                                               s_cnt, ranked);
   if constexpr (ATTN) {
     constexpr int NW = kFinThreads / kWave;
     static_assert(NW == 16, "one attention split of 16 waves");
@@ -1489,10 +1543,26 @@ int launch_rowselect(const float *scores, int64_t rows, int64_t n, int64_t m, in
   return launch_status("rowselect_kernel");
 }
 
-int launch_rowselect_gmax(const float *scores, const uint32_t *gmax, int64_t rows, int64_t n, int64_t m, int64_t k,
-                          int64_t sink, int64_t local, int64_t *idx, hipStream_t st) {
-  rowselect_gmax_kernel<false><<<(unsigned)rows, kFinThreads, 0, st>>>(scores, gmax, n, m, k, sink, local, idx, RowAttn{});
+namespace {
+// Group maxima per thread: 2 (rows of up to 32768 tokens) or 8.
+template <typename Scores, bool ATTN>
+int launch_gmax(const float *scores, int64_t G, const uint32_t *gmax, int64_t rows, int64_t n, int64_t m, int64_t k,
+                int64_t sink, int64_t local, int64_t *idx, const RowAttn &ra, hipStream_t st) {
+  const unsigned g = (unsigned)rows;
+  static_assert(kRowSelectMax == 2 * kFinThreads * kGroupTok && kGmaxSelectMax == 8 * kFinThreads * kGroupTok, "groups");
+  if (n > kGmaxSelectMax) return fail(FATHOM_ERR_INVALID, "rowselect_gmax: n=%lld exceeds %lld", (long long)n, (long long)kGmaxSelectMax);
+  if (n <= kRowSelectMax)
+    rowselect_gmax_kernel<Scores, ATTN, 2><<<g, kFinThreads, 0, st>>>(scores, G, gmax, n, m, k, sink, local, idx, ra);
+  else
+    rowselect_gmax_kernel<Scores, ATTN, 8><<<g, kFinThreads, 0, st>>>(scores, G, gmax, n, m, k, sink, local, idx, ra);
   return launch_status("rowselect_gmax_kernel");
+}
+}  // namespace
+
+int launch_rowselect_gmax(const float *scores, const uint32_t *gmax, int64_t rows, int64_t G, int64_t n, int64_t m,
+                          int64_t k, int64_t sink, int64_t local, int64_t *idx, hipStream_t st) {
+  if (!quad_order(G, n)) return launch_gmax<TileScores, false>(scores, G, gmax, rows, n, m, k, sink, local, idx, RowAttn{}, st);
+  return launch_gmax<QuadScores, false>(scores, G, gmax, rows, n, m, k, sink, local, idx, RowAttn{}, st);
 }
 
 int launch_rowselect_gmax_attn(const float *scores, const uint32_t *gmax, int64_t rows, int64_t n, int64_t m, int64_t k,
@@ -1501,8 +1571,8 @@ int launch_rowselect_gmax_attn(const float *scores, const uint32_t *gmax, int64_
   if (k > kFinThreads / 2) return fail(FATHOM_ERR_INVALID, "rowselect_gmax_attn: k=%lld exceeds 512", (long long)k);
   RowAttn ra{q, G, attn::RowSrc{(const char *)K, (const char *)V, nullptr, nullptr, cap, 0, n, 2 * attn::kAttnD}, scale,
              out};
-  rowselect_gmax_kernel<true><<<(unsigned)rows, kFinThreads, 0, st>>>(scores, gmax, n, m, k, sink, local, idx, ra);
-  return launch_status("rowselect_gmax_kernel");
+  if (!quad_order(G, n)) return launch_gmax<TileScores, true>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st);
+  return launch_gmax<QuadScores, true>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st);
 }
 
 int launch_rank_list(const uint64_t *sel, int64_t P, int64_t rows, int64_t kk, int64_t m, int64_t k, int64_t sink,

@@ -40,13 +40,41 @@ constexpr int64_t kAlphaX2 = 5;
 
 // Score rows up to this length (their 32-bit keys fit in one workgroup's LDS)
 // select their top kk in one kernel, one workgroup per row, instead of
-// sample -> select -> filter -> finalize: fewer launches for short rows.  The
-// fused scan + top-k keeps the chain (its first pass writes no scores).
+// sample -> select -> filter -> finalize: fewer launches for short rows.
 constexpr int64_t kRowSelectMax = 32768;
+
+// Longest rows that the fused scan + top-k selects from its scores' 16-token group
+// maxima, in two launches (the plan, where asked for, made in the scan) instead of
+// the sampled chain's four: the scores cost 4.25 bytes per token and head of
+// stores, the chain its latency-bound launches.  Scan + top-k, us, chain against
+// group maxima: 8 x 4 heads of 40000 tokens 34.5; 23.0, of 131072 35.7; 30.4, of
+// 262144 36.3; 43.1; 32 x 4 heads of 65536 57.5; 43.1; 8 x 7 heads of 131072 63; 51;
+// 16 x 8 heads of 131072 65; 52; 2 x 4 heads of 262144 31.6; 30.4.
+constexpr int64_t kGmaxSelectMax = 131072;
 
 // Tokens per group of the group maxima that the fused scan's short-row pass
 // writes beside its scores (one lane's 16 tokens of a block).
 constexpr int64_t kGroupTok = 16;
+
+// The fused scan's own score order, rows held in whole blocks (so no store is
+// split or unaligned, whatever n is): [bh][head][token], the drop-in order
+// padded, or -- more than four heads, long rows -- per bh and tile of 16 blocks
+// [16 token quads of a block][head][block][4].  A store instruction of the scan is
+// one quad of every block; the drop-in order leaves 16-byte pieces 256 bytes
+// apart, the quad order runs of 256 bytes per head, but a group's 64 bytes then
+// lie in four lines when the selection reads them.  The last tile's runs are as
+// long as its blocks.  Scan + selection, us (drop-in; quad): 8 x 7 heads of 131072
+// tokens 54; 51, 16 x 8 heads 71; 53, 8 x 7 heads of 20000 tokens 26.1; 28.0.  Up to
+// four heads store 8-byte pairs per lane: 8 x 4 heads of 131072 tokens 30.3; 32.8,
+// and of 131071 tokens 30.3 padded against 37.1 unpadded.
+__host__ __device__ inline int64_t tile_score_floats(int64_t n) { return cdiv(n, kBlk) * kBlk; }
+__host__ __device__ inline bool quad_order(int64_t G, int64_t n) { return G > 4 && n > kRowSelectMax; }
+// Where the first token of a quad of block beta0 + c (beta0 the tile's first) is.
+__device__ __forceinline__ int64_t quad_score_at(int64_t n, int G, int64_t bh, int h, int64_t beta0, int c, int quad) {
+  const int64_t nblk = cdiv(n, kBlk);
+  const int nbt = (int)(nblk - beta0 < kRegTok / kBlk ? nblk - beta0 : kRegTok / kBlk);
+  return (bh * nblk + beta0) * (int64_t)(kBlk * G) + ((quad * G + h) * nbt + c) * 4;
+}
 
 // Candidate counters of a row, one per 256 bytes: every workgroup of a pass
 // adds to its row's counter, and atomics to one cache line serialise.
@@ -142,9 +170,10 @@ int launch_finalize(int64_t rows, int64_t m, int64_t k, int64_t sink, int64_t lo
 int launch_rowselect(const float *scores, int64_t rows, int64_t n, int64_t m, int64_t k, int64_t sink, int64_t local,
                      int64_t *idx, hipStream_t st);
 // The same from the rows' 16-token group maxima (gmax [rows, ceil(n / 16)]
-// largest masked keys): only the groups that can hold a top-kk key are read.
-int launch_rowselect_gmax(const float *scores, const uint32_t *gmax, int64_t rows, int64_t n, int64_t m, int64_t k,
-                          int64_t sink, int64_t local, int64_t *idx, hipStream_t st);
+// largest masked keys; scores in the fused scan's order): only the groups that
+// can hold a top-kk key are read.
+int launch_rowselect_gmax(const float *scores, const uint32_t *gmax, int64_t rows, int64_t G, int64_t n, int64_t m,
+                          int64_t k, int64_t sink, int64_t local, int64_t *idx, hipStream_t st);
 // launch_rowselect_gmax, then in the same workgroup the attention of each row's
 // query head (row = bh * G + g) over its k <= 512 selected positions: K, V
 // bf16 rows [BH, cap, D = 128] in device memory, out [rows, D] fp32, equal to

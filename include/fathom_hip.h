@@ -169,8 +169,8 @@ int fathom_klt_query(const float *q, const float *Vt, const float *lam, int64_t 
  * fathom_sink_local_topk on its scores (kernels/bitplane.py:319-338 then
  * :372-378, as chained by scripts/B_kernel_bench.py:74 and
  * scripts/B_e2e_offload_v2.py:203, 224-227), without materialising the score
- * tensor for rows longer than 32768 (shorter rows keep their scores in the
- * workspace for one selection launch).  Same arguments as fathom_scan_planes
+ * tensor for rows longer than 131072 (shorter rows keep their scores, and each
+ * 16-token group's largest key, in the workspace for one selection launch).  Same arguments as fathom_scan_planes
  * over the whole sequence, plus the top-k arguments of fathom_sink_local_topk;
  * idx [BH * G, k] int64 is identical to running the two entry points.
  * workspace: fathom_scan_topk_workspace_bytes(BH, G, n, k, sink, local) bytes.
@@ -186,7 +186,7 @@ int fathom_scan_topk(const float *q, int64_t BH, int64_t G, int64_t D, const int
  * a bitmask of FATHOM_STAGE_*; fathom_scan_topk runs FATHOM_STAGE_ALL, in the
  * order sample, select, candidates, finalize.  A stage reads what the earlier
  * stages left in the workspace, so a partial call repeats a later stage over
- * the state of the last full one (same arguments).  Rows of at most 32768
+ * the state of the last full one (same arguments).  Rows of at most 131072
  * tokens have two stages only: candidates (the scores into the workspace) and
  * finalize (the selection over them).  It exists for stage timing (bench.py
  * times the candidate pass, the dominant kernel, on its own) and has no
@@ -208,7 +208,7 @@ int fathom_scan_topk_stages(const float *q, int64_t BH, int64_t G, int64_t D, co
  * is null; bmax, iters as there) then fathom_scan_topk with that plan's cls and
  * clsn (kernels/bitplane.py:83-116 then :319-338 and :372-378, the plan ->
  * scan -> top-k stages of scripts/B_kernel_bench.py:74).  For rows of at most
- * 32768 tokens (D <= 128) every workgroup of the scan makes its row's plan in
+ * 131072 tokens (D <= 128) every workgroup of the scan makes its row's plan in
  * its prologue with the plan kernel's arithmetic, so no plan launch and no
  * plan arrays precede the scan: the decode form of the chain.  Longer rows run
  * the plan kernel into the workspace first.  t_out [BH, D] int8 (nullable)
@@ -228,8 +228,8 @@ int fathom_plan_scan_topk(const float *q, const float *g, const float *budget, f
  * fathom_plan_scan_topk followed by fathom_gather_attention over its indices
  * (rows in device memory: Ksrc, Vsrc bf16 [BH, cap, 128], no recent rows),
  * the decode step's plan -> scan -> top-k -> gather + attention chain of
- * scripts/B_kernel_bench.py:64-101 in one call.  For rows of at most 32768
- * tokens and k <= 512 each selection workgroup goes on to its query head's
+ * scripts/B_kernel_bench.py:64-101 in one call.  For rows of at most 131072
+ * tokens, k <= 512 and 96 query heads or more each selection workgroup goes on to its query head's
  * attention over the indices it wrote (the arithmetic of gather_attention), so
  * idx and out equal the two calls'.  Other shapes run the two calls.  It
  * composes reference stages and has no single counterpart in the reference.
@@ -250,9 +250,10 @@ int fathom_plan_scan_topk_attention(const float *q, const float *g, const float 
  * allocate device memory (code under graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  It has no counterpart in the reference.
  * The workspace is a static device array of the library, of
- * FATHOM_NOALLOC_SCRATCH_BYTES, one per device that calls it (held until the
- * process ends); shapes whose fathom_scan_topk_workspace_bytes exceed it are
- * rejected with FATHOM_ERR_WORKSPACE before any launch.  The call allocates
+ * FATHOM_NOALLOC_SCRATCH_BYTES (plus padding), one per device that calls it (held
+ * until the process ends); shapes whose fathom_scan_topk_workspace_bytes exceed
+ * it (for rows of at most 32768 tokens and k - sink - local up to 2048: without
+ * the rows' padding to whole 64-token blocks) are rejected with FATHOM_ERR_WORKSPACE before any launch.  The call allocates
  * nothing (no hipMalloc, no library allocation).  Calls that overlap on one
  * device (several streams or threads) share the array and race.  Results are
  * those of fathom_scan_topk on the same arguments.  The array's device address

@@ -1,0 +1,90 @@
+"""Selection over 16-token group maxima, rows of up to 131072 tokens, at the edges of its shapes: equal to the top-k of the
+scan's scores (itself checked against the oracle), whatever the order of the scores, the layout of the store and the
+route a length takes on either side of the limits."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from fathom_amd import bitplane as bp
+from fathom_amd import offload as off
+from fathom_amd import workloads as W
+from oracle import fathom_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+
+
+def _oracle_topk(scores, k, sink, local, m):
+    s = scores.cpu().numpy()
+    return torch.from_numpy(O.sink_local_topk(s, k, sink, local, m=m))
+
+
+@pytest.mark.parametrize("BH,G,n,k,sub,extra", [(2, 4, 32769, 512, 16, 0), (1, 4, 131072, 2084, 0, 9), (2, 3, 131071, 100, 64, 0),
+                                                (1, 7, 131072, 512, 16, 0), (2, 5, 32833, 2084, 64, 31),
+                                                (1, 8, 100001, 300, 0, 5), (3, 1, 65600, 512, 64, 0),
+                                                (1, 4, 131073, 512, 16, 0), (2, 7, 140000, 600, 64, 0), (24, 4, 33333, 512, 16, 0)])
+def test_fused_selection_at_its_limits(BH, G, n, k, sub, extra, monkeypatch):
+    print(f"[group-select] {BH}x{G} n={n} k={k} sub={sub}", flush=True)
+    monkeypatch.setattr(bp, "SUB", sub or -(-n // 64))
+    x = W.synth_layer(BH, n, G, seed=n % 97, device=DEV, kdtype=torch.bfloat16)
+    g = ((x["q"] ** 2) * x["var"][:, None, :]).sum(1)
+    st = bp.PlaneStore(x["K"])
+    for budget in (48.0, 110.0):  # plans held in registers, and in register groups
+        plan = bp.make_plan(g, budget)
+        scores = st.scan(x["q"], plan)
+        want = _oracle_topk(scores, k, 4, 32, n + extra)
+        got = st.scan_topk(x["q"], plan, k, 4, 32, m=n + extra)
+        idx, t = st.plan_scan_topk(x["q"], g, budget, k, 4, 32, m=n + extra, return_t=True)
+        assert torch.equal(got.cpu(), want) and torch.equal(idx, got) and torch.equal(t, plan["t"])
+        if extra == 0:
+            i2, out = st.plan_scan_topk_attention(x["q"], g, budget, k, x["K"], x["K"], 4, 32)
+            ref, _ = off.gather_attention(x["q"], got, n, x["K"], x["K"], n)
+            assert torch.equal(i2, got) and torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("n", [65536, 131072, 140001])
+@pytest.mark.parametrize("G", [4, 7])
+def test_ties_and_masks(n, G):
+    """Every score equal, and scores that fall or rise along the row (every group of one end reaches the threshold; past
+    the limit the sample misleads the chain and its rows are rescanned)."""
+    print(f"[group-select ties] n={n} G={G}", flush=True)
+    for kind in ("equal", "falling", "rising"):
+        K = torch.zeros(1, n, 128, device=DEV)
+        if kind != "equal":
+            K[0, :, 0] = torch.linspace(3, -3, n, device=DEV) * (1 if kind == "falling" else -1)
+            K[0, :, 1] = torch.randn(n, device=DEV, generator=torch.Generator(DEV).manual_seed(2)) * 0.01
+        st = bp.PlaneStore(K, keep_code=False)
+        q = torch.zeros(1, G, 128, device=DEV)
+        q[..., 0], q[:, 1::2, 1] = 1.0, 1.0
+        gain = torch.ones(1, 128, device=DEV)
+        gain[0, 0], gain[0, 1] = 1000.0, 10.0
+        plan = bp.make_plan(gain, 6.0)
+        scores = st.scan(q, plan)
+        got = st.scan_topk(q, plan, 2000, 4, 32)
+        assert torch.equal(got.cpu(), _oracle_topk(scores, 2000, 4, 32, n)), kind
+
+
+@pytest.mark.parametrize("n,G", [(40000, 4), (131072, 6), (200000, 4)])
+def test_host_resident_staged_scan_equals_hbm(n, G, monkeypatch):
+    """Superblocks of 64 blocks in mapped host memory: the staged passes give the same indices, whatever the plan."""
+    print(f"[group-select host] n={n} G={G}", flush=True)
+    monkeypatch.setattr(bp, "SUB", 64)
+    x = W.synth_layer(2, n, G, seed=3, device=DEV, kdtype=torch.bfloat16)
+    g = ((x["q"] ** 2) * x["var"][:, None, :]).sum(1)
+    st = bp.PlaneStore(x["K"], keep_code=False)
+    plans = [bp.make_plan(g, b) for b in (20.0, 48.0, 64.0, 100.0)]
+    want = [st.scan_topk(x["q"], p, 512, 4, 32) for p in plans]
+    ref = [bp.sink_local_topk(st.scan(x["q"], p), 512, 4, 32) for p in plans]
+    _, pl, h1 = off.host_mapped(st.planes_k)
+    _, sc, h2 = off.host_mapped(st.scales_k)
+    try:
+        st.planes32, st.scales_k = pl, sc
+        got = [st.scan_topk(x["q"], p, 512, 4, 32) for p in plans]
+        torch.cuda.synchronize()
+    finally:
+        off.free_host(h1)
+        off.free_host(h2)
+    for a, b, c in zip(got, want, ref):
+        assert torch.equal(a, b) and torch.equal(a, c)
