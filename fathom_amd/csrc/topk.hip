@@ -14,6 +14,8 @@
 // follow the values' actual spread, so a row's candidates -- all packed just
 // above a threshold -- still spread over many bins (few atomic collisions),
 // and a 64-bit K64 needs at most six rounds.
+#include <type_traits>
+
 #include "topk_internal.hpp"
 #include "scan_core.hpp"
 #include "attn_core.hpp"
@@ -191,30 +193,54 @@ __device__ __forceinline__ void block_rank_desc(const uint64_t (&v)[E], uint64_t
   }
 }
 
+__device__ __forceinline__ bool finite_key(uint32_t key) { return key > kKeyNegInf && key < 0xFF800000u; }
+
+// Linear bins of scores over the finite range [lo, hi] of keys: -inf in the
+// bottom bin, NaN and +inf in the top one.  Every step of the map is monotone.
+struct LinearBins {
+  float flo, scale;
+  __device__ __forceinline__ LinearBins(uint32_t lo, uint32_t hi)
+      : flo(key_value(lo)), scale((float)kBins / (key_value(hi) - flo)) {}
+  __device__ __forceinline__ uint32_t of(uint32_t key) const {
+    const float x = fminf(fmaxf((key_value(key) - flo) * scale, 0.0f), (float)(kBins - 1));  // NaN (equal scores): 0
+    return finite_key(key) ? (uint32_t)x : key > kKeyNegInf ? (uint32_t)(kBins - 1) : 0u;
+  }
+  __device__ __forceinline__ bool positive(uint32_t bin) const { return flo + (float)bin / scale > 0.0f; }
+};
+
 // Descending ranks of the cnt valid values of E * 1024 (thread t holding slots
-// t + 1024 e; the valid ones are the slots below cnt, all distinct) by a
-// counting sort: 2048 bins of (v - min) >> s over the values' range, each
+// t + 1024 e; the valid ones are the slots below cnt -- LINEAR: the nonzero ones --
+// all distinct) by a
+// counting sort: 2048 bins of (v - min) >> s over the values' range (LINEAR: of
+// the scores themselves over the finite ones' range, -inf in the bottom bin, NaN
+// and +inf in the top one), each
 // value's place in its bin from a returning LDS atomic, the bins' offsets by a
 // prefix sum from the top bin down, then every value's rank = the values in
 // higher bins + the greater values of its own bin (a few, read from the
-// values placed in bin order).  Values crowd a bin only where their range is
+// values placed in bin order).  Bins whose values all rank at or past limit are
+// left out.  Values crowd a bin only where their range is
 // dominated by a few outliers: then (more than kCrowd in one bin) the ranks
 // come from block_rank_desc over the first nlim slots instead.  put(rank, v)
-// is called for every valid value.  scratch: LDS of max(E * 1024 + 2048,
+// is called for every valid value of rank below limit (and some past it).  scratch: LDS of max(E * 1024 + 2048,
 // 2 * nlim) values.
+// The bits of a key grow with the logarithm of the score's magnitude: right for the
+// tail above a threshold, with its outliers, but a whole row's scores, of both
+// signs, crowd into a few dozen bins; those take LINEAR (n = 1000, the selection:
+// 13.8 -> 4.8 us).
 constexpr uint32_t kCrowd = 48;
-template <int E, typename Put>
-__device__ __forceinline__ void bin_rank_desc(const uint64_t (&v)[E], int cnt, uint64_t *scratch, RangeShared &sh,
-                                              int nlim, Put put) {
+template <int E, bool LINEAR = false, typename Put>
+__device__ __forceinline__ void bin_rank_desc(const uint64_t (&v)[E], int cnt, int limit, uint64_t *scratch,
+                                              RangeShared &sh, int nlim, Put put) {
   static_assert(kBins == 2 * kFinThreads, "two bins per thread");
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = kFinThreads >> 6;
   uint64_t *placed = scratch;                                           // [E * 1024] values in bin order
   uint32_t *hist = reinterpret_cast<uint32_t *>(scratch + E * 1024);    // [2048] values per bin
   uint32_t *above = hist + kBins;                                       // [2048] values in higher bins
+  const auto valid = [&](int e) { return LINEAR ? v[e] != 0ull : t + 1024 * e < cnt; };
   uint64_t mn = ~0ull, mx = 0ull;
 #pragma unroll
   for (int e = 0; e < E; ++e)
-    if (t + 1024 * e < cnt) {
+    if (valid(e) && (!LINEAR || finite_key((uint32_t)(v[e] >> 32)))) {
       mn = v[e] < mn ? v[e] : mn;
       mx = v[e] > mx ? v[e] : mx;
     }
@@ -234,11 +260,12 @@ __device__ __forceinline__ void bin_rank_desc(const uint64_t (&v)[E], int cnt, u
   const uint64_t R = cnt > 0 ? hi - lo : 0ull;
   const int bl = R ? 64 - __clzll((long long)R) : 0;
   const int sft = bl > 11 ? bl - 11 : 0;  // (v - lo) >> sft < 2048
+  const LinearBins lin((uint32_t)(lo >> 32), (uint32_t)(hi >> 32));
   uint32_t bin[E], slot[E];
 #pragma unroll
   for (int e = 0; e < E; ++e)
-    if (t + 1024 * e < cnt) {
-      bin[e] = (uint32_t)((v[e] - lo) >> sft);
+    if (valid(e)) {
+      bin[e] = LINEAR ? lin.of((uint32_t)(v[e] >> 32)) : (uint32_t)((v[e] - lo) >> sft);
       slot[e] = atomicAdd(&hist[bin[e]], 1u);
     }
   __syncthreads();
@@ -246,26 +273,28 @@ __device__ __forceinline__ void bin_rank_desc(const uint64_t (&v)[E], int cnt, u
   const uint32_t c0 = hist[kBins - 1 - 2 * t], c1 = hist[kBins - 2 - 2 * t], c = c0 + c1;
   const uint32_t wi = wave_incl_scan_u32(c);
   if (lane == kWave - 1) sh.wsum[wave] = wi;
-  if (c0 > kCrowd || c1 > kCrowd) sh.fcnt = 1u;  // any thread: the same value
+  __syncthreads();
+  uint32_t ab = wi - c;
+  for (int w = 0; w < wave; ++w) ab += sh.wsum[w];
+  const uint32_t lim = (uint32_t)limit;
+  if ((c0 > kCrowd && ab < lim) || (c1 > kCrowd && ab + c0 < lim)) sh.fcnt = 1u;  // any thread: the same value
+  above[kBins - 1 - 2 * t] = ab;
+  above[kBins - 2 - 2 * t] = ab + c0;
   __syncthreads();
   if (sh.fcnt) {  // uniform
+    __syncthreads();  // scratch is rewritten
     block_rank_desc<E>(v, scratch, scratch + nlim, nlim, [&](int rank, uint64_t x) {
       if (rank < cnt) put(rank, x);
     });
     return;
   }
-  uint32_t ab = wi - c;
-  for (int w = 0; w < wave; ++w) ab += sh.wsum[w];
-  above[kBins - 1 - 2 * t] = ab;
-  above[kBins - 2 - 2 * t] = ab + c0;
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (valid(e) && above[bin[e]] < lim) placed[above[bin[e]] + slot[e]] = v[e];
   __syncthreads();
 #pragma unroll
   for (int e = 0; e < E; ++e)
-    if (t + 1024 * e < cnt) placed[above[bin[e]] + slot[e]] = v[e];
-  __syncthreads();
-#pragma unroll
-  for (int e = 0; e < E; ++e)
-    if (t + 1024 * e < cnt) {
+    if (valid(e) && above[bin[e]] < lim) {
       const uint32_t base = above[bin[e]], n = hist[bin[e]];
       uint32_t rank = base;
       for (uint32_t j = 0; j < n; ++j) rank += placed[base + j] > v[e] ? 1u : 0u;
@@ -567,6 +596,37 @@ __global__ __launch_bounds__(256) void sample_scores_kernel(const float *__restr
   }
 }
 
+// Largest masked key of each 16-token group of score rows (gmax [rows, ceil(n /
+// 16)]).  A workgroup takes 4096 tokens, every load in flight at once; a group is
+// the 16 lanes of a DPP row, and lane u of a row writes the row's u-th group.
+// Rows need no alignment.  Bound: HBM, 4.25 bytes per score.  sink_local_topk of
+// 32 rows, k = 512, with it and the selection below against the sample -> select ->
+// filter -> finalize chain: n = 32768 46 -> 17.2 us, 50021 48.8 -> 17.7, 131072 42.8 ->
+// 19.8.
+constexpr int kGmaxPer = 16;
+__global__ __launch_bounds__(256) void group_max_kernel(const float *__restrict__ scores, int64_t n, int64_t sink,
+                                                        int64_t lstart, uint32_t *__restrict__ gmax) {
+  const int64_t row = blockIdx.y, i0 = (int64_t)blockIdx.x * (256 * kGmaxPer) + threadIdx.x;
+  const float *rs = scores + row * n;
+  float v[kGmaxPer];
+#pragma unroll
+  for (int u = 0; u < kGmaxPer; ++u) v[u] = i0 + u * 256 < n ? rs[i0 + u * 256] : 0.0f;
+  uint32_t mine = 0u;
+#pragma unroll
+  for (int u = 0; u < kGmaxPer; ++u) {
+    const int64_t i = i0 + u * 256;
+    uint32_t key = i < n ? ((i < sink || i >= lstart) ? kKeyNegInf : score_key(v[u])) : 0u;
+    key = max(key, (uint32_t)__builtin_amdgcn_mov_dpp((int)key, 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
+    key = max(key, (uint32_t)__builtin_amdgcn_mov_dpp((int)key, 0x4E, 0xF, 0xF, false));   // quad_perm [2,3,0,1]
+    key = max(key, (uint32_t)__builtin_amdgcn_mov_dpp((int)key, 0x141, 0xF, 0xF, false));  // row_half_mirror
+    key = max(key, (uint32_t)__builtin_amdgcn_mov_dpp((int)key, 0x140, 0xF, 0xF, false));  // row_mirror
+    if (u == (int)(threadIdx.x & 15)) mine = key;
+  }
+  const int64_t ngrp = cdiv(n, kGroupTok);
+  const int64_t g = (int64_t)blockIdx.x * (256 * kGmaxPer / kGroupTok) + (threadIdx.x & 15) * 16 + (threadIdx.x >> 4);
+  if (g < ngrp) gmax[row * ngrp + g] = mine;
+}
+
 // Candidates of score rows (keys >= the row's threshold), 4 scores per thread
 // and step when rows are 16-byte aligned.
 template <bool VEC>
@@ -655,7 +715,7 @@ __device__ __forceinline__ void select_sorted(const Src &src, int64_t cnt, int64
   while (nlim < nv) nlim <<= 1;  // the survivors fill the first nv <= 2048 slots
   const int got = nv < (int)kk ? nv : (int)kk;
   // only the survivors are ranked and written
-  bin_rank_desc<2>(v2, nv, cl, sh, nlim, [&](int rank, uint64_t x) {
+  bin_rank_desc<2>(v2, nv, got, cl, sh, nlim, [&](int rank, uint64_t x) {
     if (rank < got) out[rank] = (int64_t)(0xFFFFFFFFu - (uint32_t)x);
   });
   write_fixed(out, got, kk, m, sink, local);
@@ -741,7 +801,7 @@ __global__ __launch_bounds__(kFinThreads) void finalize_fused_kernel(int64_t m, 
     int nlim = kWave;
     while (nlim < (int)cnt) nlim <<= 1;
     const int got = (int64_t)cnt < kk ? (int)cnt : (int)kk;
-    bin_rank_desc<4>(v4, (int)cnt, cl, sh, nlim, [&](int rank, uint64_t x) {
+    bin_rank_desc<4>(v4, (int)cnt, got, cl, sh, nlim, [&](int rank, uint64_t x) {
       if (rank < got) out[rank] = (int64_t)(0xFFFFFFFFu - (uint32_t)x);
     });
     write_fixed(out, got, kk, m, sink, local);
@@ -750,106 +810,6 @@ __global__ __launch_bounds__(kFinThreads) void finalize_fused_kernel(int64_t m, 
   } else {
     select_sorted(src, cnt, kk, m, sink, local, out, cl, ss, sh, s_cnt, false);
   }
-}
-
-// Exact top kk of a whole score row (rows up to kRowSelectMax): every element
-// is a candidate.  Rows up to 2 * kCandLds keep their 32-bit keys in LDS (all
-// of a thread's loads in flight together; the K64 of element i is rebuilt from
-// its key and index).  For kk <= 1024 a prefilter keeps the selection small:
-// the maxima of P >= kk interleaved groups of keys are ranked, the kk-th of
-// them, T, bounds the row's kk-th largest key from below (kk elements reach
-// it), and only the keys >= T (a few per cent of a row) are selected from --
-// unless more than kMaxK reach it (ties, clustered rows), when the whole row
-// is.  Longer rows are read from global memory.
-__global__ __launch_bounds__(kFinThreads) void rowselect_kernel(const float *__restrict__ scores, int64_t n, int64_t m,
-                                                                int64_t k, int64_t sink, int64_t local,
-                                                                int64_t *__restrict__ idx) {
-  constexpr int kLoad = 2 * kCandLds / kFinThreads;  // keys per thread
-  __shared__ uint64_t cl[kCandLds];
-  __shared__ uint64_t ss[kMaxK];
-  __shared__ RangeShared sh;
-  __shared__ uint32_t s_cnt;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int64_t row = blockIdx.x;
-  const float *rs = scores + row * n;
-  const int64_t lstart = (m - local) > 0 ? (m - local) : 0;
-  const int64_t kk = k - sink - local;
-  int64_t *out = idx + row * k;
-  if (n > 2 * kCandLds) {
-    const auto src = index_src([&](int64_t i) { return k64_of(masked_key(rs, i, sink, lstart), i); }, n);
-    select_sorted(src, n, kk, m, sink, local, out, cl, ss, sh, s_cnt, true);
-    return;
-  }
-  uint32_t *kl = reinterpret_cast<uint32_t *>(cl);
-  uint32_t key[kLoad];  // the thread's keys t + 1024 u stay in registers
-  {
-    float v[kLoad];
-#pragma unroll
-    for (int u = 0; u < kLoad; ++u) {
-      const int64_t i = tid + (int64_t)u * kFinThreads;
-      v[u] = i < n ? rs[i] : 0.0f;
-    }
-#pragma unroll
-    for (int u = 0; u < kLoad; ++u) {
-      const int64_t i = tid + (int64_t)u * kFinThreads;
-      key[u] = i < n ? ((i < sink || i >= lstart) ? kKeyNegInf : score_key(v[u])) : 0u;
-      if (i < n) kl[i] = key[u];
-    }
-  }
-  __syncthreads();
-  auto whole = [&]() {
-    const auto src = index_src([&](int64_t i) { return ((uint64_t)kl[i] << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)i); }, n);
-    select_sorted(src, n, kk, m, sink, local, out, cl, ss, sh, s_cnt, false);
-  };
-  if (kk > kFinThreads || n <= kMaxK) {
-    whole();
-    return;
-  }
-  // group maxima: thread t covers keys t + 1024 u; group s < P combines the
-  // threads s, s + P, ... (keys i with i mod P == s); padding keys are 0
-  int P = kWave;
-  while (P < (int)kk) P <<= 1;
-  uint32_t mk = 0u;
-#pragma unroll
-  for (int u = 0; u < kLoad; ++u) mk = max(mk, key[u]);
-  sh.hist[tid] = mk;
-  __syncthreads();
-  uint32_t gm = 0u;
-  if (tid < P)
-    for (int j = tid; j < kFinThreads; j += P) gm = max(gm, sh.hist[j]);
-  const uint64_t wg[1] = {((uint64_t)gm << 32) | (uint32_t)(tid + 1)};
-  block_rank_desc<1>(wg, ss, ss + kFinThreads, P, [&](int rank, uint64_t x) {
-    if (rank == (int)kk - 1) sh.lo = x;
-  });
-  __syncthreads();
-  const uint32_t T = (uint32_t)(sh.lo >> 32);
-  // the keys >= T: counted per thread, a workgroup prefix sum places them
-  uint32_t c = 0u;
-#pragma unroll
-  for (int u = 0; u < kLoad; ++u) c += (tid + (int64_t)u * kFinThreads < n && key[u] >= T) ? 1u : 0u;
-  const int wave = tid >> 6, nw = kFinThreads >> 6;
-  const uint32_t wi = wave_incl_scan_u32(c);
-  if (lane == kWave - 1) sh.wsum[wave] = wi;
-  __syncthreads();
-  uint32_t off = wi - c, cnt = 0u;
-  for (int w = 0; w < nw; ++w) {
-    const uint32_t ws = sh.wsum[w];
-    off += w < wave ? ws : 0u;
-    cnt += ws;
-  }
-  if (cnt > (uint32_t)kMaxK) {  // uniform
-    whole();
-    return;
-  }
-#pragma unroll
-  for (int u = 0; u < kLoad; ++u) {
-    const int64_t i = tid + (int64_t)u * kFinThreads;
-    if (i < n && key[u] >= T) ss[off++] = ((uint64_t)key[u] << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)i);
-  }
-  __syncthreads();
-  // the candidates are in ss and the keys are no longer needed: survivors go to
-  // cl, the sort works in cl + 2 * kMaxK
-  select_sorted(ArraySrc{ss, (int64_t)cnt}, cnt, kk, m, sink, local, out, cl + 2 * kMaxK, cl, sh, s_cnt, false);
 }
 
 // Wave-wide minimum and maximum of 32-bit values (in every lane): DPP row
@@ -1216,6 +1176,152 @@ struct QuadScores {  // quad_order(G, n) true
   }
 };
 
+// A row's output: ranked values below got are written (their tokens also to
+// `ranked`, LDS of k int32, if non-null), then the fixed positions.
+struct RowOut {
+  int64_t *p;
+  int64_t kk, m, sink, local;
+  int32_t *ranked;
+  int got;
+  __device__ __forceinline__ void put(int rank, uint64_t x) const {
+    if (rank >= got) return;
+    const uint32_t tok = 0xFFFFFFFFu - (uint32_t)x;
+    p[rank] = (int64_t)tok;
+    if (ranked) ranked[rank] = (int32_t)tok;
+  }
+  // true where the tokens are in `ranked` too
+  __device__ __forceinline__ bool finish() const {
+    write_fixed(p, got, kk, m, sink, local);
+    if (ranked) {  // the same tokens as write_fixed's
+      for (int i = got + (int)threadIdx.x; i < (int)kk; i += kFinThreads) ranked[i] = 0;
+      for (int i = threadIdx.x; i < (int)(sink + local); i += kFinThreads)
+        ranked[kk + i] = (int32_t)((i < sink) ? (int64_t)i : (m - local + (i - sink)));
+    }
+    return ranked != nullptr;
+  }
+};
+
+// Ranks the cnt <= 4096 candidates in cl (also the sort's scratch) into out.
+template <bool LINEAR>
+__device__ __forceinline__ void rank_cands(uint64_t *cl, uint32_t cnt, RowOut &out, RangeShared &sh) {
+  int nlim = kWave;
+  while (nlim < (int)cnt) nlim <<= 1;
+  out.got = (int64_t)cnt < out.kk ? (int)cnt : (int)out.kk;
+  const auto rank_all = [&](auto per) {
+    constexpr int E = decltype(per)::value;
+    uint64_t v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const uint32_t i = threadIdx.x + (uint32_t)e * kFinThreads;
+      v[e] = i < cnt ? cl[i] : 0ull;
+    }
+    __syncthreads();
+    bin_rank_desc<E, LINEAR>(v, (int)cnt, out.got, cl, sh, nlim, [&](int rank, uint64_t x) { out.put(rank, x); });
+  };
+  if (cnt <= (uint32_t)(2 * kFinThreads)) rank_all(std::integral_constant<int, 2>{});
+  else rank_all(std::integral_constant<int, 4>{});
+}
+
+// Exact top kk of a short row, read whole: up to 4096 tokens are ranked at once
+// (E values per thread); longer rows first keep the scores of the bin that
+// holds the kk-th largest and above, 2048 linear bins over the finite scores'
+// range (kk and a few of them for spread scores; rows whose kept scores
+// outgrow the sort are selected by range).
+template <int E, typename Scores>
+__device__ __forceinline__ bool rowrank_row(const Scores &rs, int64_t n, RowOut &out, uint64_t *cl, uint64_t *ss,
+                                            RangeShared &sh, uint32_t &s_cnt) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = kFinThreads >> 6;
+  const int64_t kk = out.kk, sink = out.sink;
+  const int64_t lstart = (out.m - out.local) > 0 ? (out.m - out.local) : 0;
+  uint32_t key[E];  // 0: no candidate (below every score's key)
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int64_t i = tid + (int64_t)e * kFinThreads;
+    key[e] = i < n ? masked_key(rs, i, sink, lstart) : 0u;
+  }
+  const auto k64 = [&](int e) { return key[e] ? k64_of(key[e], tid + (int64_t)e * kFinThreads) : 0ull; };
+  if constexpr (E <= 4) {
+    uint64_t v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = k64(e);
+    int nlim = kWave;
+    while (nlim < (int)n) nlim <<= 1;
+    out.got = (int)kk;
+    bin_rank_desc<E, true>(v, (int)n, out.got, cl, sh, nlim, [&](int rank, uint64_t x) { out.put(rank, x); });
+    return out.finish();
+  }
+  uint32_t mn = ~0u, mx = 0u;
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (finite_key(key[e])) {
+      mn = min(mn, key[e]);
+      mx = max(mx, key[e]);
+    }
+  wave_minmax_u32(mn, mx);
+  if (lane == 0) {
+    sh.wmin[wave] = mn;
+    sh.wmax[wave] = mx;
+  }
+  sh.hist[tid] = sh.hist[tid + kFinThreads] = 0u;
+  __syncthreads();
+  uint32_t lo = ~0u, hi = 0u;
+  for (int w = 0; w < nw; ++w) {
+    lo = min(lo, (uint32_t)sh.wmin[w]);
+    hi = max(hi, (uint32_t)sh.wmax[w]);
+  }
+  const LinearBins bins(lo, hi);
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (key[e]) atomicAdd(&sh.hist[bins.of(key[e])], 1u);
+  __syncthreads();
+  // running counts from the top bin down: thread t holds bins 2047 - 2t, 2046 - 2t
+  const uint32_t c0 = sh.hist[kBins - 1 - 2 * tid], c1 = sh.hist[kBins - 2 - 2 * tid], c = c0 + c1;
+  const uint32_t wi = wave_incl_scan_u32(c);
+  if (lane == kWave - 1) sh.wsum[wave] = wi;
+  __syncthreads();
+  uint32_t above = wi - c;
+  for (int w = 0; w < wave; ++w) above += sh.wsum[w];
+  const uint32_t need = (uint32_t)kk;
+  if (above < need && above + c0 >= need) sh.hsel = (uint32_t)(kBins - 1 - 2 * tid);
+  if (above + c0 < need && above + c >= need) sh.hsel = (uint32_t)(kBins - 2 - 2 * tid);
+  __syncthreads();
+  const uint32_t b = sh.hsel;  // set: n >= kk scores are counted
+  uint32_t own = 0u;
+#pragma unroll
+  for (int e = 0; e < E; ++e) own += key[e] && bins.of(key[e]) >= b ? 1u : 0u;
+  const uint32_t oi = wave_incl_scan_u32(own);
+  if (lane == kWave - 1) sh.wsum[wave] = oi;
+  __syncthreads();
+  uint32_t off = oi - own, cnt = 0u;
+  for (int w = 0; w < nw; ++w) {
+    const uint32_t s = sh.wsum[w];
+    off += w < wave ? s : 0u;
+    cnt += s;
+  }
+  if (cnt > (uint32_t)(4 * kFinThreads)) {  // uniform: ties, or a range that outliers stretch
+    const auto src = index_src([&](int64_t i) { return k64_of(masked_key(rs, i, sink, lstart), i); }, n);
+    select_sorted(src, n, kk, out.m, sink, out.local, out.p, cl, ss, sh, s_cnt, true);
+    return false;
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (key[e] && bins.of(key[e]) >= b) cl[off++] = k64(e);
+  __syncthreads();
+  // scores of both signs: linear bins again; a tail of positive ones: the keys'
+  if (bins.positive(b)) rank_cands<false>(cl, cnt, out, sh);
+  else rank_cands<true>(cl, cnt, out, sh);
+  return out.finish();
+}
+// The rows that rowrank_row takes: short ones, and those with few groups per
+// selected key, whose maxima bound little.  sink_local_topk of 32 rows, us, by
+// group maxima (with their pass) and read whole: n = 1000, kk = 92 17.2; 4.9, 4096,
+// 476 20; 7.8, 8192, 264 13.9; 11.2, 8192, 476 15.9; 11.3, 14000, 476 15.2; 17.4, 16384,
+// 988 21.5; 18.7, 32768, 1064 21.6; 26.0, 32768, 2012 38.0; 26.7.
+inline bool rowrank_takes(int64_t n, int64_t kk) {
+  const int64_t ngrp = cdiv(n, kGroupTok);
+  return n <= 4 * kFinThreads || (n <= 8 * kFinThreads && ngrp <= 2 * kk) || (n <= kRowSelectMax && 4 * ngrp <= 5 * kk);
+}
+
 // Exact top kk of short score rows whose 16-token group maxima the scan
 // wrote beside them (gmax [rows, ceil(n / 16)]: the largest masked key of each
 // group).  T, a lower bound of the kk-th largest group maximum, bounds the
@@ -1232,16 +1338,14 @@ static_assert(kGmaxSelectMax / kGroupTok <= 65536, "group numbers fit 16 bits");
 // call returns true.
 template <int kPer, typename Scores>
 __device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint32_t *__restrict__ gmax, int64_t n,
-                                                   int64_t m, int64_t k, int64_t sink, int64_t local,
-                                                   int64_t *__restrict__ idx, uint64_t *cl, uint64_t *ss,
-                                                   RangeShared &sh, uint32_t &s_cnt, int32_t *ranked = nullptr) {
+                                                   RowOut &out, uint64_t *cl, uint64_t *ss, RangeShared &sh,
+                                                   uint32_t &s_cnt) {
   uint16_t *glist = reinterpret_cast<uint16_t *>(ss);  // ss holds the survivors only after the groups are read
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = kFinThreads >> 6;
   const int64_t row = blockIdx.x;
+  const int64_t kk = out.kk, m = out.m, sink = out.sink, local = out.local;
   const int64_t lstart = (m - local) > 0 ? (m - local) : 0;
-  const int64_t kk = k - sink - local;
   const int ngrp = (int)cdiv(n, kGroupTok);
-  int64_t *out = idx + row * k;
   uint32_t gm[kPer];
 #pragma unroll
   for (int u = 0; u < kPer; ++u) {
@@ -1276,7 +1380,7 @@ __device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint3
   }
   if (ngr > (uint32_t)kGroupList) {  // uniform: ties around T
     const auto src = index_src([&](int64_t i) { return k64_of(masked_key(rs, i, sink, lstart), i); }, n);
-    select_sorted(src, n, kk, m, sink, local, out, cl, ss, sh, s_cnt, true);
+    select_sorted(src, n, kk, m, sink, local, out.p, cl, ss, sh, s_cnt, true);
     return false;
   }
   // their keys >= T, one group per thread, placed by a workgroup prefix sum
@@ -1314,39 +1418,20 @@ __device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint3
   }
   if (cnt > (uint32_t)kCandLds) {  // uniform: ties around T
     const auto src = index_src([&](int64_t i) { return k64_of(masked_key(rs, i, sink, lstart), i); }, n);
-    select_sorted(src, n, kk, m, sink, local, out, cl, ss, sh, s_cnt, true);
+    select_sorted(src, n, kk, m, sink, local, out.p, cl, ss, sh, s_cnt, true);
     return false;
   }
-  if (cnt > (uint32_t)(2 * kFinThreads)) {
-    select_sorted(ArraySrc{cl, (int64_t)cnt}, cnt, kk, m, sink, local, out, cl, ss, sh, s_cnt, false);
+  if (cnt > (uint32_t)(4 * kFinThreads)) {
+    select_sorted(ArraySrc{cl, (int64_t)cnt}, cnt, kk, m, sink, local, out.p, cl, ss, sh, s_cnt, false);
     return false;
   }
-  // at most 2048 candidates: one sort ranks them, the first kk are written
-  uint64_t v2[2];
-  v2[0] = (uint32_t)tid < cnt ? cl[tid] : 0ull;  // zero: padding (below every K64)
-  v2[1] = (uint32_t)(tid + kFinThreads) < cnt ? cl[tid + kFinThreads] : 0ull;
-  __syncthreads();  // cl is the sort scratch from here
-  int nlim = kWave;
-  while (nlim < (int)cnt) nlim <<= 1;
-  const int got = (int64_t)cnt < kk ? (int)cnt : (int)kk;
-  bin_rank_desc<2>(v2, (int)cnt, cl, sh, nlim, [&](int rank, uint64_t x) {
-    if (rank < got) {
-      const uint32_t tok = 0xFFFFFFFFu - (uint32_t)x;
-      out[rank] = (int64_t)tok;
-      if (ranked) ranked[rank] = (int32_t)tok;
-    }
-  });
-  write_fixed(out, got, kk, m, sink, local);
-  if (ranked) {  // the same tokens as write_fixed's
-    for (int i = got + tid; i < (int)kk; i += kFinThreads) ranked[i] = 0;
-    for (int i = tid; i < (int)(sink + local); i += kFinThreads)
-      ranked[kk + i] = (int32_t)((i < sink) ? (int64_t)i : (m - local + (i - sink)));
-  }
-  return ranked != nullptr;
+  rank_cands<false>(cl, cnt, out, sh);  // at most 4096 candidates: one sort ranks them
+  return out.finish();
 }
 
-// The selection of rowselect_gmax_row, one workgroup per row.  ATTN (the
-// decode step's selection + attention, k <= 512, rows in device memory): the
+// A row's selection, one workgroup per row: rowrank_row with E tokens per thread,
+// or (E = 0) rowselect_gmax_row with kPer groups per thread.  ATTN (the decode
+// step's selection + attention, k <= 512, rows in device memory): the
 // workgroup then runs the attention of its query head over the k indices it
 // wrote, exactly as gather_attention's attn_stream_kernel does for one split
 // (16 waves of 32 positions), so out equals gather_attention's output.
@@ -1357,11 +1442,11 @@ struct RowAttn {
   float scale;
   float *out;      // [rows, D] fp32
 };
-template <typename Scores, bool ATTN, int kPer>
-__global__ __launch_bounds__(kFinThreads) void rowselect_gmax_kernel(const float *__restrict__ scores, int64_t G,
-                                                                     const uint32_t *__restrict__ gmax, int64_t n,
-                                                                     int64_t m, int64_t k, int64_t sink, int64_t local,
-                                                                     int64_t *__restrict__ idx, RowAttn ra) {
+template <typename Scores, bool ATTN, int kPer, int E>
+__global__ __launch_bounds__(kFinThreads) void rowselect_kernel(const float *__restrict__ scores, int64_t G,
+                                                                const uint32_t *__restrict__ gmax, int64_t n, int64_t m,
+                                                                int64_t k, int64_t sink, int64_t local,
+                                                                int64_t *__restrict__ idx, RowAttn ra) {
   __shared__ uint64_t cl[kCandLds];
   __shared__ uint64_t ss[kMaxK];
   __shared__ RangeShared sh;
@@ -1369,10 +1454,14 @@ __global__ __launch_bounds__(kFinThreads) void rowselect_gmax_kernel(const float
   // ATTN: the ranked tokens also in LDS, in cl's upper half (past the sort's
   // scratch and the attention's triples)
   int32_t *ranked = ATTN ? reinterpret_cast<int32_t *>(cl + kCandLds / 2) : nullptr;
-  static_assert(kCandLds / 2 >= 2 * 2 * kFinThreads + kBins && 2 * (kCandLds / 2) >= kMaxK + kFinThreads,
+  static_assert(kCandLds / 2 >= 4 * kFinThreads + kBins && kCandLds / 2 >= 2 * 4 * kFinThreads &&
+                    2 * (kCandLds / 2) >= kMaxK + kFinThreads,
                 "the ranked tokens lie past the sort's scratch and hold k of them");
-  const bool in_lds = rowselect_gmax_row<kPer>(Scores(scores, n, G), gmax, n, m, k, sink, local, idx, cl, ss, sh,
-                                               s_cnt, ranked);
+  RowOut ro{idx + blockIdx.x * k, k - sink - local, m, sink, local, ranked, 0};
+  const Scores rs(scores, n, G);
+  bool in_lds;
+  if constexpr (E > 0) in_lds = rowrank_row<E>(rs, n, ro, cl, ss, sh, s_cnt);
+  else in_lds = rowselect_gmax_row<kPer>(rs, gmax, n, ro, cl, ss, sh, s_cnt);
   if constexpr (ATTN) {
     constexpr int NW = kFinThreads / kWave;
     static_assert(NW == 16, "one attention split of 16 waves");
@@ -1415,7 +1504,7 @@ __global__ __launch_bounds__(kFinThreads) void rank_list_kernel(const uint64_t *
   int nlim = kWave;
   while (nlim < (int)kk) nlim <<= 1;
   int64_t *out = idx + row * k;
-  bin_rank_desc<E>(v, (int)kk, cl, sh, nlim,
+  bin_rank_desc<E>(v, (int)kk, (int)kk, cl, sh, nlim,
                    [&](int rank, uint64_t x) { out[rank] = (int64_t)(0xFFFFFFFFu - (uint32_t)x); });
   write_fixed(out, (int)kk, kk, m, sink, local);
 }
@@ -1537,32 +1626,33 @@ int launch_finalize_fused(const sc::ScanArgs &a, const sc::Emit &em, int64_t row
   return launch_status("finalize_fused_kernel");
 }
 
-int launch_rowselect(const float *scores, int64_t rows, int64_t n, int64_t m, int64_t k, int64_t sink, int64_t local,
-                     int64_t *idx, hipStream_t st) {
-  rowselect_kernel<<<(unsigned)rows, kFinThreads, 0, st>>>(scores, n, m, k, sink, local, idx);
-  return launch_status("rowselect_kernel");
-}
-
 namespace {
-// Group maxima per thread: 2 (rows of up to 32768 tokens) or 8.
 template <typename Scores, bool ATTN>
-int launch_gmax(const float *scores, int64_t G, const uint32_t *gmax, int64_t rows, int64_t n, int64_t m, int64_t k,
-                int64_t sink, int64_t local, int64_t *idx, const RowAttn &ra, hipStream_t st) {
-  const unsigned g = (unsigned)rows;
+int launch_row_select(const float *scores, int64_t G, const uint32_t *gmax, int64_t rows, int64_t n, int64_t m, int64_t k,
+                      int64_t sink, int64_t local, int64_t *idx, const RowAttn &ra, hipStream_t st) {
   static_assert(kRowSelectMax == 2 * kFinThreads * kGroupTok && kGmaxSelectMax == 8 * kFinThreads * kGroupTok, "groups");
-  if (n > kGmaxSelectMax) return fail(FATHOM_ERR_INVALID, "rowselect_gmax: n=%lld exceeds %lld", (long long)n, (long long)kGmaxSelectMax);
-  if (n <= kRowSelectMax)
-    rowselect_gmax_kernel<Scores, ATTN, 2><<<g, kFinThreads, 0, st>>>(scores, G, gmax, n, m, k, sink, local, idx, ra);
-  else
-    rowselect_gmax_kernel<Scores, ATTN, 8><<<g, kFinThreads, 0, st>>>(scores, G, gmax, n, m, k, sink, local, idx, ra);
-  return launch_status("rowselect_gmax_kernel");
+  if (n > kGmaxSelectMax)
+    return fail(FATHOM_ERR_INVALID, "row selection: n=%lld exceeds %lld", (long long)n, (long long)kGmaxSelectMax);
+  const unsigned g = (unsigned)rows;
+  const auto run = [&](auto kernel) { kernel<<<g, kFinThreads, 0, st>>>(scores, G, gmax, n, m, k, sink, local, idx, ra); };
+  if (rowrank_takes(n, k - sink - local)) {
+    if (n <= kFinThreads) run(rowselect_kernel<Scores, ATTN, 0, 1>);
+    else if (n <= 4 * kFinThreads) run(rowselect_kernel<Scores, ATTN, 0, 4>);
+    else if (n <= 8 * kFinThreads) run(rowselect_kernel<Scores, ATTN, 0, 8>);
+    else run(rowselect_kernel<Scores, ATTN, 0, 32>);
+  } else if (n <= kRowSelectMax) {
+    run(rowselect_kernel<Scores, ATTN, 2, 0>);
+  } else {
+    run(rowselect_kernel<Scores, ATTN, 8, 0>);
+  }
+  return launch_status("rowselect_kernel");
 }
 }  // namespace
 
 int launch_rowselect_gmax(const float *scores, const uint32_t *gmax, int64_t rows, int64_t G, int64_t n, int64_t m,
                           int64_t k, int64_t sink, int64_t local, int64_t *idx, hipStream_t st) {
-  if (!quad_order(G, n)) return launch_gmax<TileScores, false>(scores, G, gmax, rows, n, m, k, sink, local, idx, RowAttn{}, st);
-  return launch_gmax<QuadScores, false>(scores, G, gmax, rows, n, m, k, sink, local, idx, RowAttn{}, st);
+  if (!quad_order(G, n)) return launch_row_select<TileScores, false>(scores, G, gmax, rows, n, m, k, sink, local, idx, RowAttn{}, st);
+  return launch_row_select<QuadScores, false>(scores, G, gmax, rows, n, m, k, sink, local, idx, RowAttn{}, st);
 }
 
 int launch_rowselect_gmax_attn(const float *scores, const uint32_t *gmax, int64_t rows, int64_t n, int64_t m, int64_t k,
@@ -1571,8 +1661,8 @@ int launch_rowselect_gmax_attn(const float *scores, const uint32_t *gmax, int64_
   if (k > kFinThreads / 2) return fail(FATHOM_ERR_INVALID, "rowselect_gmax_attn: k=%lld exceeds 512", (long long)k);
   RowAttn ra{q, G, attn::RowSrc{(const char *)K, (const char *)V, nullptr, nullptr, cap, 0, n, 2 * attn::kAttnD}, scale,
              out};
-  if (!quad_order(G, n)) return launch_gmax<TileScores, true>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st);
-  return launch_gmax<QuadScores, true>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st);
+  if (!quad_order(G, n)) return launch_row_select<TileScores, true>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st);
+  return launch_row_select<QuadScores, true>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st);
 }
 
 int launch_rank_list(const uint64_t *sel, int64_t P, int64_t rows, int64_t kk, int64_t m, int64_t k, int64_t sink,
@@ -1676,8 +1766,16 @@ extern "C" int fathom_sink_local_topk(const float *scores, int64_t rows, int64_t
   int64_t samp_cap = 0, S = 1;
   topk_layout(rows, n, k, false, static_cast<char *>(workspace), &samp, &samp_cap, &s, &S);
   s.kk = (uint32_t)kk;
-  if (n <= kRowSelectMax) return launch_rowselect(scores, rows, n, m, k, sink, local, idx, st);
   const int64_t lstart = (m - local) > 0 ? (m - local) : 0;
+  if (n <= kGmaxSelectMax) {
+    uint32_t *gmax = static_cast<uint32_t *>(workspace);  // 4 bytes per 16 scores, the layout has 8 per score
+    if (!rowrank_takes(n, kk)) {
+      group_max_kernel<<<dim3((unsigned)cdiv(n, 256 * kGmaxPer), (unsigned)rows), 256, 0, st>>>(scores, n, sink, lstart, gmax);
+      rc = launch_status("group_max_kernel");
+    }
+    return rc ? rc
+              : launch_row_select<RowScores, false>(scores, 1, gmax, rows, n, m, k, sink, local, idx, RowAttn{}, st);
+  }
   const int64_t r_hi = topk_hi_rank(n, S, kk, kTileTok);
   rc = launch_sample_scores(scores, rows, n, S, sink, lstart, samp, samp_cap, st);
   if (rc) return rc;

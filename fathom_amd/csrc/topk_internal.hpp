@@ -38,9 +38,8 @@ constexpr int64_t kMaxSample = 65536; // sampled keys per row (held in registers
 // expected first-pass candidates per row, in units of kk: kAlphaX2 / 2
 constexpr int64_t kAlphaX2 = 5;
 
-// Score rows up to this length (their 32-bit keys fit in one workgroup's LDS)
-// select their top kk in one kernel, one workgroup per row, instead of
-// sample -> select -> filter -> finalize: fewer launches for short rows.
+// Rows up to this length have their group maxima held two per thread (longer ones,
+// up to kGmaxSelectMax, eight), and are kept in the drop-in order by the fused scan.
 constexpr int64_t kRowSelectMax = 32768;
 
 // Longest rows that the fused scan + top-k selects from its scores' 16-token group
@@ -166,10 +165,7 @@ int launch_filter_scores(const float *scores, int64_t rows, int64_t n, int64_t s
 // Either layout (s.rc1 set: regions).
 int launch_finalize(int64_t rows, int64_t m, int64_t k, int64_t sink, int64_t local, TopkSel s, int64_t *idx,
                     hipStream_t st);
-// Exact top kk of whole score rows [rows, n] (n <= kRowSelectMax).
-int launch_rowselect(const float *scores, int64_t rows, int64_t n, int64_t m, int64_t k, int64_t sink, int64_t local,
-                     int64_t *idx, hipStream_t st);
-// The same from the rows' 16-token group maxima (gmax [rows, ceil(n / 16)]
+// Exact top kk of score rows from their 16-token group maxima (gmax [rows, ceil(n / 16)]
 // largest masked keys; scores in the fused scan's order): only the groups that
 // can hold a top-kk key are read.
 int launch_rowselect_gmax(const float *scores, const uint32_t *gmax, int64_t rows, int64_t G, int64_t n, int64_t m,

@@ -88,3 +88,50 @@ def test_host_resident_staged_scan_equals_hbm(n, G, monkeypatch):
         off.free_host(h2)
     for a, b, c in zip(got, want, ref):
         assert torch.equal(a, b) and torch.equal(a, c)
+
+
+def _score_rows(kind, rows, n, seed):
+    rng = np.random.default_rng(seed)
+    s = rng.standard_normal((rows, n)).astype(np.float32)
+    if kind == "equal":
+        s[:] = -1.5
+    elif kind == "specials":
+        for v in (np.nan, np.inf, -np.inf, 0.0, -0.0, 3e38, -3e38, 1e-45):
+            s[:, rng.integers(0, n, max(1, n // 20))] = v
+    elif kind == "outliers":
+        s[:, rng.integers(0, n, 3)] = 1e30
+        s[0] = np.abs(s[0])
+    elif kind == "lowest":  # more -inf than finite scores
+        s[:, rng.random(n) < 0.8] = -np.inf
+    elif kind == "steps":
+        s = np.round(s * 2) / 2
+    return s
+
+
+@pytest.mark.parametrize("n,k,sink,local,extra", [
+    (64, 60, 4, 32, 0), (50, 50, 0, 0, 0), (1000, 1000, 4, 32, 0), (1024, 128, 4, 32, 3), (1025, 700, 0, 1, 0),
+    (4096, 2084, 4, 32, 0), (4097, 257, 1, 0, 0), (4097, 300, 4, 32, 40), (8192, 548, 4, 32, 0), (8193, 549, 4, 32, 0),
+    (8193, 512, 4, 32, 0), (16384, 1060, 4, 32, 0), (32192, 2048, 4, 32, 0), (32768, 2084, 4, 32, 0), (32768, 2048, 0, 0, 0),
+    (32769, 512, 4, 32, 0), (40003, 2084, 4, 32, 31), (131072, 512, 4, 32, 0), (131071, 2084, 4, 32, 0),
+    (131073, 512, 4, 32, 0)])
+def test_score_rows_at_every_route(n, k, sink, local, extra):
+    print(f"[row-select] n={n} k={k} sink={sink} local={local}", flush=True)
+    for i, kind in enumerate(("normal", "equal", "specials", "outliers", "lowest", "steps")):
+        s = _score_rows(kind, 3, n, n + i)
+        got = bp.sink_local_topk(torch.from_numpy(s).to(DEV), k, sink, local, m=n + extra).cpu().numpy()
+        np.testing.assert_array_equal(got, O.sink_local_topk(s, k, sink, local, m=n + extra), err_msg=kind)
+
+
+@pytest.mark.parametrize("n,k", [(700, 128), (3000, 512), (6000, 512), (8192, 600), (20000, 1500), (30001, 2048)])
+def test_fused_selection_of_short_rows(n, k):
+    print(f"[row-select fused] n={n} k={k}", flush=True)
+    for BH, G in ((1, 1), (2, 5), (24, 4)):
+        x = W.synth_layer(BH, n, G, seed=n, device=DEV, kdtype=torch.bfloat16)
+        g = ((x["q"] ** 2) * x["var"][:, None, :]).sum(1)
+        st = bp.PlaneStore(x["K"], keep_code=False)
+        plan = bp.make_plan(g, 48.0)
+        want = _oracle_topk(st.scan(x["q"], plan), k, 4, 32, n)
+        assert torch.equal(st.scan_topk(x["q"], plan, k, 4, 32).cpu(), want)
+        idx, out = st.plan_scan_topk_attention(x["q"], g, 48.0, k, x["K"], x["K"], 4, 32)
+        ref, _ = off.gather_attention(x["q"], idx, n, x["K"], x["K"], n)
+        assert torch.equal(idx.cpu(), want) and torch.equal(out, ref)
