@@ -14,9 +14,15 @@ constexpr int kPartStride = kAttnD + 2;    // (max, sum, weighted V[128])
 constexpr int kStreamWide = 16;            // waves of a workgroup that takes 512 positions of a head
 
 // gather_attention's choice for rows per selected position: workgroups of 16
-// waves (512 positions, one split per head for k <= 512) when that gives the
-// chip about 128 workgroups or more, else of 4 waves (128 positions).
-inline bool attn_wide(int64_t BH, int64_t G, int64_t k) { return BH * G * cdiv(k, (int64_t)(32 * kStreamWide)) >= 96; }
+// waves (512 positions) for heads of 129 to 512 -- one split, no merge launch --
+// and for longer ones when that gives the chip about 128 workgroups or more; else
+// of 4 waves (128 positions).  us, 4 waves and merge; 16 waves: 1 to 32 heads of
+// k = 512 9.0-9.4; 6.4-6.7, 64 heads 9.5; 6.8, 8 heads of 2048 9.3; 12.2, 32 heads of 1024
+// 9.5; 12.3, 32 of 4096 18.7; 18.3.
+inline bool attn_wide(int64_t BH, int64_t G, int64_t k) {
+  constexpr int64_t kOne = 32 * kStreamWide;
+  return k <= kOne ? k > 128 : BH * G * cdiv(k, kOne) >= 96;
+}
 
 __device__ __forceinline__ uint32_t tok_key(int64_t v) {
   return v < 0 ? kTokNeg : (uint32_t)(v < (int64_t)kTokNeg - 1 ? v : (int64_t)kTokNeg - 1);
@@ -65,32 +71,16 @@ __device__ __forceinline__ float across_rows(float v) {
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(1))) u32x4 *gptr4;
 
-// Attention of one query head's positions streamed through registers (no
-// union, rows in device memory): a workgroup of NW waves takes positions
-// [32 NW s, 32 NW (s + 1)) of the head's k selected tokens tok_at(j) of row
-// bh, each with a count of one (a row selected twice counts twice).  Wave w
-// holds 32 of them: lane l works on dims 8 (l & 15) .. + 7 of the rows of
-// positions 4 t + (l >> 4), t < 8.  Every K and V row piece of the wave is
-// requested before the first score is formed (K first), so the scores follow
-// the K rows as they arrive and the values the V rows.  A position without a
-// row (negative token, beyond the cache) scores 0 and reads kZeroRow, which
-// adds nothing to V.  The wave's softmax is taken against its own maximum, so no
-// barrier is needed until the waves' (M, sum, weighted V) triples are
-// combined (LDS wm[NW], wl[NW], wo[NW][kAttnD]).  single: the workgroup
-// writes the head's output out_row; else its (M, sum, weighted V) triple to
-// pb for attn_merge_kernel.
 constexpr int kStreamTok = 32;               // positions per wave
 constexpr uint64_t kRowBytes = 2 * kAttnD;   // a bf16 row
 __device__ const u32x4 kZeroRow[kRowBytes / 16] = {};
-template <int NW, bool REC, typename TokAt>
-__device__ __forceinline__ void attn_stream_block(const float *__restrict__ qg, TokAt tok_at, int64_t k, int64_t s,
-                                                  int64_t bh, const RowSrc &rs, float scale, float *wm, float *wl,
-                                                  float (*wo)[kAttnD], float *__restrict__ out_row,
-                                                  float *__restrict__ pb, bool single) {
+// A wave's 32 positions: its (M, sum, weighted V).
+template <bool REC, typename TokAt>
+__device__ __forceinline__ void attn_stream_wave(const float *__restrict__ qg, TokAt tok_at, int64_t k, int64_t p0,
+                                                 int64_t bh, const RowSrc &rs, float scale, int lane, float &wm, float &wl,
+                                                 float (&wo)[kAttnD]) {
   constexpr int kSteps = kStreamTok / 4;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int rg = lane >> 4, ds = lane & 15;
-  const int64_t p0 = (s * NW + wave) * kStreamTok + rg;
   const float4 qa = *reinterpret_cast<const float4 *>(qg + 8 * ds);
   const float4 qb = *reinterpret_cast<const float4 *>(qg + 8 * ds + 4);
   int64_t tk[kSteps];  // positions past k read the last one (and are masked)
@@ -167,12 +157,48 @@ __device__ __forceinline__ void attn_stream_block(const float *__restrict__ qg, 
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = across_rows<false>(o[e]);
   if (rg == 0) {
-    *reinterpret_cast<float4 *>(&wo[wave][8 * ds]) = make_float4(o[0], o[1], o[2], o[3]);
-    *reinterpret_cast<float4 *>(&wo[wave][8 * ds + 4]) = make_float4(o[4], o[5], o[6], o[7]);
+    *reinterpret_cast<float4 *>(&wo[8 * ds]) = make_float4(o[0], o[1], o[2], o[3]);
+    *reinterpret_cast<float4 *>(&wo[8 * ds + 4]) = make_float4(o[4], o[5], o[6], o[7]);
   }
   if (lane == 0) {
-    wm[wave] = m;
-    wl[wave] = l;
+    wm = m;
+    wl = l;
+  }
+}
+
+// Attention of one query head's positions streamed through registers (no
+// union, rows in device memory): a workgroup of NW waves takes positions
+// [32 NW s, 32 NW (s + 1)) of the head's k selected tokens tok_at(j) of row
+// bh, each with a count of one (a row selected twice counts twice).  Wave w
+// holds 32 of them: lane l works on dims 8 (l & 15) .. + 7 of the rows of
+// positions 4 t + (l >> 4), t < 8.  Every K and V row piece of the wave is
+// requested before the first score is formed (K first), so the scores follow
+// the K rows as they arrive and the values the V rows.  A position without a
+// row (negative token, beyond the cache) scores 0 and reads kZeroRow, which
+// adds nothing to V.  The wave's softmax is taken against its own maximum, so no
+// barrier is needed until the waves' (M, sum, weighted V) triples are
+// combined (LDS wm[NW], wl[NW], wo[NW][kAttnD]).  single: the workgroup
+// writes the head's output out_row; else its (M, sum, weighted V) triple to
+// pb for attn_merge_kernel.
+template <int NW, bool REC, typename TokAt>
+__device__ __forceinline__ void attn_stream_block(const float *__restrict__ qg, TokAt tok_at, int64_t k, int64_t s,
+                                                  int64_t bh, const RowSrc &rs, float scale, float *wm, float *wl,
+                                                  float (*wo)[kAttnD], float *__restrict__ out_row,
+                                                  float *__restrict__ pb, bool single) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rg = lane >> 4, ds = lane & 15;
+  const int64_t p0 = (s * NW + wave) * kStreamTok + rg;
+  if ((s * NW + wave) * kStreamTok >= k) {  // uniform per wave: no position
+    if (rg == 0) {
+      *reinterpret_cast<float4 *>(&wo[wave][8 * ds]) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      *reinterpret_cast<float4 *>(&wo[wave][8 * ds + 4]) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    if (lane == 0) {
+      wm[wave] = -INFINITY;
+      wl[wave] = 0.0f;
+    }
+  } else {
+    attn_stream_wave<REC>(qg, tok_at, k, p0, bh, rs, scale, lane, wm[wave], wl[wave], wo[wave]);
   }
   __syncthreads();
   if (tid < kAttnD) {

@@ -564,11 +564,13 @@ __global__ __launch_bounds__(NW * kWave) void attn_stream_kernel(const float *__
 // out[bh, g, d] = sum_s O_s e^(M_s - M) / sum_s L_s e^(M_s - M) over the
 // row's splits, by every thread for its own dimension d with no barrier:
 // M = max_s M_s first, then the weighted sums in split order, kB splits per
-// round of loads (rows of at most kB splits: one round).  A split where a head
+// round of loads (rows of at most kB splits: one round; kB of 4, 8 or 32, as every
+// slot's loads are issued: attention of 56 heads of 2048 positions, 4 splits, 17.1 ->
+// 14.5 us).  A split where a head
 // selected nothing (M_s = -inf) adds nothing to it.
+template <int kB>
 __global__ __launch_bounds__(kAttnD) void attn_merge_kernel(const float *__restrict__ part, int64_t G,
                                                             int64_t nsplit, float *__restrict__ out) {
-  constexpr int kB = 32;
   const int64_t r = blockIdx.x;  // bh * G + g
   const int64_t bh = r / G, g = r % G;
   const int d = threadIdx.x;
@@ -600,6 +602,14 @@ __global__ __launch_bounds__(kAttnD) void attn_merge_kernel(const float *__restr
     }
   }
   out[r * kAttnD + d] = O / L;
+}
+
+int launch_merge(const float *part, int64_t BH, int64_t G, int64_t nsplit, float *out, hipStream_t st) {
+  const unsigned g = (unsigned)(BH * G);
+  if (nsplit <= 4) attn_merge_kernel<4><<<g, kAttnD, 0, st>>>(part, G, nsplit, out);
+  else if (nsplit <= 8) attn_merge_kernel<8><<<g, kAttnD, 0, st>>>(part, G, nsplit, out);
+  else attn_merge_kernel<32><<<g, kAttnD, 0, st>>>(part, G, nsplit, out);
+  return launch_status("attn_merge_kernel");
 }
 
 int hash_bits(int64_t GK) {
@@ -744,8 +754,7 @@ extern "C" int fathom_gather_attention(const float *q, const int64_t *idx, int64
       attn_stream_kernel<4, false><<<grid, 4 * kWave, 0, st>>>(q, idx, G, k, rs, scale, out, part, ns);
     rc = launch_status("attn_stream_kernel");
     if (rc || ns == 1) return rc;
-    attn_merge_kernel<<<(unsigned)(BH * G), kAttnD, 0, st>>>(part, G, ns, out);
-    return launch_status("attn_merge_kernel");
+    return launch_merge(part, BH, G, ns, out, st);
   } else {
     // the union list (each distinct row read once), then its groups of kAttnTok tokens
     rc = launch_union(idx, BH, GK, k, n, w, n_unique, st);
@@ -763,6 +772,5 @@ extern "C" int fathom_gather_attention(const float *q, const int64_t *idx, int64
     rc = launch_status("attn_partial_kernel");
   }
   if (rc) return rc;
-  attn_merge_kernel<<<(unsigned)(BH * G), kAttnD, 0, st>>>(part, G, nsplit, out);
-  return launch_status("attn_merge_kernel");
+  return launch_merge(part, BH, G, nsplit, out, st);
 }

@@ -247,7 +247,7 @@ namespace fathom {
 int scan_topk_run(const float *q, int64_t BH, int64_t G, int64_t D, const int32_t *cls, const int32_t *clsn, int bmax,
                   int64_t units_max, const void *planes_sb, const void *scales_sb, int64_t n, int64_t nsb, int64_t sub, int64_t m,
                   int64_t k, int64_t sink, int64_t local, int64_t *idx, void *workspace, size_t workspace_bytes,
-                  int stages, void *stream) {
+                  int stages, void *stream, const AttnArgs *att) {
   int rc = check_scan(q, BH, G, D, cls, clsn, bmax, planes_sb, scales_sb, n, nsb, sub, "scan_topk");
   if (rc) return rc;
   if (!idx) return fail(FATHOM_ERR_INVALID, "scan_topk: null output");
@@ -268,8 +268,8 @@ int scan_topk_run(const float *q, int64_t BH, int64_t G, int64_t D, const int32_
   a.wt0 = 0;
   const int64_t nwt = cdiv(nblk, kWB);
   const int64_t um = units_bound(units_max, D, bmax);
-  if (kk > kSelMaxK) {
-    // kk beyond the LDS-resident selections: the scores in the workspace (the
+  if (kk > kSelMaxK && !group_select_takes(n, kk)) {
+    // kk or rows beyond the one-workgroup selections: the scores in the workspace (the
     // candidate stage), then the score-row chain and the wide selection over
     // its candidate lists (the finalize stage)
     Emit es{};
@@ -285,7 +285,7 @@ int scan_topk_run(const float *q, int64_t BH, int64_t G, int64_t D, const int32_
                                workspace_bytes - sb, st)
                : FATHOM_OK;
   }
-  if (n <= kGmaxSelectMax) {
+  if (group_select_takes(n, kk)) {
     // the scores and their 16-token group maxima in the workspace (the
     // candidate stage), then the rows selected in one launch from the groups
     // that can hold a top-kk key (the finalize stage)
@@ -294,7 +294,7 @@ int scan_topk_run(const float *q, int64_t BH, int64_t G, int64_t D, const int32_
       rc = launch_scores_max(a, nwt, BH, es, um, st);
       if (rc) return rc;
     }
-    return (stages & FATHOM_STAGE_FINALIZE) ? launch_rowselect_gmax(es.out, es.gmax, rows, G, n, m, k, sink, local, idx, st)
+    return (stages & FATHOM_STAGE_FINALIZE) ? launch_rowselect_gmax(es.out, es.gmax, rows, G, n, m, k, sink, local, idx, att, st)
                                             : FATHOM_OK;
   }
   Emit em{};
@@ -323,7 +323,7 @@ int scan_topk_run(const float *q, int64_t BH, int64_t G, int64_t D, const int32_
   // workgroup of a row with fewer than kk candidates rescans it with T_lo
   a.wt_stride = 1;
   a.nwt = nwt;
-  return (stages & FATHOM_STAGE_FINALIZE) ? launch_finalize_fused(a, em, rows, m, k, sink, local, idx, st)
+  return (stages & FATHOM_STAGE_FINALIZE) ? launch_finalize_fused(a, em, rows, m, k, sink, local, idx, att, st)
                                           : FATHOM_OK;
 }
 }  // namespace fathom
@@ -364,18 +364,10 @@ extern "C" size_t fathom_plan_scan_topk_workspace_bytes(int64_t BH, int64_t G, i
 
 namespace fathom {
 namespace {
-// The attention of fathom_plan_scan_topk_attention (null: none).
-struct AttnOut {
-  const void *K, *V;
-  int64_t cap;
-  float scale;
-  float *out;
-};
-
 int plan_scan_topk_run(const float *q, const float *g, const float *budget, float budget_value, int64_t BH, int64_t G,
                        int64_t D, int bmax, int iters, int64_t units_max, const void *planes_sb, const void *scales_sb,
                        int64_t n, int64_t nsb, int64_t sub, int64_t m, int64_t k, int64_t sink, int64_t local,
-                       int64_t *idx, int8_t *t_out, void *workspace, size_t workspace_bytes, const AttnOut *att,
+                       int64_t *idx, int8_t *t_out, void *workspace, size_t workspace_bytes, const AttnArgs *att,
                        void *stream) {
   if (!g) return fail(FATHOM_ERR_INVALID, "plan_scan_topk: null pointer");
   if (iters < 0 || iters > 200) return fail(FATHOM_ERR_INVALID, "plan_scan_topk: iters=%d outside [0, 200]", iters);
@@ -391,7 +383,7 @@ int plan_scan_topk_run(const float *q, const float *g, const float *budget, floa
   hipStream_t st = (hipStream_t)stream;
   const int64_t kk = k - sink - local;
   const size_t sws = scan_topk_ws(rows, n, k, kk);
-  if (n > kGmaxSelectMax || kk == 0 || kk > kSelMaxK) {
+  if (kk == 0 || !group_select_takes(n, kk)) {
     // make_plan into the workspace, then the fused scan + top-k
     char *p = static_cast<char *>(workspace) + sws;
     int8_t *t = t_out ? t_out : reinterpret_cast<int8_t *>(p);
@@ -410,7 +402,7 @@ int plan_scan_topk_run(const float *q, const float *g, const float *budget, floa
     rc = make_plan_run(g, budget, budget_value, BH, D, bmax, iters, t, pairs, npairs, act, nact, cls, clsn, stream);
     if (rc) return rc;
     return scan_topk_run(q, BH, G, D, cls, clsn, bmax, units_max, planes_sb, scales_sb, n, nsb, sub, m, k, sink, local,
-                         idx, workspace, sws, FATHOM_STAGE_ALL, stream);
+                         idx, workspace, sws, FATHOM_STAGE_ALL, stream, att);
   }
   // every workgroup of the scan plans its row in the prologue
   // (the plan kernel's arithmetic), then the rows are selected as in scan_topk
@@ -427,10 +419,7 @@ int plan_scan_topk_run(const float *q, const float *g, const float *budget, floa
   const Emit es = group_max_emit(rows, n, m, sink, local, workspace);
   rc = launch_scores_max(a, cdiv(nblk, kWB), BH, es, units_bound(units_max, D, bmax), st);
   if (rc) return rc;
-  if (att)  // the selection's workgroups go on to their head's attention
-    return launch_rowselect_gmax_attn(es.out, es.gmax, rows, n, m, k, sink, local, idx, q, G, att->K, att->V, att->cap,
-                                      att->scale, att->out, st);
-  return launch_rowselect_gmax(es.out, es.gmax, rows, G, n, m, k, sink, local, idx, st);
+  return launch_rowselect_gmax(es.out, es.gmax, rows, G, n, m, k, sink, local, idx, att, st);
 }
 }  // namespace
 }  // namespace fathom
@@ -465,13 +454,13 @@ extern "C" int fathom_plan_scan_topk_attention(const float *q, const float *g, c
     return fail(FATHOM_ERR_WORKSPACE, "plan_scan_topk_attention: workspace %zu bytes, need %zu", workspace_bytes, need);
   const size_t pws = fathom_plan_scan_topk_workspace_bytes(BH, G, D, bmax, n, k, sink, local);
   const int64_t kk = k - sink - local;
-  // fused where gather_attention would take one 16-wave split per head, so
-  // the outputs are the two calls' bit for bit
-  const bool fused = n <= kGmaxSelectMax && kk > 0 && k <= 512 && attn::attn_wide(BH, G, k) &&
+  // fused where gather_attention would take one split per head, so the outputs
+  // are the two calls' bit for bit
+  const bool fused = kk > 0 && kk <= kSelMaxK && k <= kAttnFusedMax &&
                      ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(Ksrc) |
                        reinterpret_cast<uintptr_t>(Vsrc)) & 7) == 0;
   if (fused) {
-    const AttnOut att{Ksrc, Vsrc, cap, scale, out};
+    const AttnArgs att{q, G, Ksrc, Vsrc, cap, scale, out};
     return plan_scan_topk_run(q, g, budget, budget_value, BH, G, D, bmax, iters, units_max, planes_sb, scales_sb, n, nsb,
                               sub, m, k, sink, local, idx, t_out, workspace, pws, &att, stream);
   }

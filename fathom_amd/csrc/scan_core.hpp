@@ -1661,6 +1661,6 @@ __device__ __forceinline__ void tile_pass(const ScanArgs &a, const Emit &em, con
 // regions; a row whose first pass holds fewer than kk candidates (a sample that
 // misled T_hi) is first rescanned with T_lo by its finalize workgroup.
 int launch_finalize_fused(const sc::ScanArgs &a, const sc::Emit &em, int64_t rows, int64_t m, int64_t k, int64_t sink,
-                          int64_t local, int64_t *idx, hipStream_t st);
+                          int64_t local, int64_t *idx, const AttnArgs *att, hipStream_t st);
 
 }  // namespace fathom

@@ -10,11 +10,14 @@ namespace fathom {
 // limit is stated in).
 size_t scan_topk_ws(int64_t rows, int64_t n, int64_t k, int64_t kk, bool whole_blocks = true);
 
-// The fused scan + top-k (stages: FATHOM_STAGE_* mask) on a caller-provided workspace.
+struct AttnArgs;  // topk_internal.hpp
+
+// The fused scan + top-k (stages: FATHOM_STAGE_* mask) on a caller-provided
+// workspace; att (null: none): the attention that its selection goes on to.
 int scan_topk_run(const float *q, int64_t BH, int64_t G, int64_t D, const int32_t *cls, const int32_t *clsn, int bmax,
                   int64_t units_max, const void *planes_sb, const void *scales_sb, int64_t n, int64_t nsb, int64_t sub, int64_t m,
                   int64_t k, int64_t sink, int64_t local, int64_t *idx, void *workspace, size_t workspace_bytes,
-                  int stages, void *stream);
+                  int stages, void *stream, const AttnArgs *att = nullptr);
 
 // make_plan on the device (budget [BH], or budget_value when budget is null).
 int make_plan_run(const float *g, const float *budget, float budget_value, int64_t BH, int64_t D, int bmax, int iters,

@@ -207,6 +207,19 @@ struct LinearBins {
   }
   __device__ __forceinline__ bool positive(uint32_t bin) const { return flo + (float)bin / scale > 0.0f; }
 };
+// Bins of keys over the finite range [lo, hi], NaN and +inf in the top one.
+struct KeyBins {
+  uint32_t lo;
+  int sft;
+  __device__ __forceinline__ KeyBins(uint32_t lo_, uint32_t hi) : lo(lo_) {
+    const uint32_t R = hi > lo_ ? hi - lo_ : 0u;
+    const int bl = R ? 32 - __clz((int)R) : 0;
+    sft = bl > 11 ? bl - 11 : 0;
+  }
+  __device__ __forceinline__ uint32_t of(uint32_t key) const {
+    return finite_key(key) ? (key - lo) >> sft : key > kKeyNegInf ? (uint32_t)(kBins - 1) : 0u;
+  }
+};
 
 // Descending ranks of the cnt valid values of E * 1024 (thread t holding slots
 // t + 1024 e; the valid ones are the slots below cnt -- LINEAR: the nonzero ones --
@@ -739,6 +752,69 @@ __global__ __launch_bounds__(kFinThreads) void finalize_kernel(int64_t m, int64_
   select_sorted(ArraySrc{gc, cnt}, cnt, kk, m, sink, local, out, cl, ss, sh, s_cnt, true);
 }
 
+// A row's output: ranked values below got are written (their tokens also to
+// `ranked`, LDS of k int32, if non-null), then the fixed positions.
+struct RowOut {
+  int64_t *p;
+  int64_t kk, m, sink, local;
+  int32_t *ranked;
+  int got;
+  __device__ __forceinline__ void put(int rank, uint64_t x) const {
+    if (rank >= got) return;
+    const uint32_t tok = 0xFFFFFFFFu - (uint32_t)x;
+    p[rank] = (int64_t)tok;
+    if (ranked) ranked[rank] = (int32_t)tok;
+  }
+  // true where the tokens are in `ranked` too
+  __device__ __forceinline__ bool finish() const {
+    write_fixed(p, got, kk, m, sink, local);
+    if (ranked) {  // the same tokens as write_fixed's
+      for (int i = got + (int)threadIdx.x; i < (int)kk; i += kFinThreads) ranked[i] = 0;
+      for (int i = threadIdx.x; i < (int)(sink + local); i += kFinThreads)
+        ranked[kk + i] = (int32_t)((i < sink) ? (int64_t)i : (m - local + (i - sink)));
+    }
+    return ranked != nullptr;
+  }
+};
+
+// The attention that follows a row's selection (k <= 512, rows in device memory):
+// the workgroup's 16 waves take the row's k positions, exactly as gather_attention's
+// attn_stream_kernel does for one split (empty waves add nothing), so out equals
+// gather_attention's output.  The ranked tokens stay in LDS, in cl's upper half, past
+// the sort's scratch and the attention's triples.
+struct RowAttn {
+  const float *q;  // [rows, D] fp32 query heads (row = bh * G + g)
+  int64_t G;
+  attn::RowSrc rs;
+  float scale;
+  float *out;      // [rows, D] fp32
+};
+__device__ __forceinline__ int32_t *ranked_lds(uint64_t *cl) {
+  static_assert(kCandLds / 2 >= 4 * kFinThreads + kBins && kCandLds / 2 >= 2 * 4 * kFinThreads &&
+                    2 * (kCandLds / 2) >= kMaxK + kFinThreads,
+                "the ranked tokens lie past the sort's scratch and hold k of them");
+  return reinterpret_cast<int32_t *>(cl + kCandLds / 2);
+}
+__device__ __forceinline__ void row_attention(const RowAttn &ra, const int64_t *ig, int64_t k, bool in_lds,
+                                              const int32_t *ranked, uint64_t *cl) {
+  constexpr int NW = kFinThreads / kWave;
+  static_assert(NW == 16, "one attention split of 16 waves");
+  static_assert(sizeof(float) * (2 * NW + NW * attn::kAttnD) <= sizeof(uint64_t) * (kCandLds / 2),
+                "the attention's LDS in cl's lower half");
+  __syncthreads();  // the row's indices are written (and cl's lower half is free)
+  const int64_t row = blockIdx.x, bh = row / ra.G;
+  float *wm = reinterpret_cast<float *>(cl), *wl = wm + NW;
+  auto wo = reinterpret_cast<float(*)[attn::kAttnD]>(wl + NW);
+  const float *qr = ra.q + row * attn::kAttnD;
+  float *orow = ra.out + row * attn::kAttnD;
+  if (in_lds)  // uniform: the tokens from LDS, else from the index list just written
+    attn::attn_stream_block<NW, false>(qr, [&](int64_t j) { return (int64_t)ranked[j]; }, k, 0, bh, ra.rs, ra.scale, wm,
+                                       wl, wo, orow, nullptr, true);
+  else
+    attn::attn_stream_block<NW, false>(qr, [&](int64_t j) { return ig[j]; }, k, 0, bh, ra.rs, ra.scale, wm, wl, wo, orow,
+                                       nullptr, true);
+}
+
 // The fallback of the fused scan + top-k, run by the finalize workgroup of a
 // row whose candidate pass found fewer than kk candidates: the row (head h of
 // bh) is rescanned with T_lo into the regions under the second count array by
@@ -766,9 +842,10 @@ __device__ __forceinline__ void rescan_row(const sc::ScanArgs &a, const sc::Emit
 // (row = bh * G + h), copied to LDS while they are counted; a row with more
 // than kCandLds candidates is selected from its regions in place.  A row with
 // fewer than kk first-pass candidates is rescanned first (rescan_row).
+template <bool ATTN>
 __global__ __launch_bounds__(kFinThreads) void finalize_fused_kernel(int64_t m, int64_t k, int64_t sink, int64_t local,
                                                                      sc::ScanArgs a, sc::Emit em,
-                                                                     int64_t *__restrict__ idx) {
+                                                                     int64_t *__restrict__ idx, RowAttn ra) {
   __shared__ uint64_t cl[kCandLds];
   __shared__ uint64_t ss[kMaxK];
   __shared__ RangeShared sh;
@@ -779,6 +856,8 @@ __global__ __launch_bounds__(kFinThreads) void finalize_fused_kernel(int64_t m, 
   const int64_t kk = k - sink - local;
   const uint64_t *gc = s.cand + row * s.cand_cap;
   int64_t *out = idx + row * k;
+  int32_t *ranked = ATTN ? ranked_lds(cl) : nullptr;
+  bool in_lds = false;
   uint32_t *pre = reinterpret_cast<uint32_t *>(ss);  // free until the survivors are collected
   RegionSrc src{s.rc1 + row * s.nreg, gc, s.nreg};
   uint32_t cnt = stage_regions(src.rc, gc, s.nreg, cl, (uint32_t)kCandLds, pre, sh);
@@ -800,16 +879,14 @@ __global__ __launch_bounds__(kFinThreads) void finalize_fused_kernel(int64_t m, 
     __syncthreads();  // cl is the ranking scratch from here
     int nlim = kWave;
     while (nlim < (int)cnt) nlim <<= 1;
-    const int got = (int64_t)cnt < kk ? (int)cnt : (int)kk;
-    bin_rank_desc<4>(v4, (int)cnt, got, cl, sh, nlim, [&](int rank, uint64_t x) {
-      if (rank < got) out[rank] = (int64_t)(0xFFFFFFFFu - (uint32_t)x);
-    });
-    write_fixed(out, got, kk, m, sink, local);
+    const RowOut ro{out, kk, m, sink, local, ranked, (int64_t)cnt < kk ? (int)cnt : (int)kk};
+    bin_rank_desc<4>(v4, (int)cnt, ro.got, cl, sh, nlim, [&](int rank, uint64_t x) { ro.put(rank, x); });
+    in_lds = ro.finish();
   } else if (cnt <= (uint32_t)kCandLds) {
     select_sorted(ArraySrc{cl, (int64_t)cnt}, cnt, kk, m, sink, local, out, cl, ss, sh, s_cnt, false);
   } else {
     select_sorted(src, cnt, kk, m, sink, local, out, cl, ss, sh, s_cnt, false);
-  }
+  }  if constexpr (ATTN) row_attention(ra, out, k, in_lds, ranked, cl);
 }
 
 // Wave-wide minimum and maximum of 32-bit values (in every lane): DPP row
@@ -1176,33 +1253,9 @@ struct QuadScores {  // quad_order(G, n) true
   }
 };
 
-// A row's output: ranked values below got are written (their tokens also to
-// `ranked`, LDS of k int32, if non-null), then the fixed positions.
-struct RowOut {
-  int64_t *p;
-  int64_t kk, m, sink, local;
-  int32_t *ranked;
-  int got;
-  __device__ __forceinline__ void put(int rank, uint64_t x) const {
-    if (rank >= got) return;
-    const uint32_t tok = 0xFFFFFFFFu - (uint32_t)x;
-    p[rank] = (int64_t)tok;
-    if (ranked) ranked[rank] = (int32_t)tok;
-  }
-  // true where the tokens are in `ranked` too
-  __device__ __forceinline__ bool finish() const {
-    write_fixed(p, got, kk, m, sink, local);
-    if (ranked) {  // the same tokens as write_fixed's
-      for (int i = got + (int)threadIdx.x; i < (int)kk; i += kFinThreads) ranked[i] = 0;
-      for (int i = threadIdx.x; i < (int)(sink + local); i += kFinThreads)
-        ranked[kk + i] = (int32_t)((i < sink) ? (int64_t)i : (m - local + (i - sink)));
-    }
-    return ranked != nullptr;
-  }
-};
-
-// Ranks the cnt <= 4096 candidates in cl (also the sort's scratch) into out.
-template <bool LINEAR>
+// Ranks the cnt <= 4096 (WIDE: 8192) candidates in cl (also the sort's scratch)
+// into out.
+template <bool LINEAR, bool WIDE>
 __device__ __forceinline__ void rank_cands(uint64_t *cl, uint32_t cnt, RowOut &out, RangeShared &sh) {
   int nlim = kWave;
   while (nlim < (int)cnt) nlim <<= 1;
@@ -1218,8 +1271,131 @@ __device__ __forceinline__ void rank_cands(uint64_t *cl, uint32_t cnt, RowOut &o
     __syncthreads();
     bin_rank_desc<E, LINEAR>(v, (int)cnt, out.got, cl, sh, nlim, [&](int rank, uint64_t x) { out.put(rank, x); });
   };
-  if (cnt <= (uint32_t)(2 * kFinThreads)) rank_all(std::integral_constant<int, 2>{});
+  if (WIDE && cnt > (uint32_t)(4 * kFinThreads)) rank_all(std::integral_constant<int, 8>{});
+  else if (!WIDE && cnt <= (uint32_t)(2 * kFinThreads)) rank_all(std::integral_constant<int, 2>{});
   else rank_all(std::integral_constant<int, 4>{});
+}
+
+// The range of the finite keys of E per thread (0: no key), and sh.hist cleared.
+template <int E>
+__device__ __forceinline__ void key_range(const uint32_t (&key)[E], uint32_t &lo, uint32_t &hi, RangeShared &sh) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = kFinThreads >> 6;
+  uint32_t mn = ~0u, mx = 0u;
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (finite_key(key[e])) {
+      mn = min(mn, key[e]);
+      mx = max(mx, key[e]);
+    }
+  wave_minmax_u32(mn, mx);
+  if (lane == 0) {
+    sh.wmin[wave] = mn;
+    sh.wmax[wave] = mx;
+  }
+  sh.hist[tid] = sh.hist[tid + kFinThreads] = 0u;
+  __syncthreads();
+  lo = ~0u;
+  hi = 0u;
+  for (int w = 0; w < nw; ++w) {
+    lo = min(lo, (uint32_t)sh.wmin[w]);
+    hi = max(hi, (uint32_t)sh.wmax[w]);
+  }
+}
+
+// The bin that holds the need-th largest of the keys (at least need of them),
+// after key_range.
+template <int E, typename Bins>
+__device__ __forceinline__ uint32_t rank_bin(const uint32_t (&key)[E], uint32_t need, const Bins &bins, RangeShared &sh) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (key[e]) atomicAdd(&sh.hist[bins.of(key[e])], 1u);
+  __syncthreads();
+  // running counts from the top bin down: thread t holds bins 2047 - 2t, 2046 - 2t
+  const uint32_t c0 = sh.hist[kBins - 1 - 2 * tid], c1 = sh.hist[kBins - 2 - 2 * tid], c = c0 + c1;
+  const uint32_t wi = wave_incl_scan_u32(c);
+  if (lane == kWave - 1) sh.wsum[wave] = wi;
+  __syncthreads();
+  uint32_t above = wi - c;
+  for (int w = 0; w < wave; ++w) above += sh.wsum[w];
+  if (above < need && above + c0 >= need) sh.hsel = (uint32_t)(kBins - 1 - 2 * tid);
+  if (above + c0 < need && above + c >= need) sh.hsel = (uint32_t)(kBins - 2 - 2 * tid);
+  __syncthreads();
+  return sh.hsel;
+}
+
+// The keys in bin b and above: their count, and the place of the thread's first.
+template <int E, typename Bins>
+__device__ __forceinline__ uint32_t place_from_bin(const uint32_t (&key)[E], uint32_t b, const Bins &bins, uint32_t &off,
+                                                   RangeShared &sh) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = kFinThreads >> 6;
+  uint32_t own = 0u, cnt = 0u;
+#pragma unroll
+  for (int e = 0; e < E; ++e) own += key[e] && bins.of(key[e]) >= b ? 1u : 0u;
+  const uint32_t wi = wave_incl_scan_u32(own);
+  if (lane == kWave - 1) sh.wsum[wave] = wi;
+  __syncthreads();
+  off = wi - own;
+  for (int w = 0; w < nw; ++w) {
+    const uint32_t s = sh.wsum[w];
+    off += w < wave ? s : 0u;
+    cnt += s;
+  }
+  return cnt;
+}
+
+// Top kk of cnt distinct values of src where more than one sort takes reach the
+// bound (ties, clustered rows).  kk up to kMaxK by select_sorted; WIDE: up to 8192,
+// from the values in cl (src is cl then) those of the bin that holds the kk-th and
+// above, else the exact kk largest by range selection, gathered in cl, then one
+// sort.  False: the tokens are not in out.ranked.
+template <bool WIDE, typename Src>
+__device__ __forceinline__ bool select_cands(const Src &src, int64_t cnt, RowOut &out, uint64_t *cl, uint64_t *ss,
+                                             RangeShared &sh, uint32_t &s_cnt, bool in_lds) {
+  if constexpr (!WIDE) {
+    select_sorted(src, cnt, out.kk, out.m, out.sink, out.local, out.p, cl, ss, sh, s_cnt, !in_lds);
+    return false;
+  } else {
+    constexpr int kHold = kCandLds / kFinThreads;
+    static_assert(kHold * kFinThreads == kCandLds && 8 * kFinThreads + kBins <= kCandLds, "cl held in registers");
+    const int lane = threadIdx.x & 63;
+    uint64_t v[kHold];
+    if (in_lds) {  // uniform
+      uint32_t key[kHold], lo, hi, off;
+#pragma unroll
+      for (int e = 0; e < kHold; ++e) {
+        const int64_t i = threadIdx.x + (int64_t)e * kFinThreads;
+        v[e] = i < cnt ? cl[i] : 0ull;
+        key[e] = (uint32_t)(v[e] >> 32);
+      }
+      key_range<kHold>(key, lo, hi, sh);
+      const KeyBins bins(lo, hi);
+      const uint32_t b = rank_bin<kHold>(key, (uint32_t)out.kk, bins, sh);
+      const uint32_t kept = place_from_bin<kHold>(key, b, bins, off, sh);
+      if (kept <= 8u * kFinThreads) {  // uniform; every thread has read cl
+#pragma unroll
+        for (int e = 0; e < kHold; ++e)
+          if (key[e] && bins.of(key[e]) >= b) cl[off++] = v[e];
+        __syncthreads();
+        rank_cands<false, true>(cl, kept, out, sh);
+        return out.finish();
+      }
+      __syncthreads();
+    }
+    const uint64_t thr = range_select(src, cnt, (uint32_t)out.kk, sh);
+    __syncthreads();
+    if (threadIdx.x == 0) s_cnt = 0u;
+    __syncthreads();
+    if (in_lds) {  // the survivors take the candidates' place
+#pragma unroll
+      for (int e = 0; e < kHold; ++e) lds_append(v[e] >= thr && v[e] != 0ull, v[e], &s_cnt, cl, 8u * kFinThreads, lane);
+    } else {
+      src.for_each([&](bool ok, uint64_t v) { lds_append(ok && v >= thr, v, &s_cnt, cl, 8u * kFinThreads, lane); });
+    }
+    __syncthreads();
+    rank_cands<false, true>(cl, min(s_cnt, 8u * kFinThreads), out, sh);
+    return out.finish();
+  }
 }
 
 // Exact top kk of a short row, read whole: up to 4096 tokens are ranked at once
@@ -1227,10 +1403,10 @@ __device__ __forceinline__ void rank_cands(uint64_t *cl, uint32_t cnt, RowOut &o
 // holds the kk-th largest and above, 2048 linear bins over the finite scores'
 // range (kk and a few of them for spread scores; rows whose kept scores
 // outgrow the sort are selected by range).
-template <int E, typename Scores>
+template <int E, bool WIDE, typename Scores>
 __device__ __forceinline__ bool rowrank_row(const Scores &rs, int64_t n, RowOut &out, uint64_t *cl, uint64_t *ss,
                                             RangeShared &sh, uint32_t &s_cnt) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = kFinThreads >> 6;
+  const int tid = threadIdx.x;
   const int64_t kk = out.kk, sink = out.sink;
   const int64_t lstart = (out.m - out.local) > 0 ? (out.m - out.local) : 0;
   uint32_t key[E];  // 0: no candidate (below every score's key)
@@ -1250,66 +1426,23 @@ __device__ __forceinline__ bool rowrank_row(const Scores &rs, int64_t n, RowOut 
     bin_rank_desc<E, true>(v, (int)n, out.got, cl, sh, nlim, [&](int rank, uint64_t x) { out.put(rank, x); });
     return out.finish();
   }
-  uint32_t mn = ~0u, mx = 0u;
-#pragma unroll
-  for (int e = 0; e < E; ++e)
-    if (finite_key(key[e])) {
-      mn = min(mn, key[e]);
-      mx = max(mx, key[e]);
-    }
-  wave_minmax_u32(mn, mx);
-  if (lane == 0) {
-    sh.wmin[wave] = mn;
-    sh.wmax[wave] = mx;
-  }
-  sh.hist[tid] = sh.hist[tid + kFinThreads] = 0u;
-  __syncthreads();
-  uint32_t lo = ~0u, hi = 0u;
-  for (int w = 0; w < nw; ++w) {
-    lo = min(lo, (uint32_t)sh.wmin[w]);
-    hi = max(hi, (uint32_t)sh.wmax[w]);
-  }
+  uint32_t lo, hi;
+  key_range<E>(key, lo, hi, sh);
   const LinearBins bins(lo, hi);
-#pragma unroll
-  for (int e = 0; e < E; ++e)
-    if (key[e]) atomicAdd(&sh.hist[bins.of(key[e])], 1u);
-  __syncthreads();
-  // running counts from the top bin down: thread t holds bins 2047 - 2t, 2046 - 2t
-  const uint32_t c0 = sh.hist[kBins - 1 - 2 * tid], c1 = sh.hist[kBins - 2 - 2 * tid], c = c0 + c1;
-  const uint32_t wi = wave_incl_scan_u32(c);
-  if (lane == kWave - 1) sh.wsum[wave] = wi;
-  __syncthreads();
-  uint32_t above = wi - c;
-  for (int w = 0; w < wave; ++w) above += sh.wsum[w];
-  const uint32_t need = (uint32_t)kk;
-  if (above < need && above + c0 >= need) sh.hsel = (uint32_t)(kBins - 1 - 2 * tid);
-  if (above + c0 < need && above + c >= need) sh.hsel = (uint32_t)(kBins - 2 - 2 * tid);
-  __syncthreads();
-  const uint32_t b = sh.hsel;  // set: n >= kk scores are counted
-  uint32_t own = 0u;
-#pragma unroll
-  for (int e = 0; e < E; ++e) own += key[e] && bins.of(key[e]) >= b ? 1u : 0u;
-  const uint32_t oi = wave_incl_scan_u32(own);
-  if (lane == kWave - 1) sh.wsum[wave] = oi;
-  __syncthreads();
-  uint32_t off = oi - own, cnt = 0u;
-  for (int w = 0; w < nw; ++w) {
-    const uint32_t s = sh.wsum[w];
-    off += w < wave ? s : 0u;
-    cnt += s;
-  }
-  if (cnt > (uint32_t)(4 * kFinThreads)) {  // uniform: ties, or a range that outliers stretch
+  const uint32_t b = rank_bin<E>(key, (uint32_t)kk, bins, sh);  // n >= kk keys are counted
+  uint32_t off;
+  const uint32_t cnt = place_from_bin<E>(key, b, bins, off, sh);
+  if (cnt > (uint32_t)((WIDE ? 8 : 4) * kFinThreads)) {  // uniform: ties, or a range that outliers stretch
     const auto src = index_src([&](int64_t i) { return k64_of(masked_key(rs, i, sink, lstart), i); }, n);
-    select_sorted(src, n, kk, out.m, sink, out.local, out.p, cl, ss, sh, s_cnt, true);
-    return false;
+    return select_cands<WIDE>(src, n, out, cl, ss, sh, s_cnt, false);
   }
 #pragma unroll
   for (int e = 0; e < E; ++e)
     if (key[e] && bins.of(key[e]) >= b) cl[off++] = k64(e);
   __syncthreads();
   // scores of both signs: linear bins again; a tail of positive ones: the keys'
-  if (bins.positive(b)) rank_cands<false>(cl, cnt, out, sh);
-  else rank_cands<true>(cl, cnt, out, sh);
+  if (bins.positive(b)) rank_cands<false, WIDE>(cl, cnt, out, sh);
+  else rank_cands<true, WIDE>(cl, cnt, out, sh);
   return out.finish();
 }
 // The rows that rowrank_row takes: short ones, and those with few groups per
@@ -1336,15 +1469,15 @@ static_assert(kGmaxSelectMax / kGroupTok <= 65536, "group numbers fit 16 bits");
 // ranked (LDS of k int32, past the sort's scratch in cl; null: none): rows of
 // at most 2048 candidates also leave their k output tokens there, and the
 // call returns true.
-template <int kPer, typename Scores>
+template <int kPer, bool WIDE, typename Scores>
 __device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint32_t *__restrict__ gmax, int64_t n,
                                                    RowOut &out, uint64_t *cl, uint64_t *ss, RangeShared &sh,
                                                    uint32_t &s_cnt) {
   uint16_t *glist = reinterpret_cast<uint16_t *>(ss);  // ss holds the survivors only after the groups are read
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = kFinThreads >> 6;
   const int64_t row = blockIdx.x;
-  const int64_t kk = out.kk, m = out.m, sink = out.sink, local = out.local;
-  const int64_t lstart = (m - local) > 0 ? (m - local) : 0;
+  const int64_t kk = out.kk, sink = out.sink;
+  const int64_t lstart = (out.m - out.local) > 0 ? (out.m - out.local) : 0;
   const int ngrp = (int)cdiv(n, kGroupTok);
   uint32_t gm[kPer];
 #pragma unroll
@@ -1380,23 +1513,30 @@ __device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint3
   }
   if (ngr > (uint32_t)kGroupList) {  // uniform: ties around T
     const auto src = index_src([&](int64_t i) { return k64_of(masked_key(rs, i, sink, lstart), i); }, n);
-    select_sorted(src, n, kk, m, sink, local, out.p, cl, ss, sh, s_cnt, true);
-    return false;
+    return select_cands<WIDE>(src, n, out, cl, ss, sh, s_cnt, false);
   }
-  // their keys >= T, one group per thread, placed by a workgroup prefix sum
+  // their keys >= T, kU groups per thread and round, placed by a workgroup prefix sum
+  constexpr int kU = WIDE ? 2 : 1;
   uint32_t cnt = 0u;
-  for (uint32_t e0 = 0; e0 < ngr; e0 += kFinThreads) {  // uniform
-    const uint32_t e = e0 + tid;
-    const int64_t t0 = e < ngr ? (int64_t)glist[e] * kGroupTok : n;
-    float v[kGroupTok] = {};
-    rs.group(t0, v);
-    uint32_t key[kGroupTok], c = 0u;
+  for (uint32_t e0 = 0; e0 < ngr; e0 += kU * kFinThreads) {  // uniform
+    int64_t t0[kU];
+    float v[kU][kGroupTok] = {};
 #pragma unroll
-    for (int r = 0; r < kGroupTok; ++r) {
-      const int64_t i = t0 + r;
-      key[r] = (i < sink || i >= lstart) ? kKeyNegInf : score_key(v[r]);
-      c += (i < n && key[r] >= T) ? 1u : 0u;
+    for (int u = 0; u < kU; ++u) {
+      const uint32_t e = e0 + u * kFinThreads + tid;
+      t0[u] = e < ngr ? (int64_t)glist[e] * kGroupTok : n;
     }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) rs.group(t0[u], v[u]);
+    uint32_t key[kU][kGroupTok], c = 0u;
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int r = 0; r < kGroupTok; ++r) {
+        const int64_t i = t0[u] + r;
+        key[u][r] = (i < sink || i >= lstart) ? kKeyNegInf : score_key(v[u][r]);
+        c += (i < n && key[u][r] >= T) ? 1u : 0u;
+      }
     const uint32_t wi = wave_incl_scan_u32(c);
     if (lane == kWave - 1) sh.wsum[wave] = wi;
     __syncthreads();
@@ -1407,25 +1547,24 @@ __device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint3
       cnt += ws;
     }
 #pragma unroll
-    for (int r = 0; r < kGroupTok; ++r) {
-      const int64_t i = t0 + r;
-      if (i < n && key[r] >= T) {
-        if (off < (uint32_t)kCandLds) cl[off] = k64_of(key[r], i);
-        ++off;
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int r = 0; r < kGroupTok; ++r) {
+        const int64_t i = t0[u] + r;
+        if (i < n && key[u][r] >= T) {
+          if (off < (uint32_t)kCandLds) cl[off] = k64_of(key[u][r], i);
+          ++off;
+        }
       }
-    }
     __syncthreads();  // sh.wsum is rewritten by the next step
   }
   if (cnt > (uint32_t)kCandLds) {  // uniform: ties around T
     const auto src = index_src([&](int64_t i) { return k64_of(masked_key(rs, i, sink, lstart), i); }, n);
-    select_sorted(src, n, kk, m, sink, local, out.p, cl, ss, sh, s_cnt, true);
-    return false;
+    return select_cands<WIDE>(src, n, out, cl, ss, sh, s_cnt, false);
   }
-  if (cnt > (uint32_t)(4 * kFinThreads)) {
-    select_sorted(ArraySrc{cl, (int64_t)cnt}, cnt, kk, m, sink, local, out.p, cl, ss, sh, s_cnt, false);
-    return false;
-  }
-  rank_cands<false>(cl, cnt, out, sh);  // at most 4096 candidates: one sort ranks them
+  if (cnt > (uint32_t)((WIDE ? 8 : 4) * kFinThreads))
+    return select_cands<WIDE>(ArraySrc{cl, (int64_t)cnt}, cnt, out, cl, ss, sh, s_cnt, true);
+  rank_cands<false, WIDE>(cl, cnt, out, sh);  // one sort ranks them
   return out.finish();
 }
 
@@ -1435,14 +1574,7 @@ __device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint3
 // workgroup then runs the attention of its query head over the k indices it
 // wrote, exactly as gather_attention's attn_stream_kernel does for one split
 // (16 waves of 32 positions), so out equals gather_attention's output.
-struct RowAttn {
-  const float *q;  // [rows, D] fp32 query heads (row = bh * G + g)
-  int64_t G;
-  attn::RowSrc rs;
-  float scale;
-  float *out;      // [rows, D] fp32
-};
-template <typename Scores, bool ATTN, int kPer, int E>
+template <typename Scores, bool ATTN, bool WIDE, int kPer, int E>
 __global__ __launch_bounds__(kFinThreads) void rowselect_kernel(const float *__restrict__ scores, int64_t G,
                                                                 const uint32_t *__restrict__ gmax, int64_t n, int64_t m,
                                                                 int64_t k, int64_t sink, int64_t local,
@@ -1451,36 +1583,14 @@ __global__ __launch_bounds__(kFinThreads) void rowselect_kernel(const float *__r
   __shared__ uint64_t ss[kMaxK];
   __shared__ RangeShared sh;
   __shared__ uint32_t s_cnt;
-  // ATTN: the ranked tokens also in LDS, in cl's upper half (past the sort's
-  // scratch and the attention's triples)
-  int32_t *ranked = ATTN ? reinterpret_cast<int32_t *>(cl + kCandLds / 2) : nullptr;
-  static_assert(kCandLds / 2 >= 4 * kFinThreads + kBins && kCandLds / 2 >= 2 * 4 * kFinThreads &&
-                    2 * (kCandLds / 2) >= kMaxK + kFinThreads,
-                "the ranked tokens lie past the sort's scratch and hold k of them");
+  static_assert(!ATTN || !WIDE, "the attention's tokens lie past a sort of 4096");
+  int32_t *ranked = ATTN ? ranked_lds(cl) : nullptr;
   RowOut ro{idx + blockIdx.x * k, k - sink - local, m, sink, local, ranked, 0};
   const Scores rs(scores, n, G);
   bool in_lds;
-  if constexpr (E > 0) in_lds = rowrank_row<E>(rs, n, ro, cl, ss, sh, s_cnt);
-  else in_lds = rowselect_gmax_row<kPer>(rs, gmax, n, ro, cl, ss, sh, s_cnt);
-  if constexpr (ATTN) {
-    constexpr int NW = kFinThreads / kWave;
-    static_assert(NW == 16, "one attention split of 16 waves");
-    static_assert(sizeof(float) * (2 * NW + NW * attn::kAttnD) <= sizeof(uint64_t) * (kCandLds / 2),
-                  "the attention's LDS in cl's lower half");
-    __syncthreads();  // the row's indices are written (and cl's lower half is free)
-    const int64_t row = blockIdx.x, bh = row / ra.G;
-    const int64_t *ig = idx + row * k;
-    float *wm = reinterpret_cast<float *>(cl), *wl = wm + NW;
-    auto wo = reinterpret_cast<float(*)[attn::kAttnD]>(wl + NW);
-    const float *qr = ra.q + row * attn::kAttnD;
-    float *orow = ra.out + row * attn::kAttnD;
-    if (in_lds)  // uniform: the tokens from LDS, else from the index list just written
-      attn::attn_stream_block<NW, false>(qr, [&](int64_t j) { return (int64_t)ranked[j]; }, k, 0, bh, ra.rs, ra.scale,
-                                         wm, wl, wo, orow, nullptr, true);
-    else
-      attn::attn_stream_block<NW, false>(qr, [&](int64_t j) { return ig[j]; }, k, 0, bh, ra.rs, ra.scale, wm, wl, wo,
-                                         orow, nullptr, true);
-  }
+  if constexpr (E > 0) in_lds = rowrank_row<E, WIDE>(rs, n, ro, cl, ss, sh, s_cnt);
+  else in_lds = rowselect_gmax_row<kPer, WIDE>(rs, gmax, n, ro, cl, ss, sh, s_cnt);
+  if constexpr (ATTN) row_attention(ra, idx + blockIdx.x * k, k, in_lds, ranked, cl);
 }
 
 // The wide selection's kk <= 8192 values of a row (sel [rows, P], all
@@ -1614,6 +1724,13 @@ int launch_filter_scores(const float *scores, int64_t rows, int64_t n, int64_t s
   return launch_status("filter_scores_kernel");
 }
 
+namespace {
+RowAttn row_attn(const AttnArgs &t, int64_t n) {
+  return RowAttn{t.q, t.G, attn::RowSrc{(const char *)t.K, (const char *)t.V, nullptr, nullptr, t.cap, 0, n, 2 * attn::kAttnD},
+                 t.scale, t.out};
+}
+}  // namespace
+
 int launch_finalize(int64_t rows, int64_t m, int64_t k, int64_t sink, int64_t local, TopkSel s, int64_t *idx,
                     hipStream_t st) {
   finalize_kernel<<<(unsigned)rows, kFinThreads, 0, st>>>(m, k, sink, local, s, idx);
@@ -1621,8 +1738,11 @@ int launch_finalize(int64_t rows, int64_t m, int64_t k, int64_t sink, int64_t lo
 }
 
 int launch_finalize_fused(const sc::ScanArgs &a, const sc::Emit &em, int64_t rows, int64_t m, int64_t k, int64_t sink,
-                          int64_t local, int64_t *idx, hipStream_t st) {
-  finalize_fused_kernel<<<(unsigned)rows, kFinThreads, 0, st>>>(m, k, sink, local, a, em, idx);
+                          int64_t local, int64_t *idx, const AttnArgs *att, hipStream_t st) {
+  if (att)
+    finalize_fused_kernel<true><<<(unsigned)rows, kFinThreads, 0, st>>>(m, k, sink, local, a, em, idx, row_attn(*att, a.n));
+  else
+    finalize_fused_kernel<false><<<(unsigned)rows, kFinThreads, 0, st>>>(m, k, sink, local, a, em, idx, RowAttn{});
   return launch_status("finalize_fused_kernel");
 }
 
@@ -1630,39 +1750,46 @@ namespace {
 template <typename Scores, bool ATTN>
 int launch_row_select(const float *scores, int64_t G, const uint32_t *gmax, int64_t rows, int64_t n, int64_t m, int64_t k,
                       int64_t sink, int64_t local, int64_t *idx, const RowAttn &ra, hipStream_t st) {
-  static_assert(kRowSelectMax == 2 * kFinThreads * kGroupTok && kGmaxSelectMax == 8 * kFinThreads * kGroupTok, "groups");
-  if (n > kGmaxSelectMax)
-    return fail(FATHOM_ERR_INVALID, "row selection: n=%lld exceeds %lld", (long long)n, (long long)kGmaxSelectMax);
+  static_assert(kRowSelectMax == 2 * kFinThreads * kGroupTok && kGmaxSelectMax == 8 * kFinThreads * kGroupTok &&
+                    kGmaxWideMax == 32 * kFinThreads * kGroupTok,
+                "groups per thread");
+  const int64_t kk = k - sink - local;
+  if (!group_select_takes(n, kk))
+    return fail(FATHOM_ERR_INVALID, "row selection: n=%lld kk=%lld not taken", (long long)n, (long long)kk);
   const unsigned g = (unsigned)rows;
   const auto run = [&](auto kernel) { kernel<<<g, kFinThreads, 0, st>>>(scores, G, gmax, n, m, k, sink, local, idx, ra); };
-  if (rowrank_takes(n, k - sink - local)) {
-    if (n <= kFinThreads) run(rowselect_kernel<Scores, ATTN, 0, 1>);
-    else if (n <= 4 * kFinThreads) run(rowselect_kernel<Scores, ATTN, 0, 4>);
-    else if (n <= 8 * kFinThreads) run(rowselect_kernel<Scores, ATTN, 0, 8>);
-    else run(rowselect_kernel<Scores, ATTN, 0, 32>);
+  const bool whole = rowrank_takes(n, kk);
+  if constexpr (!ATTN) {
+    if (kk > kSelMaxK && n > 4 * kFinThreads) {
+      if (whole && n <= 8 * kFinThreads) run(rowselect_kernel<Scores, false, true, 0, 8>);
+      else if (whole) run(rowselect_kernel<Scores, false, true, 0, 32>);
+      else if (n <= kGmaxSelectMax) run(rowselect_kernel<Scores, false, true, 8, 0>);
+      else run(rowselect_kernel<Scores, false, true, 32, 0>);
+      return launch_status("rowselect_kernel");
+    }
+  }
+  if (whole) {
+    if (n <= kFinThreads) run(rowselect_kernel<Scores, ATTN, false, 0, 1>);
+    else if (n <= 4 * kFinThreads) run(rowselect_kernel<Scores, ATTN, false, 0, 4>);
+    else if (n <= 8 * kFinThreads) run(rowselect_kernel<Scores, ATTN, false, 0, 8>);
+    else run(rowselect_kernel<Scores, ATTN, false, 0, 32>);
   } else if (n <= kRowSelectMax) {
-    run(rowselect_kernel<Scores, ATTN, 2, 0>);
+    run(rowselect_kernel<Scores, ATTN, false, 2, 0>);
   } else {
-    run(rowselect_kernel<Scores, ATTN, 8, 0>);
+    run(rowselect_kernel<Scores, ATTN, false, 8, 0>);
   }
   return launch_status("rowselect_kernel");
 }
 }  // namespace
 
 int launch_rowselect_gmax(const float *scores, const uint32_t *gmax, int64_t rows, int64_t G, int64_t n, int64_t m,
-                          int64_t k, int64_t sink, int64_t local, int64_t *idx, hipStream_t st) {
-  if (!quad_order(G, n)) return launch_row_select<TileScores, false>(scores, G, gmax, rows, n, m, k, sink, local, idx, RowAttn{}, st);
-  return launch_row_select<QuadScores, false>(scores, G, gmax, rows, n, m, k, sink, local, idx, RowAttn{}, st);
-}
-
-int launch_rowselect_gmax_attn(const float *scores, const uint32_t *gmax, int64_t rows, int64_t n, int64_t m, int64_t k,
-                               int64_t sink, int64_t local, int64_t *idx, const float *q, int64_t G, const void *K,
-                               const void *V, int64_t cap, float scale, float *out, hipStream_t st) {
-  if (k > kFinThreads / 2) return fail(FATHOM_ERR_INVALID, "rowselect_gmax_attn: k=%lld exceeds 512", (long long)k);
-  RowAttn ra{q, G, attn::RowSrc{(const char *)K, (const char *)V, nullptr, nullptr, cap, 0, n, 2 * attn::kAttnD}, scale,
-             out};
-  if (!quad_order(G, n)) return launch_row_select<TileScores, true>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st);
-  return launch_row_select<QuadScores, true>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st);
+                          int64_t k, int64_t sink, int64_t local, int64_t *idx, const AttnArgs *att, hipStream_t st) {
+  const RowAttn ra = att ? row_attn(*att, n) : RowAttn{};
+  if (att)
+    return quad_order(G, n) ? launch_row_select<QuadScores, true>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st)
+                            : launch_row_select<TileScores, true>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st);
+  return quad_order(G, n) ? launch_row_select<QuadScores, false>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st)
+                          : launch_row_select<TileScores, false>(scores, G, gmax, rows, n, m, k, sink, local, idx, ra, st);
 }
 
 int launch_rank_list(const uint64_t *sel, int64_t P, int64_t rows, int64_t kk, int64_t m, int64_t k, int64_t sink,
@@ -1757,17 +1884,12 @@ extern "C" int fathom_sink_local_topk(const float *scores, int64_t rows, int64_t
   hipStream_t st = (hipStream_t)stream;
   const int64_t kk = k - sink - local;
   if (kk == 0) return launch_fixed_only(rows, m, k, sink, local, idx, st);
-  if (kk > kSelMaxK) return wide_topk_run(scores, rows, n, m, k, sink, local, idx, workspace, workspace_bytes, st);
-  const size_t need = topk_layout(rows, n, k, false, nullptr, nullptr, nullptr, nullptr, nullptr);
+  const size_t need = kk > kSelMaxK ? wide_topk_bytes(rows, n, k)
+                                    : topk_layout(rows, n, k, false, nullptr, nullptr, nullptr, nullptr, nullptr);
   if (!workspace || workspace_bytes < need)
     return fail(FATHOM_ERR_WORKSPACE, "sink_local_topk: workspace %zu bytes, need %zu", workspace_bytes, need);
-  TopkSel s;
-  uint32_t *samp = nullptr;
-  int64_t samp_cap = 0, S = 1;
-  topk_layout(rows, n, k, false, static_cast<char *>(workspace), &samp, &samp_cap, &s, &S);
-  s.kk = (uint32_t)kk;
   const int64_t lstart = (m - local) > 0 ? (m - local) : 0;
-  if (n <= kGmaxSelectMax) {
+  if (group_select_takes(n, kk)) {
     uint32_t *gmax = static_cast<uint32_t *>(workspace);  // 4 bytes per 16 scores, the layout has 8 per score
     if (!rowrank_takes(n, kk)) {
       group_max_kernel<<<dim3((unsigned)cdiv(n, 256 * kGmaxPer), (unsigned)rows), 256, 0, st>>>(scores, n, sink, lstart, gmax);
@@ -1776,6 +1898,12 @@ extern "C" int fathom_sink_local_topk(const float *scores, int64_t rows, int64_t
     return rc ? rc
               : launch_row_select<RowScores, false>(scores, 1, gmax, rows, n, m, k, sink, local, idx, RowAttn{}, st);
   }
+  if (kk > kSelMaxK) return wide_topk_run(scores, rows, n, m, k, sink, local, idx, workspace, workspace_bytes, st);
+  TopkSel s;
+  uint32_t *samp = nullptr;
+  int64_t samp_cap = 0, S = 1;
+  topk_layout(rows, n, k, false, static_cast<char *>(workspace), &samp, &samp_cap, &s, &S);
+  s.kk = (uint32_t)kk;
   const int64_t r_hi = topk_hi_rank(n, S, kk, kTileTok);
   rc = launch_sample_scores(scores, rows, n, S, sink, lstart, samp, samp_cap, st);
   if (rc) return rc;

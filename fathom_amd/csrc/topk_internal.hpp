@@ -35,6 +35,11 @@ constexpr int64_t kTileTok = 2048;  // tokens per sample tile of the score-row t
 constexpr int64_t kRegTok = 1024;   // tokens per candidate region and sample tile of the fused scan (one wave-tile)
 constexpr int64_t kMaxSample = 65536; // sampled keys per row (held in registers by select)
 
+// Largest kk of the sampled chains (sample -> select -> filter -> finalize, the
+// fused scan's), and of the selections that sort once.
+constexpr int64_t kSelMaxK = 2048;
+constexpr int64_t kRankListMax = 8192;
+
 // expected first-pass candidates per row, in units of kk: kAlphaX2 / 2
 constexpr int64_t kAlphaX2 = 5;
 
@@ -50,10 +55,25 @@ constexpr int64_t kRowSelectMax = 32768;
 // 262144 36.3; 43.1; 32 x 4 heads of 65536 57.5; 43.1; 8 x 7 heads of 131072 63; 51;
 // 16 x 8 heads of 131072 65; 52; 2 x 4 heads of 262144 31.6; 30.4.
 constexpr int64_t kGmaxSelectMax = 131072;
+constexpr int64_t kGmaxWideMax = 524288;  // and of the wide selection (kk above kSelMaxK)
 
 // Tokens per group of the group maxima that the fused scan's short-row pass
 // writes beside its scores (one lane's 16 tokens of a block).
 constexpr int64_t kGroupTok = 16;
+
+// The rows selected by one workgroup each: from the group maxima, or (up to
+// kRowSelectMax tokens, few groups per selected key) read whole.  Above kSelMaxK
+// the groups must number at least 5/4 kk and their list must fit; the others take
+// the chain and the wide selection.  sink_local_topk of 32 rows, us, chain and wide
+// selection against this one: n = 8192, k = 4096 107; 17.5, 30000, 4096 104; 29, 32768,
+// 8000 136; 37, 100000, 4096 82; 47, 300007, 4096 104; 71, 524288, 4096 91; 72; beyond
+// the limits 1048576, 4096 98; 97 and 300007, 8192 121; 116 (198 on rows whose list
+// does not fit).
+inline bool group_select_takes(int64_t n, int64_t kk) {
+  if (kk <= kSelMaxK) return n <= kGmaxSelectMax;
+  if (n <= kRowSelectMax) return kk <= kRankListMax;
+  return n <= kGmaxWideMax && kk <= 6144 && 4 * cdiv(n, kGroupTok) >= 5 * kk;
+}
 
 // The fused scan's own score order, rows held in whole blocks (so no store is
 // split or unaligned, whatever n is): [bh][head][token], the drop-in order
@@ -150,6 +170,20 @@ size_t topk_sel_layout(int64_t rows, int64_t cand_cap, int64_t nreg, char *base,
 size_t topk_layout(int64_t rows, int64_t n, int64_t k, bool regions, char *base, uint32_t **samp, int64_t *samp_cap,
                    TopkSel *sel, int64_t *S_out);
 
+// The attention over each row's k <= 512 selected positions that a selection goes on
+// to: q [rows, D] query heads (row = bh * G + g), K, V bf16 rows [BH, cap, D = 128] in
+// device memory, out [rows, D] fp32, equal to gather_attention's output for the
+// selected indices.
+struct AttnArgs {
+  const float *q;
+  int64_t G;
+  const void *K, *V;
+  int64_t cap;
+  float scale;
+  float *out;
+};
+constexpr int64_t kAttnFusedMax = 512;
+
 // T_lo (rank kk) and T_hi (rank r_hi <= kk) of every row's sample; clears the counters.
 int launch_select_keys(const uint32_t *samp, int64_t rows, int64_t samp_cap, int64_t kk, int64_t r_hi, TopkSel s,
                        hipStream_t st);
@@ -168,27 +202,17 @@ int launch_finalize(int64_t rows, int64_t m, int64_t k, int64_t sink, int64_t lo
 // Exact top kk of score rows from their 16-token group maxima (gmax [rows, ceil(n / 16)]
 // largest masked keys; scores in the fused scan's order): only the groups that
 // can hold a top-kk key are read.
+// att (k <= 512): the same workgroups go on to their query heads' attention.
 int launch_rowselect_gmax(const float *scores, const uint32_t *gmax, int64_t rows, int64_t G, int64_t n, int64_t m,
-                          int64_t k, int64_t sink, int64_t local, int64_t *idx, hipStream_t st);
-// launch_rowselect_gmax, then in the same workgroup the attention of each row's
-// query head (row = bh * G + g) over its k <= 512 selected positions: K, V
-// bf16 rows [BH, cap, D = 128] in device memory, out [rows, D] fp32, equal to
-// gather_attention's output for those indices.
-int launch_rowselect_gmax_attn(const float *scores, const uint32_t *gmax, int64_t rows, int64_t n, int64_t m, int64_t k,
-                               int64_t sink, int64_t local, int64_t *idx, const float *q, int64_t G, const void *K,
-                               const void *V, int64_t cap, float scale, float *out, hipStream_t st);
+                          int64_t k, int64_t sink, int64_t local, int64_t *idx, const AttnArgs *att, hipStream_t st);
 // kk == 0: only the sink and local positions are written.
 int launch_fixed_only(int64_t rows, int64_t m, int64_t k, int64_t sink, int64_t local, int64_t *idx, hipStream_t st);
-// Largest kk of the LDS-resident selections (sample -> select -> filter ->
-// finalize, row-select, the fused scan's chains); larger kk take the wide path.
-constexpr int64_t kSelMaxK = 2048;
 // State of the wide selection (exact top kk of candidate lists for any kk by a
 // 64-bit radix select, then a counting or bitonic sort; launches of
 // data-independent shape).
 size_t wide_select_bytes(int64_t rows, int64_t kk);
 // Ranks of the kk <= kRankListMax distinct values of each row of sel [rows, P]
 // by one counting sort, written as idx [rows, k] (then the fixed positions).
-constexpr int64_t kRankListMax = 8192;
 int launch_rank_list(const uint64_t *sel, int64_t P, int64_t rows, int64_t kk, int64_t m, int64_t k, int64_t sink,
                      int64_t local, int64_t *idx, hipStream_t st);
 // The wide selection over the candidate lists (list layout) of the chain's filter passes.

@@ -135,3 +135,49 @@ def test_fused_selection_of_short_rows(n, k):
         idx, out = st.plan_scan_topk_attention(x["q"], g, 48.0, k, x["K"], x["K"], 4, 32)
         ref, _ = off.gather_attention(x["q"], idx, n, x["K"], x["K"], n)
         assert torch.equal(idx.cpu(), want) and torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("n,k,extra", [(2100, 2085, 0), (4097, 4097, 0), (8192, 4096, 0), (8193, 8228, 40), (30000, 4096, 0),
+                                       (32768, 8000, 0), (32769, 8228, 0), (131072, 4000, 0), (131073, 2085, 0),
+                                       (200001, 8228, 7), (524289, 3000, 0), (1048576, 2100, 0), (1048577, 2100, 0)])
+def test_wide_selection_at_every_route(n, k, extra):
+    print(f"[wide-select] n={n} k={k}", flush=True)
+    rows = 2 if n < 300000 else 1
+    for i, kind in enumerate(("normal", "equal", "specials", "outliers", "lowest", "steps")):
+        s = _score_rows(kind, rows, n, n + i)
+        got = bp.sink_local_topk(torch.from_numpy(s).to(DEV), k, 4, 32, m=n + extra).cpu().numpy()
+        np.testing.assert_array_equal(got, O.sink_local_topk(s, k, 4, 32, m=n + extra), err_msg=kind)
+
+
+@pytest.mark.parametrize("BH,G,n,k", [(2, 5, 200001, 4096), (1, 4, 40000, 3000), (1, 8, 9000, 8228), (1, 4, 600000, 5000)])
+def test_wide_fused_selection(BH, G, n, k):
+    print(f"[wide-select fused] {BH}x{G} n={n} k={k}", flush=True)
+    x = W.synth_layer(BH, n, G, seed=n % 31, device=DEV, kdtype=torch.bfloat16)
+    g = ((x["q"] ** 2) * x["var"][:, None, :]).sum(1)
+    st = bp.PlaneStore(x["K"], keep_code=False)
+    plan = bp.make_plan(g, 56.0)
+    want = _oracle_topk(st.scan(x["q"], plan), k, 4, 32, n)
+    assert torch.equal(st.scan_topk(x["q"], plan, k, 4, 32).cpu(), want)
+    assert torch.equal(st.plan_scan_topk(x["q"], g, 56.0, k, 4, 32).cpu(), want)
+
+
+@pytest.mark.parametrize("BH,G,k", [(1, 1, 1), (1, 3, 33), (2, 4, 128), (2, 4, 129), (1, 5, 500), (8, 4, 512), (3, 2, 513),
+                                    (1, 7, 1024), (2, 4, 1030), (14, 7, 2048), (1, 2, 4200), (40, 3, 1500)])
+def test_attention_splits(BH, G, k):
+    """Splits of 128 and 512 positions, merged over up to 4, 8 and more of them, against softmax attention in float64 on
+    the CPU: float32 products and sums over k terms stay within 1e-5 of the largest value."""
+    print(f"[attention] {BH}x{G} k={k}", flush=True)
+    n = 5000
+    gen = torch.Generator().manual_seed(k)
+    K, V = (torch.randn(BH, n, 128, generator=gen).bfloat16() for _ in range(2))
+    q = torch.randn(BH, G, 128, generator=gen)
+    idx = torch.randint(0, n, (BH, G, k), generator=gen)
+    idx[0, 0, :1] = -1                           # a zero row
+    out, _ = off.gather_attention(q.to(DEV), idx.to(DEV), n, K.to(DEV), V.to(DEV), n)
+    for b in range(BH):
+        for h in range(G):
+            rows = idx[b, h]
+            Ks, Vs = K[b, rows.clamp_min(0)].double(), V[b, rows.clamp_min(0)].double()
+            Ks[rows < 0], Vs[rows < 0] = 0.0, 0.0
+            ref = torch.softmax(Ks @ q[b, h].double() * 128 ** -0.5, 0) @ Vs
+            assert (out[b, h].cpu().double() - ref).abs().max() <= 1e-5 * ref.abs().max().clamp_min(1.0)
