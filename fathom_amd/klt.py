@@ -25,7 +25,7 @@ once per layer) runs in float64 on the CPU.
 import torch
 
 from . import _lib
-from .bitplane import D, PlaneStore, make_plan, _need_gpu, _ptr, _stream
+from .bitplane import D, PlaneStore, make_plan, _KDT, _need_gpu, _ptr, _stream
 
 SINK = 4  # scripts/sketch.py: calibration statistics skip the first SINK * 4 tokens
 
@@ -68,6 +68,17 @@ def klt_query(q, Vt, lam):
     return qr, gain
 
 
+def _centered(K, mu):
+    """float(K) - mu [BH, n, D] float32 in one kernel; other key dtypes and layouts,
+    and shapes that torch broadcasts, through torch."""
+    if K.dim() != 3 or K.numel() == 0 or K.shape[0] > 65535 or K.dtype not in _KDT or not K.is_contiguous() or \
+            tuple(mu.shape) != (K.shape[0], K.shape[2]):
+        return K.float() - mu[:, None, :]
+    out = torch.empty(K.shape, dtype=torch.float32, device=K.device)
+    _lib.call("fathom_klt_center", _ptr(K), _KDT[K.dtype], _ptr(mu), *K.shape, _ptr(out), _stream(K.device))
+    return out
+
+
 class KLTPlaneStore(PlaneStore):
     """Bit-plane store of the KLT-rotated keys (K - mu) @ Vt (scripts/R_ruler.py:63-64).
 
@@ -80,7 +91,7 @@ class KLTPlaneStore(PlaneStore):
         self.mu = params["mu"].to(K.device, torch.float32).contiguous()
         self.Vt = params["Vt"].to(K.device, torch.float32).contiguous()
         self.lam = params["lam"].to(K.device, torch.float32).contiguous()
-        Kr = torch.matmul(K.float() - self.mu[:, None, :], self.Vt)
+        Kr = torch.matmul(_centered(K, self.mu), self.Vt)
         super().__init__(Kr, scale_dtype, keep_code)
 
     def query(self, q):

@@ -165,6 +165,14 @@ int fathom_klt_query(const float *q, const float *Vt, const float *lam, int64_t 
                      float *gain, void *stream);
 
 /*
+ * Centred keys of the KLT-rotated store's build (scripts/R_ruler.py:63-64):
+ * out[bh, i, j] = float(K[bh, i, j]) - mu[bh, j], float32.  K [BH, n, D] of
+ * k_dtype (FATHOM_DT_*), mu [BH, D] float32, BH <= 65535.
+ */
+int fathom_klt_center(const void *K, int k_dtype, const float *mu, int64_t BH, int64_t n, int64_t D, float *out,
+                      void *stream);
+
+/*
  * Fused scan + sink/local top-k: the selection of fathom_scan_planes followed by
  * fathom_sink_local_topk on its scores (kernels/bitplane.py:319-338 then
  * :372-378, as chained by scripts/B_kernel_bench.py:74 and

@@ -62,3 +62,16 @@ def test_build_equals_oracle_at_tile_edges(BH, n, sub, sdt, dtype, monkeypatch):
     np.testing.assert_array_equal(st.scales_blk[:, -1:].float().cpu().numpy(), sc_t)
     planes = bp.pack_planes(st.code[:, tail:].contiguous())
     np.testing.assert_array_equal(planes.cpu().numpy().view(np.uint64), O.pack_planes(code_t))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("BH,n,cut", [(1, 1, 0), (3, 257, 0), (2, 1000, 1)])
+def test_klt_centering_equals_torch(BH, n, cut, dtype):
+    """One rounding per element, as the conversion and the subtraction: equal bit for bit, whatever the alignment."""
+    from fathom_amd.klt import _centered
+    print(f"[klt center] {BH}x{n} {dtype}", flush=True)
+    flat = torch.randn(BH * n * 128 + cut, generator=torch.Generator().manual_seed(n)).to(dtype).to(DEV)
+    K = flat[cut:].view(BH, n, 128)             # cut = 1: rows off the vector loads' alignment
+    mu = torch.randn(BH, 128, generator=torch.Generator().manual_seed(1)).to(DEV)
+    assert torch.equal(_centered(K, mu), K.float() - mu[:, None, :])
+    assert torch.equal(_centered(K.transpose(0, 1).contiguous().transpose(0, 1), mu), K.float() - mu[:, None, :])
