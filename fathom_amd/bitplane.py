@@ -378,9 +378,8 @@ class PlaneStore:
         """plan_scan_topk(q, g, budget, k, ...) then offload.gather_attention over its
         indices with K/V bf16 rows [BH, cap, 128] in device memory: the decode
         step's plan -> scan -> top-k -> gather + attention chain
-        (scripts/B_kernel_bench.py:64-101) in one call.  Rows of at most 131072
-        tokens with k <= 512 and 96 query heads or more select and attend in the
-        same workgroups.  Returns
+        (scripts/B_kernel_bench.py:64-101) in one call.  With k <= 512 each row
+        is selected and attended in the same workgroup.  Returns
         (idx [BH, G, k] int64, out [BH, G, 128] fp32), equal to the separate
         calls'."""
         _need_gpu(q, g, Ksrc, Vsrc)
@@ -414,7 +413,7 @@ class PlaneStore:
     def plan_scan_topk(self, q, g, budget, k, sink=4, local=32, m=None, bmax=4, iters=30, return_t=False):
         """make_plan(g, budget, bmax, iters) then scan_topk(q, plan, k, sink, local, m)
         in one call (kernels/bitplane.py:83-116, then the scan and top-k): the same
-        indices [BH, G, k].  Rows of at most 131072 tokens are planned inside the
+        indices [BH, G, k].  Rows are planned inside the
         scan's prologue, so no plan launch precedes it (the decode chain of
         scripts/B_kernel_bench.py:74).  return_t=True also returns the plan's
         depths t [BH, D] int8."""

@@ -247,25 +247,33 @@ namespace fathom {
 int scan_topk_run(const float *q, int64_t BH, int64_t G, int64_t D, const int32_t *cls, const int32_t *clsn, int bmax,
                   int64_t units_max, const void *planes_sb, const void *scales_sb, int64_t n, int64_t nsb, int64_t sub, int64_t m,
                   int64_t k, int64_t sink, int64_t local, int64_t *idx, void *workspace, size_t workspace_bytes,
-                  int stages, void *stream, const AttnArgs *att) {
-  int rc = check_scan(q, BH, G, D, cls, clsn, bmax, planes_sb, scales_sb, n, nsb, sub, "scan_topk");
+                  int stages, void *stream, const AttnArgs *att, const OwnPlan *own) {
+  const char *who = own ? "plan_scan_topk" : "scan_topk";
+  int rc = check_scan(q, BH, G, D, cls, clsn, bmax, planes_sb, scales_sb, n, nsb, sub, who, own != nullptr);
   if (rc) return rc;
-  if (!idx) return fail(FATHOM_ERR_INVALID, "scan_topk: null output");
+  if (!idx) return fail(FATHOM_ERR_INVALID, "%s: null output", who);
   if (stages & ~FATHOM_STAGE_ALL) return fail(FATHOM_ERR_INVALID, "scan_topk: unknown stage bits 0x%x", stages);
   const int64_t rows = BH * G;
-  rc = check_topk_args(rows, n, m, k, sink, local, "scan_topk");
+  rc = check_topk_args(rows, n, m, k, sink, local, who);
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   const int64_t kk = k - sink - local;
   if (kk == 0) return (stages & FATHOM_STAGE_FINALIZE) ? launch_fixed_only(rows, m, k, sink, local, idx, st) : FATHOM_OK;
   const size_t need = scan_topk_ws(rows, n, k, kk);
   if (!workspace || workspace_bytes < need)
-    return fail(FATHOM_ERR_WORKSPACE, "scan_topk: workspace %zu bytes, need %zu", workspace_bytes, need);
+    return fail(FATHOM_ERR_WORKSPACE, "%s: workspace %zu bytes, need %zu", who, workspace_bytes, need);
   const int64_t nblk = cdiv(n, kBlk);
   ScanArgs a = make_args(q, G, D, cls, clsn, bmax, planes_sb, scales_sb, n, nsb, sub);
   a.blk0 = 0;
   a.blk_end = nblk;
   a.wt0 = 0;
+  if (own) {
+    a.g = own->g;
+    a.budget = own->budget;
+    a.budget_value = own->budget_value;
+    a.iters = own->iters;
+    a.t_out = own->t_out;
+  }
   const int64_t nwt = cdiv(nblk, kWB);
   const int64_t um = units_bound(units_max, D, bmax);
   if (kk > kSelMaxK && !group_select_takes(n, kk)) {
@@ -347,7 +355,8 @@ extern "C" int fathom_scan_topk_stages(const float *q, int64_t BH, int64_t G, in
 
 namespace fathom {
 namespace {
-// make_plan's arrays for plan_scan_topk's long rows, past the scan's workspace.
+// make_plan's arrays of plan_scan_topk with nothing to select, past the scan's
+// workspace.
 size_t plan_arrays_ws(int64_t BH, int64_t D, int bmax) {
   return ws_align((size_t)(BH * D)) + ws_align((size_t)(BH * D * bmax) * 4) + 2 * ws_align((size_t)BH * 4) +
          ws_align((size_t)(BH * D) * 4) + ws_align((size_t)(BH * bmax * D) * 4) + ws_align((size_t)(BH * bmax) * 4);
@@ -380,46 +389,34 @@ int plan_scan_topk_run(const float *q, const float *g, const float *budget, floa
   const size_t need = fathom_plan_scan_topk_workspace_bytes(BH, G, D, bmax, n, k, sink, local);
   if (!workspace || workspace_bytes < need)
     return fail(FATHOM_ERR_WORKSPACE, "plan_scan_topk: workspace %zu bytes, need %zu", workspace_bytes, need);
-  hipStream_t st = (hipStream_t)stream;
   const int64_t kk = k - sink - local;
   const size_t sws = scan_topk_ws(rows, n, k, kk);
-  if (kk == 0 || !group_select_takes(n, kk)) {
-    // make_plan into the workspace, then the fused scan + top-k
-    char *p = static_cast<char *>(workspace) + sws;
-    int8_t *t = t_out ? t_out : reinterpret_cast<int8_t *>(p);
-    p += ws_align((size_t)(BH * D));
-    int32_t *pairs = reinterpret_cast<int32_t *>(p);
-    p += ws_align((size_t)(BH * D * bmax) * 4);
-    int32_t *npairs = reinterpret_cast<int32_t *>(p);
-    p += ws_align((size_t)BH * 4);
-    int32_t *nact = reinterpret_cast<int32_t *>(p);
-    p += ws_align((size_t)BH * 4);
-    int32_t *act = reinterpret_cast<int32_t *>(p);
-    p += ws_align((size_t)(BH * D) * 4);
-    int32_t *cls = reinterpret_cast<int32_t *>(p);
-    p += ws_align((size_t)(BH * bmax * D) * 4);
-    int32_t *clsn = reinterpret_cast<int32_t *>(p);
-    rc = make_plan_run(g, budget, budget_value, BH, D, bmax, iters, t, pairs, npairs, act, nact, cls, clsn, stream);
-    if (rc) return rc;
-    return scan_topk_run(q, BH, G, D, cls, clsn, bmax, units_max, planes_sb, scales_sb, n, nsb, sub, m, k, sink, local,
-                         idx, workspace, sws, FATHOM_STAGE_ALL, stream, att);
+  if (kk == 0) {
+    // only the fixed positions are written; the plan's depths where asked for
+    if (t_out) {
+      char *p = static_cast<char *>(workspace) + sws + ws_align((size_t)(BH * D));
+      int32_t *pairs = reinterpret_cast<int32_t *>(p);
+      p += ws_align((size_t)(BH * D * bmax) * 4);
+      int32_t *npairs = reinterpret_cast<int32_t *>(p);
+      p += ws_align((size_t)BH * 4);
+      int32_t *nact = reinterpret_cast<int32_t *>(p);
+      p += ws_align((size_t)BH * 4);
+      int32_t *act = reinterpret_cast<int32_t *>(p);
+      p += ws_align((size_t)(BH * D) * 4);
+      int32_t *cls = reinterpret_cast<int32_t *>(p);
+      p += ws_align((size_t)(BH * bmax * D) * 4);
+      int32_t *clsn = reinterpret_cast<int32_t *>(p);
+      rc = make_plan_run(g, budget, budget_value, BH, D, bmax, iters, t_out, pairs, npairs, act, nact, cls, clsn, stream);
+      if (rc) return rc;
+    }
+    return launch_fixed_only(rows, m, k, sink, local, idx, (hipStream_t)stream);
   }
-  // every workgroup of the scan plans its row in the prologue
-  // (the plan kernel's arithmetic), then the rows are selected as in scan_topk
-  const int64_t nblk = cdiv(n, kBlk);
-  ScanArgs a = make_args(q, G, D, nullptr, nullptr, bmax, planes_sb, scales_sb, n, nsb, sub);
-  a.blk0 = 0;
-  a.blk_end = nblk;
-  a.wt0 = 0;
-  a.g = g;
-  a.budget = budget;
-  a.budget_value = budget_value;
-  a.iters = iters;
-  a.t_out = t_out;
-  const Emit es = group_max_emit(rows, n, m, sink, local, workspace);
-  rc = launch_scores_max(a, cdiv(nblk, kWB), BH, es, units_bound(units_max, D, bmax), st);
-  if (rc) return rc;
-  return launch_rowselect_gmax(es.out, es.gmax, rows, G, n, m, k, sink, local, idx, att, st);
+  // every workgroup of the scan (long rows: of its sample pass, which leaves the
+  // plan tables to the others) plans its row in the prologue with the plan
+  // kernel's arithmetic
+  const OwnPlan own{g, budget, budget_value, iters, t_out};
+  return scan_topk_run(q, BH, G, D, nullptr, nullptr, bmax, units_max, planes_sb, scales_sb, n, nsb, sub, m, k, sink,
+                       local, idx, workspace, sws, FATHOM_STAGE_ALL, stream, att, &own);
 }
 }  // namespace
 }  // namespace fathom

@@ -215,11 +215,10 @@ int fathom_scan_topk_stages(const float *q, int64_t BH, int64_t G, int64_t D, co
  * to fathom_make_plan (budget [BH], or budget_value for every row when budget
  * is null; bmax, iters as there) then fathom_scan_topk with that plan's cls and
  * clsn (kernels/bitplane.py:83-116 then :319-338 and :372-378, the plan ->
- * scan -> top-k stages of scripts/B_kernel_bench.py:74).  For rows of at most
- * 131072 tokens (D <= 128) every workgroup of the scan makes its row's plan in
- * its prologue with the plan kernel's arithmetic, so no plan launch and no
- * plan arrays precede the scan: the decode form of the chain.  Longer rows run
- * the plan kernel into the workspace first.  t_out [BH, D] int8 (nullable)
+ * scan -> top-k stages of scripts/B_kernel_bench.py:74).  Every workgroup of the
+ * scan (of its first pass, where there are several) makes its row's plan in its
+ * prologue with the plan kernel's arithmetic, so no plan launch and no plan arrays
+ * precede the scan: the decode form of the chain.  t_out [BH, D] int8 (nullable)
  * receives the plan's depths.  It composes reference stages and has no single
  * counterpart in the reference.
  * workspace: fathom_plan_scan_topk_workspace_bytes(BH, G, D, bmax, n, k, sink,
@@ -236,8 +235,7 @@ int fathom_plan_scan_topk(const float *q, const float *g, const float *budget, f
  * fathom_plan_scan_topk followed by fathom_gather_attention over its indices
  * (rows in device memory: Ksrc, Vsrc bf16 [BH, cap, 128], no recent rows),
  * the decode step's plan -> scan -> top-k -> gather + attention chain of
- * scripts/B_kernel_bench.py:64-101 in one call.  For rows of at most 131072
- * tokens, k <= 512 and 96 query heads or more each selection workgroup goes on to its query head's
+ * scripts/B_kernel_bench.py:64-101 in one call.  For k <= 512 each selection workgroup goes on to its query head's
  * attention over the indices it wrote (the arithmetic of gather_attention), so
  * idx and out equal the two calls'.  Other shapes run the two calls.  It
  * composes reference stages and has no single counterpart in the reference.

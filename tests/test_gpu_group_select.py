@@ -44,6 +44,19 @@ def test_fused_selection_at_its_limits(BH, G, n, k, sub, extra, monkeypatch):
             assert torch.equal(i2, got) and torch.equal(out, ref)
 
 
+def test_planned_call_with_nothing_to_select():
+    """k = sink + local: the fixed positions, and the plan's depths where asked for, on short and long rows."""
+    print("[group-select] k = sink + local", flush=True)
+    for n in (5000, 140000):
+        x = W.synth_layer(2, n, 4, seed=1, device=DEV, kdtype=torch.bfloat16)
+        g = ((x["q"] ** 2) * x["var"][:, None, :]).sum(1)
+        st = bp.PlaneStore(x["K"], keep_code=False)
+        idx, t = st.plan_scan_topk(x["q"], g, 48.0, 36, 4, 32, return_t=True)
+        assert torch.equal(t, bp.make_plan(g, 48.0)["t"])
+        want = torch.cat([torch.arange(4), torch.arange(n - 32, n)]).expand(2, 4, 36)
+        assert torch.equal(idx.cpu(), want) and torch.equal(st.plan_scan_topk(x["q"], g, 48.0, 36, 4, 32).cpu(), want)
+
+
 @pytest.mark.parametrize("n", [65536, 131072, 140001])
 @pytest.mark.parametrize("G", [4, 7])
 def test_ties_and_masks(n, G):
@@ -64,6 +77,8 @@ def test_ties_and_masks(n, G):
         scores = st.scan(q, plan)
         got = st.scan_topk(q, plan, 2000, 4, 32)
         assert torch.equal(got.cpu(), _oracle_topk(scores, 2000, 4, 32, n)), kind
+        idx, t = st.plan_scan_topk(q, gain, 6.0, 2000, 4, 32, return_t=True)
+        assert torch.equal(idx, got) and torch.equal(t, plan["t"]), kind
 
 
 @pytest.mark.parametrize("n,G", [(40000, 4), (131072, 6), (200000, 4)])
