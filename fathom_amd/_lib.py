@@ -27,6 +27,7 @@ PROTOTYPES = {
     "fathom_make_plan": (_i32, [_vp, _vp, _i64, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "fathom_make_plan_uniform": (_i32, [_vp, ctypes.c_float, _i64, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp,
                                         _vp, _vp]),
+    "fathom_row_values": (_i32, [_vp, _i64, _vp, _vp]),
     "fathom_scan_planes": (_i32, [_vp, _i64, _i64, _i64, _vp, _vp, _i32, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
                                   _vp, _vp]),
     "fathom_pack_chan4": (_i32, [_vp, _i64, _i64, _i64, _i64, _vp, _vp]),

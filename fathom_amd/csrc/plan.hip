@@ -102,10 +102,33 @@ __global__ __launch_bounds__(64) void channel_list_kernel(const uint8_t *__restr
   if (lane == 0) nact[bh] = total;
 }
 
+// Host values written to device memory as kernel arguments: the launch takes a copy
+// of them, so nothing waits for the device and the host buffer is free on return (a
+// copy from pageable memory holds the host until the stream gets to it).
+constexpr int kRowVals = 64;
+struct RowVals {
+  float v[kRowVals];
+};
+__global__ __launch_bounds__(kRowVals) void row_values_kernel(RowVals r, int n, float *__restrict__ out) {
+  if ((int)threadIdx.x < n) out[threadIdx.x] = r.v[threadIdx.x];
+}
+
 }  // namespace
 }  // namespace fathom
 
 using namespace fathom;
+
+extern "C" int fathom_row_values(const float *host_values, int64_t n, float *out, void *stream) {
+  if (!host_values || !out) return fail(FATHOM_ERR_INVALID, "row_values: null pointer");
+  if (n < 1 || n > 0x7FFFFFFF) return fail(FATHOM_ERR_INVALID, "row_values: n=%lld", (long long)n);
+  for (int64_t i = 0; i < n; i += kRowVals) {
+    RowVals r{};
+    const int m = (int)(n - i < kRowVals ? n - i : kRowVals);
+    for (int e = 0; e < m; ++e) r.v[e] = host_values[i + e];
+    row_values_kernel<<<1, kRowVals, 0, (hipStream_t)stream>>>(r, m, out + i);
+  }
+  return launch_status("row_values_kernel");
+}
 
 namespace fathom {
 int make_plan_run(const float *g, const float *budget, float budget_value, int64_t BH, int64_t D, int bmax, int iters,

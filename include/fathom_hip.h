@@ -108,6 +108,13 @@ int fathom_make_plan_uniform(const float *g, float budget, int64_t BH, int64_t D
                              int32_t *clsn, void *stream);
 
 /*
+ * n floats of host memory written to device memory in kernel arguments (per-row
+ * budgets that the caller holds on the host, kernels/bitplane.py:108-116): the
+ * values are taken before the call returns, and nothing waits for the stream.
+ */
+int fathom_row_values(const float *host_values, int64_t n, float *out, void *stream);
+
+/*
  * PlaneStore.scan (kernels/bitplane.py:319-338, scan_planes_cls_kernel :275-307):
  * out[bh, g, tok] = sum_j q[bh, g, j] * value_{t_j}(tok, j) over the channels of
  * the plan's depth classes 1..min(bmax, 4), for the 64-token blocks [blk0, blk1)

@@ -196,3 +196,18 @@ def test_attention_splits(BH, G, k):
             Ks[rows < 0], Vs[rows < 0] = 0.0, 0.0
             ref = torch.softmax(Ks @ q[b, h].double() * 128 ** -0.5, 0) @ Vs
             assert (out[b, h].cpu().double() - ref).abs().max() <= 1e-5 * ref.abs().max().clamp_min(1.0)
+
+
+@pytest.mark.parametrize("BH", [1, 3, 64, 65, 200, 257])
+def test_host_budgets_equal_device_budgets(BH):
+    """Per-row budgets from the host, of any dtype and shape that expands, reused at once by the caller."""
+    print(f"[budgets] BH={BH}", flush=True)
+    g = torch.rand(BH, 128, generator=torch.Generator().manual_seed(BH)).to(DEV) * 100
+    for host in (torch.linspace(40, 92, BH), torch.arange(BH) % 50 + 40, torch.tensor([48.5], dtype=torch.float64)):
+        want = bp.make_plan(g, host.to(DEV))["t"]
+        mine = host.clone()
+        got = bp.make_plan(g, mine)
+        mine.zero_()
+        assert torch.equal(got["t"], want)
+    with pytest.raises(RuntimeError):
+        bp.make_plan(g, torch.ones(BH + 1 if BH > 1 else 2))
