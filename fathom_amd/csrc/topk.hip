@@ -3,8 +3,10 @@
 // Orderable keys: score_key maps a float to a uint32 whose unsigned order is
 // torch.topk's value order; K64 = key << 32 | (0xFFFFFFFF - index) makes every
 // element of a row distinct and orders equal scores by ascending index.
-// The selection runs select -> filter -> finalize (topk_internal.hpp); the
-// fused scan+top-k path replaces `filter` by the scan kernel's own emission.
+// Rows of up to 131072 tokens (wide selections: 524288) are selected by one
+// workgroup each, from their 16-token group maxima or read whole; longer ones run
+// select -> filter -> finalize (topk_internal.hpp), where the fused scan+top-k
+// replaces `filter` by the scan kernel's own emission.
 //
 // Selection of the need-th largest value of a set (range_select): the active
 // values lie in [lo, hi]; a 2048-bin LDS histogram of (v - lo) >> s, with s
@@ -27,7 +29,6 @@ constexpr int kSelThreads = 1024;
 constexpr int kSelPer = (int)(kMaxSample / kSelThreads);  // keys per thread in select
 constexpr int kFinThreads = 1024;
 constexpr int kFilterThreads = 256;
-constexpr int64_t kFilterChunk = 16384;
 constexpr uint32_t kFilterLocal = 2048;  // LDS candidates per filter workgroup
 constexpr int kCandLds = 16384;          // candidates selected in LDS (128 KB)
 constexpr int kMaxK = (int)kSelMaxK;      // largest kk of these selections
@@ -640,12 +641,13 @@ __global__ __launch_bounds__(256) void group_max_kernel(const float *__restrict_
   if (g < ngrp) gmax[row * ngrp + g] = mine;
 }
 
-// Candidates of score rows (keys >= the row's threshold), 4 scores per thread
-// and step when rows are 16-byte aligned.
-template <bool VEC>
+// Candidates of score rows (keys >= the row's threshold): kPer scores per thread
+// and step, their loads in flight at once, 16-byte loads when rows are 16-byte aligned.
+// Bound: HBM, 4 bytes per score (sink_local_topk: see launch_filter_scores).
+template <bool VEC, int kPer>
 __global__ __launch_bounds__(kFilterThreads) void filter_scores_kernel(const float *__restrict__ scores, int64_t n,
                                                                        int64_t sink, int64_t lstart, TopkSel s,
-                                                                       bool fallback) {
+                                                                       bool fallback, int steps) {
   __shared__ uint64_t lbuf[kFilterLocal];
   __shared__ uint32_t lcnt, lbase;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -657,30 +659,31 @@ __global__ __launch_bounds__(kFilterThreads) void filter_scores_kernel(const flo
   uint64_t *cand = s.cand + row * s.cand_cap;
   if (tid == 0) lcnt = 0u;
   __syncthreads();
-  const int64_t start = (int64_t)blockIdx.x * kFilterChunk;
-  const int64_t end = min(start + kFilterChunk, n);
-  if (VEC) {
-    for (int64_t i0 = start; i0 < end; i0 += 4 * kFilterThreads) {
-      const int64_t i = i0 + 4 * tid;
-      float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (i < end) f = *reinterpret_cast<const float4 *>(rs + i);
-      const float fv[4] = {f.x, f.y, f.z, f.w};
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int64_t iu = i + u;
-        const bool in = iu < end;
-        const uint32_t key = in ? ((iu < sink || iu >= lstart) ? kKeyNegInf : score_key(fv[u])) : 0u;
-        wave_append_local(in && key >= thr, k64_of(key, iu), &lcnt, lbuf, kFilterLocal, cnt, cand,
-                          (uint64_t)s.cand_cap, lane);
+  constexpr int64_t kFilterStep = kPer * kFilterThreads;
+  const int64_t end = min((int64_t)(blockIdx.x + 1) * steps * kFilterStep, n);
+  for (int64_t start = (int64_t)blockIdx.x * steps * kFilterStep; start < end; start += kFilterStep) {  // uniform
+    const auto at = [&](int u) { return start + (VEC ? 4 * (tid + kFilterThreads * (u >> 2)) + (u & 3) : tid + kFilterThreads * u); };
+    float v[kPer];
+  #pragma unroll
+    for (int u = 0; u < kPer; u += VEC ? 4 : 1) {
+      const int64_t i = at(u);
+      if constexpr (VEC) {  // n is a multiple of 4
+        float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (i < n) f = *reinterpret_cast<const float4 *>(rs + i);
+        v[u] = f.x;
+        v[u + 1] = f.y;
+        v[u + 2] = f.z;
+        v[u + 3] = f.w;
+      } else {
+        v[u] = i < n ? rs[i] : 0.0f;
       }
     }
-  } else {
-    for (int64_t i0 = start; i0 < end; i0 += kFilterThreads) {
-      const int64_t i = i0 + tid;
-      const bool in = i < end;
-      const uint32_t key = in ? masked_key(rs, i, sink, lstart) : 0u;
-      wave_append_local(in && key >= thr, k64_of(key, i), &lcnt, lbuf, kFilterLocal, cnt, cand,
-                        (uint64_t)s.cand_cap, lane);
+  #pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int64_t i = at(u);
+      const bool in = i < n;
+      const uint32_t key = in ? ((i < sink || i >= lstart) ? kKeyNegInf : score_key(v[u])) : 0u;
+      wave_append_local(in && key >= thr, k64_of(key, i), &lcnt, lbuf, kFilterLocal, cnt, cand, (uint64_t)s.cand_cap, lane);
     }
   }
   __syncthreads();
@@ -1714,13 +1717,20 @@ int launch_sample_scores(const float *scores, int64_t rows, int64_t n, int64_t S
   return launch_status("sample_scores_kernel");
 }
 
+// One step of 4096 scores per workgroup, four where the launch is large anyway
+// (fewer counter atomics per row).  sink_local_topk, k = 512, us, before (16384 scores
+// per workgroup, a load per step) and now: 32 rows of 200001 tokens 54.6; 34.5, 4 rows
+// 43.3; 29.2, 32 of 300007 56.2; 38.2, 4 of 1048576 38.4; 30.7, 32 of 1048576 48.5; ZZ (54.6
+// in single steps).
 int launch_filter_scores(const float *scores, int64_t rows, int64_t n, int64_t sink, int64_t lstart, TopkSel s,
                          bool fallback, hipStream_t st) {
-  const dim3 grid((unsigned)cdiv(n, kFilterChunk), (unsigned)rows);
-  if (n % 4 == 0 && reinterpret_cast<uintptr_t>(scores) % 16 == 0)
-    filter_scores_kernel<true><<<grid, kFilterThreads, 0, st>>>(scores, n, sink, lstart, s, fallback);
-  else
-    filter_scores_kernel<false><<<grid, kFilterThreads, 0, st>>>(scores, n, sink, lstart, s, fallback);
+  const bool large = rows * n >= (int64_t)1 << 24;
+  const int steps = large ? 16 : 1;
+  const dim3 grid((unsigned)cdiv(n, 16 * kFilterThreads * (large ? 4 : 1)), (unsigned)rows);
+  const bool vec = n % 4 == 0 && reinterpret_cast<uintptr_t>(scores) % 16 == 0;
+  const auto run = [&](auto kernel) { kernel<<<grid, kFilterThreads, 0, st>>>(scores, n, sink, lstart, s, fallback, steps); };
+  if (large) vec ? run(filter_scores_kernel<true, 4>) : run(filter_scores_kernel<false, 4>);
+  else vec ? run(filter_scores_kernel<true, 16>) : run(filter_scores_kernel<false, 16>);
   return launch_status("filter_scores_kernel");
 }
 
