@@ -1545,7 +1545,9 @@ __device__ __forceinline__ void tile_loop(const ScanArgs &a, const Emit &em, con
 }
 
 // The workgroup's unit -> channel slot map of the stage (units of one channel
-// are consecutive and share a scale offset) and the slots' scale offsets.
+// are consecutive and share a scale offset) and the slots' scale offsets.  A
+// plan without units has no slot; slot 0 then holds unit 0's offset (zero, as
+// every padding unit's), since host_stage's loads fall back to that slot.
 __device__ __forceinline__ void host_slots(HostStage &hs, const Shared &sh, int ureal) {
   const int tid = threadIdx.x;
   if (tid < kWave) {
@@ -1555,7 +1557,7 @@ __device__ __forceinline__ void host_slots(HostStage &hs, const Shared &sh, int 
     const uint64_t le = u == kWave - 1 ? ~0ull : (2ull << u) - 1ull;  // lanes <= u
     const int slot = (int)__builtin_popcountll(m & le) - 1;
     hs.uslot[u] = (uint8_t)(u < ureal && slot >= 0 ? slot : 0);
-    if (first) hs.soff1[slot] = sh.soff[u];
+    if (first || u == 0) hs.soff1[u == 0 ? 0 : slot] = sh.soff[u];
     if (u == 0) hs.nch = (int)__builtin_popcountll(m);
   }
 }

@@ -105,6 +105,29 @@ def test_host_resident_staged_scan_equals_hbm(n, G, monkeypatch):
         assert torch.equal(a, b) and torch.equal(a, c)
 
 
+@pytest.mark.parametrize("n,G", [(40000, 4), (40000, 6), (200000, 4)])
+def test_staged_scan_of_plans_without_units(n, G, monkeypatch):
+    """Superblocks of 64 blocks (staged tiles): rows whose plan lists no channel -- budget 0, and a zero query row among
+    others -- give the indices of the direct scan over superblocks of 16."""
+    print(f"[group-select empty plan] n={n} G={G}", flush=True)
+    x = W.synth_layer(2, n, G, seed=4, device=DEV, kdtype=torch.bfloat16)
+    q = x["q"].clone()
+    q[1] = 0.0                              # a padded batch slot: every gain at the floor
+    g = ((q ** 2) * x["var"][:, None, :]).sum(1)
+    got = {}
+    for sub in (16, 64):
+        monkeypatch.setattr(bp, "SUB", sub)
+        st = bp.PlaneStore(x["K"], keep_code=False)
+        for budget in (0.0, 48.0, torch.tensor([0.5, 48.0])):
+            plan = bp.make_plan(g, budget)
+            idx, t = st.plan_scan_topk(q, g, budget, 512, 4, 32, return_t=True)
+            assert torch.equal(st.scan_topk(q, plan, 512, 4, 32), idx) and torch.equal(t, plan["t"])
+            got.setdefault(sub, []).append(idx)
+    assert all(torch.equal(a, b) for a, b in zip(got[16], got[64]))
+    first = torch.cat([torch.arange(4, 480), torch.arange(4), torch.arange(n - 32, n)])  # every score equal
+    assert torch.equal(got[64][0].cpu(), first.expand(2, G, 512))
+
+
 def _score_rows(kind, rows, n, seed):
     rng = np.random.default_rng(seed)
     s = rng.standard_normal((rows, n)).astype(np.float32)
