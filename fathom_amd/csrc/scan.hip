@@ -58,8 +58,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(
       const int nsl = __builtin_amdgcn_readfirstlane(sh.U) / kSlice;
       const int ureal = __builtin_amdgcn_readfirstlane(sh.ureal);
       if (nsl <= NSMAX) {  // uniform; larger plans read the store directly
-        if (a.G <= kMaxG / 2)
-          host_tile_loop<MODE, NSMAX, false, true>(a, em, sh, hst, bh, lane, wave, nlist, 0u, nsl, ureal);
+        constexpr bool kStk = MODE != kEmitQuadsMax;  // quad order: more than four heads
+        if (kStk && a.G <= kMaxG / 2)
+          host_tile_loop<MODE, NSMAX, false, kStk>(a, em, sh, hst, bh, lane, wave, nlist, 0u, nsl, ureal);
         else
           host_tile_loop<MODE, NSMAX, false, false>(a, em, sh, hst, bh, lane, wave, nlist, 0u, nsl, ureal);
         return;
@@ -134,7 +135,6 @@ int launch_scores_max(const ScanArgs &a, int64_t nwt, int64_t BH, const Emit &em
 Emit group_max_emit(int64_t rows, int64_t n, int64_t m, int64_t sink, int64_t local, void *workspace) {
   Emit es{};
   es.out = static_cast<float *>(workspace);
-  es.ostride = tile_score_floats(n);
   es.gmax = reinterpret_cast<uint32_t *>(static_cast<char *>(workspace) +
                                          ws_align((size_t)rows * (size_t)tile_score_floats(n) * 4));
   es.sink = sink;
@@ -214,7 +214,6 @@ extern "C" int fathom_scan_planes(const float *q, int64_t BH, int64_t G, int64_t
   a.wt0 = blk0 / kWB;
   Emit em{};
   em.out = out;
-  em.ostride = n;
   return launch_scan<kEmitScores>(a, cdiv(blk_end, kWB) - a.wt0, BH, em, units_bound(units_max, D, bmax),
                                   (hipStream_t)stream);
 }
@@ -282,7 +281,6 @@ int scan_topk_run(const float *q, int64_t BH, int64_t G, int64_t D, const int32_
     // its candidate lists (the finalize stage)
     Emit es{};
     es.out = static_cast<float *>(workspace);
-    es.ostride = n;
     const size_t sb = ws_align((size_t)rows * (size_t)n * 4);
     if (stages & FATHOM_STAGE_CANDIDATES) {
       rc = launch_scan<kEmitScores>(a, nwt, BH, es, um, st);

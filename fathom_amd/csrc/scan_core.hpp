@@ -95,8 +95,7 @@ struct ScanArgs {
 struct PlanTab;
 
 struct Emit {
-  float *out;        // scores [BH, G] rows of ostride floats (kEmitQuadsMax: quad order)
-  int64_t ostride;   // n, or whole blocks (kEmitScoresMax)
+  float *out;        // scores [BH, G] rows of n floats (kEmitScoresMax: of whole blocks; kEmitQuadsMax: quad order)
   uint32_t *gmax;    // kEmitScoresMax, kEmitQuadsMax: [BH * G, ceil(n / 16)] each 16-token group's largest masked key
   uint32_t *samp;    // sampled keys [BH * G, samp_cap]: list entry L at L * kWTok
   int64_t samp_cap;
@@ -813,12 +812,9 @@ __device__ __forceinline__ void emit_filter_w(const Emit &em, const ScanArgs &a,
 }
 
 // Scores of step group V of quarter qs, from the four step classes' scores
-// s4[slot][w]: each lane stores its block's four consecutive tokens per head
-// (and, GMAX, folds them into the quarter's group maximum, written once the
-// quarter ends).
-template <bool GMAX, bool QUADS>
-__device__ __forceinline__ void store_scores(const Emit &em, const ScanArgs &a, const float (&s4)[2][4], EmitState &es,
-                                             int64_t bh, int64_t beta0, int qs, int V, int lane) {
+// s4[slot][w]: each lane stores its block's four consecutive tokens per head.
+__device__ __forceinline__ void store_scores(const Emit &em, const ScanArgs &a, const float (&s4)[2][4], int64_t bh,
+                                             int64_t beta0, int qs, int V, int lane) {
   const int c = lane & 15, gp = lane >> 4;
   const int64_t blk = beta0 + c;
   const bool inr = blk >= a.blk0 && blk < a.blk_end;
@@ -829,31 +825,77 @@ __device__ __forceinline__ void store_scores(const Emit &em, const ScanArgs &a, 
     const int h = 2 * gp + i;
     if (h >= a.G || !inr || tq >= a.n) continue;
     const float *s = s4[i];
-    float *dst = em.out + (QUADS ? quad_score_at(a.n, a.G, bh, h, beta0, c, 4 * qs + V) : (bh * a.G + h) * em.ostride + t4);
-    if (GMAX || (t4 + 4 <= a.n && (a.n & 3) == 0)) {
+    float *dst = em.out + (bh * a.G + h) * a.n + t4;
+    if (t4 + 4 <= a.n && (a.n & 3) == 0) {
       *reinterpret_cast<f4 *>(dst) = f4{s[0], s[1], s[2], s[3]};
     } else {
 #pragma unroll
       for (int w = 0; w < 4; ++w)
         if (t4 + w < a.n) dst[w] = s[w];
     }
-    if constexpr (GMAX) {  // a quarter's step groups come V = 3 first, V = 0 last
-      if (V == 3) {
-        es.gm[i] = -INFINITY;
-        es.gnan[i] = false;
-      }
+  }
+}
+
+// The scores with group maxima (whole rows of at most kGmaxWideMax tokens): a
+// row's heads lie within 2^32 bytes of its first, so a lane addresses them by a
+// 32-bit offset from a wave-uniform base, and its tokens by their number in the
+// tile.  With 64-bit row and token numbers per lane and head the kernels of four
+// waves per SIMD held 93 (four slices), 14 (three) and 60 (four, quad order)
+// registers in scratch, now 14, 0 and 0: a decode call over 32 x 4 heads of 32768
+// tokens 38.0 -> 36.8 us, the rotated store's calls over 8 x 7 heads of 131072 81.3 -> 78.0.
+static_assert(kMaxG * (kGmaxWideMax + kBlk) * 4 < ((int64_t)1 << 31), "a row's heads in 32-bit offsets");
+template <bool QUADS>
+__device__ __forceinline__ char *score_base(const Emit &em, const ScanArgs &a, int64_t bh, int64_t beta0) {
+  const int64_t nblk = cdiv(a.n, kBlk);
+  return reinterpret_cast<char *>(em.out + (QUADS ? (bh * nblk + beta0) * (kBlk * a.G) : bh * a.G * nblk * kBlk + beta0 * kBlk));
+}
+// Byte offset from score_base of token tt of the tile (QUADS: a quad's first), head h.
+template <bool QUADS>
+__device__ __forceinline__ uint32_t score_off(const ScanArgs &a, int64_t beta0, int h, uint32_t tt) {
+  const uint32_t nblk = (uint32_t)cdiv(a.n, kBlk);
+  if constexpr (QUADS) return quad_off(nblk, (uint32_t)a.G, (uint32_t)h, (uint32_t)beta0, tt) * 4u;
+  else return ((uint32_t)h * (nblk * kBlk) + tt) * 4u;
+}
+// A quarter's group maximum.
+__device__ __forceinline__ void store_gmax(const Emit &em, const ScanArgs &a, const EmitState &es, int64_t bh,
+                                           int64_t beta0, int h, int c, int qs, float gm, bool gnan) {
+  const int64_t ngrp = cdiv(a.n, kR);
+  char *base = reinterpret_cast<char *>(em.gmax + bh * a.G * ngrp + beta0 * kQS);
+  *reinterpret_cast<uint32_t *>(base + ((uint32_t)h * (uint32_t)ngrp + (uint32_t)(c * kQS + qs)) * 4u) =
+      gnan ? 0xFFFFFFFFu : score_key(gm);
+}
+// Folds the scores s[0 .. N) of the tokens from tt of the tile into a slot's
+// running group maximum; a quarter's step groups come V = 3 first, V = 0 last.
+template <int N>
+__device__ __forceinline__ void fold_gmax(EmitState &es, int i, const float (&s)[N], uint32_t tt, int V) {
+  if (V == 3) {
+    es.gm[i] = -INFINITY;
+    es.gnan[i] = false;
+  }
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const int64_t tok = t4 + w;
-        const float v = (es.plain || (tok < a.n && tok >= em.sink && tok < em.lstart)) ? s[w] : -INFINITY;
-        es.gm[i] = fmaxf(es.gm[i], v);
-        es.gnan[i] = es.gnan[i] || (v != v);
-      }
-      if (V == 0) {
-        const int64_t ngrp = (a.n + kR - 1) / kR;
-        em.gmax[(bh * a.G + h) * ngrp + blk * 4 + qs] = es.gnan[i] ? 0xFFFFFFFFu : score_key(es.gm[i]);
-      }
-    }
+  for (int w = 0; w < N; ++w) {
+    const float v = (es.plain || tt + w - es.mlo < es.mlen) ? s[w] : -INFINITY;
+    es.gm[i] = fmaxf(es.gm[i], v);
+    es.gnan[i] = es.gnan[i] || (v != v);
+  }
+}
+
+// Scores and group maxima of step group V of quarter qs (store_scores).  Rows
+// are held in whole blocks, so a stored quad may pass the row's end.
+template <bool QUADS>
+__device__ __forceinline__ void store_scores_max(const Emit &em, const ScanArgs &a, const float (&s4)[2][4],
+                                                 EmitState &es, int64_t bh, int64_t beta0, int qs, int V, int lane) {
+  const int c = lane & 15, gp = lane >> 4;
+  const uint32_t tq = (uint32_t)(c * kBlk + 16 * qs), t4 = tq + 4 * V;
+  char *base = score_base<QUADS>(em, a, bh, beta0);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int h = 2 * gp + i;
+    if (h >= a.G || tq >= es.vlen) continue;
+    const float *s = s4[i];
+    *reinterpret_cast<f4 *>(base + score_off<QUADS>(a, beta0, h, t4)) = f4{s[0], s[1], s[2], s[3]};
+    fold_gmax(es, i, s4[i], t4, V);
+    if (V == 0) store_gmax(em, a, es, bh, beta0, h, c, qs, es.gm[i], es.gnan[i]);
   }
 }
 
@@ -906,8 +948,8 @@ __device__ __forceinline__ void emit_w(const Emit &em, const ScanArgs &a, const 
 template <int MODE>
 __device__ __forceinline__ void emit_flush(const Emit &em, const ScanArgs &a, EmitState &es, const StepOut &o,
                                            int64_t bh, int64_t beta0, int64_t L, int qs, int V, int lane) {
-  if constexpr (MODE == kEmitScores) store_scores<false, false>(em, a, o.s4, es, bh, beta0, qs, V, lane);
-  if constexpr (emits_max(MODE)) store_scores<true, MODE == kEmitQuadsMax>(em, a, o.s4, es, bh, beta0, qs, V, lane);
+  if constexpr (MODE == kEmitScores) store_scores(em, a, o.s4, bh, beta0, qs, V, lane);
+  if constexpr (emits_max(MODE)) store_scores_max<MODE == kEmitQuadsMax>(em, a, o.s4, es, bh, beta0, qs, V, lane);
   if constexpr (MODE == kEmitSample) store_sample(em, a, o.s4, es, bh, beta0, L, qs, V, lane);
 }
 
@@ -942,7 +984,7 @@ __device__ __forceinline__ void tile_setup(EmitState &es, const Emit &em, const 
   const int64_t t0 = beta0 * kBlk, t1 = t0 + kWTok;
   es.plain = beta0 >= a.blk0 && beta0 + kWB <= a.blk_end && t1 <= a.n && t0 >= em.sink && t1 <= em.lstart;
   es.off[0] = es.off[1] = 0u;
-  if constexpr (MODE == kEmitFilter) {
+  if constexpr (MODE == kEmitFilter || emits_max(MODE)) {
     if (es.plain) {  // uniform
       es.vlo = es.mlo = 0u;
       es.vlen = es.mlen = (uint32_t)kWTok;
@@ -955,8 +997,10 @@ __device__ __forceinline__ void tile_setup(EmitState &es, const Emit &em, const 
         rlen = (uint32_t)max(h - l, (int64_t)0);
       };
       rel(max(a.blk0 * kBlk, (int64_t)0), min(a.blk_end * kBlk, a.n), es.vlo, es.vlen);
-      rel(em.sink, em.lstart, es.mlo, es.mlen);
+      rel(em.sink, emits_max(MODE) ? min(em.lstart, a.n) : em.lstart, es.mlo, es.mlen);
     }
+  }
+  if constexpr (MODE == kEmitFilter) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       es.head[i] = rk.head[i];
@@ -1193,11 +1237,9 @@ __device__ __forceinline__ void emit_pair(const Emit &em, const ScanArgs &a, con
 }
 
 // store_scores for stacked classes: each lane stores its block's two
-// consecutive tokens 4V + 2 (lane >= 32) + {0, 1} per head; a quarter's group
-// maximum joins the halves of lanes l and l ^ 32.
-template <bool GMAX>
-__device__ __forceinline__ void store_scores_stk(const Emit &em, const ScanArgs &a, const float (&s2)[2][2],
-                                                 EmitState &es, int64_t bh, int64_t beta0, int qs, int V, int lane) {
+// consecutive tokens 4V + 2 (lane >= 32) + {0, 1} per head.
+__device__ __forceinline__ void store_scores_stk(const Emit &em, const ScanArgs &a, const float (&s2)[2][2], int64_t bh,
+                                                 int64_t beta0, int qs, int V, int lane) {
   const int c = lane & 15, gh = (lane >> 4) & 1, up = lane >> 5;
   const int64_t blk = beta0 + c;
   const bool inr = blk >= a.blk0 && blk < a.blk_end;
@@ -1206,38 +1248,34 @@ __device__ __forceinline__ void store_scores_stk(const Emit &em, const ScanArgs 
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int h = 2 * gh + i;
-    const bool on = h < a.G && inr && tq < a.n;
-    if (on) {
-      float *dst = em.out + (bh * a.G + h) * em.ostride + t2;
-      if (GMAX || (t2 + 2 <= a.n && (a.n & 1) == 0)) {
-        *reinterpret_cast<f2 *>(dst) = f2{s2[i][0], s2[i][1]};
-      } else {
-        if (t2 < a.n) dst[0] = s2[i][0];
-        if (t2 + 1 < a.n) dst[1] = s2[i][1];
-      }
+    if (h >= a.G || !inr || tq >= a.n) continue;
+    float *dst = em.out + (bh * a.G + h) * a.n + t2;
+    if (t2 + 2 <= a.n && (a.n & 1) == 0) {
+      *reinterpret_cast<f2 *>(dst) = f2{s2[i][0], s2[i][1]};
+    } else {
+      if (t2 < a.n) dst[0] = s2[i][0];
+      if (t2 + 1 < a.n) dst[1] = s2[i][1];
     }
-    if constexpr (GMAX) {  // a quarter's step groups come V = 3 first, V = 0 last
-      if (V == 3) {
-        es.gm[i] = -INFINITY;
-        es.gnan[i] = false;
-      }
+  }
+}
+
+// store_scores_max for stacked classes (rows of at most four heads keep the
+// padded order); a quarter's group maximum joins the halves of lanes l and l ^ 32.
+__device__ __forceinline__ void store_scores_max_stk(const Emit &em, const ScanArgs &a, const float (&s2)[2][2],
+                                                     EmitState &es, int64_t bh, int64_t beta0, int qs, int V, int lane) {
+  const int c = lane & 15, gh = (lane >> 4) & 1, up = lane >> 5;
+  const uint32_t tq = (uint32_t)(c * kBlk + 16 * qs), t2 = tq + 4 * V + 2 * up;
+  char *base = score_base<false>(em, a, bh, beta0);
 #pragma unroll
-      for (int w = 0; w < 2; ++w) {
-        const int64_t tok = t2 + w;
-        const float v = (es.plain || (tok < a.n && tok >= em.sink && tok < em.lstart)) ? s2[i][w] : -INFINITY;
-        es.gm[i] = fmaxf(es.gm[i], v);
-        es.gnan[i] = es.gnan[i] || (v != v);
-      }
-      if (V == 0) {
-        const float og = __shfl_xor(es.gm[i], 32, 64);
-        const int on2 = __shfl_xor((int)es.gnan[i], 32, 64);
-        const bool gnan = es.gnan[i] || on2 != 0;
-        const float gm = fmaxf(es.gm[i], og);
-        if (on && up == 0) {
-          const int64_t ngrp = (a.n + kR - 1) / kR;
-          em.gmax[(bh * a.G + h) * ngrp + blk * 4 + qs] = gnan ? 0xFFFFFFFFu : score_key(gm);
-        }
-      }
+  for (int i = 0; i < 2; ++i) {
+    const int h = 2 * gh + i;
+    const bool on = h < a.G && tq < es.vlen;
+    if (on) *reinterpret_cast<f2 *>(base + score_off<false>(a, beta0, h, t2)) = f2{s2[i][0], s2[i][1]};
+    fold_gmax(es, i, s2[i], t2, V);
+    if (V == 0) {
+      const float gm = fmaxf(es.gm[i], __shfl_xor(es.gm[i], 32, 64));
+      const bool gnan = es.gnan[i] || __shfl_xor((int)es.gnan[i], 32, 64) != 0;
+      if (on && up == 0) store_gmax(em, a, es, bh, beta0, h, c, qs, gm, gnan);
     }
   }
 }
@@ -1290,8 +1328,8 @@ __device__ __forceinline__ void step_group_stk(const uint32_t (&qlo)[NS][2], con
   emit_pair<MODE, 0>(em, a, p0, k, es, o, bh, beta0, qs, V, lane);
   __builtin_amdgcn_sched_barrier(0);
   emit_pair<MODE, 1>(em, a, p1, k, es, o, bh, beta0, qs, V, lane);
-  if constexpr (MODE == kEmitScores) store_scores_stk<false>(em, a, o.s, es, bh, beta0, qs, V, lane);
-  if constexpr (emits_max(MODE)) store_scores_stk<true>(em, a, o.s, es, bh, beta0, qs, V, lane);
+  if constexpr (MODE == kEmitScores) store_scores_stk(em, a, o.s, bh, beta0, qs, V, lane);
+  if constexpr (MODE == kEmitScoresMax) store_scores_max_stk(em, a, o.s, es, bh, beta0, qs, V, lane);
   if constexpr (MODE == kEmitSample) store_sample_stk(em, a, o.s, es, bh, beta0, L, qs, V, lane);
 }
 
@@ -1649,8 +1687,9 @@ __device__ __forceinline__ void tile_pass(const ScanArgs &a, const Emit &em, con
   constexpr int GS = ACC == 4 ? kGS : 2;  // the register groups of a kernel tuned for small plans stay small
   const int nsl = __builtin_amdgcn_readfirstlane(sh.U) / kSlice;
   const int ureal = __builtin_amdgcn_readfirstlane(sh.ureal);
-  if (nsl <= NSMAX && a.G <= kMaxG / 2)
-    tile_loop<MODE, NSMAX, ACC, FB, GS, true>(a, em, sh, bh, lane, L0, Ls, nlist, qa0, qa1, skipm, nsl, ureal);
+  constexpr bool kStk = MODE != kEmitQuadsMax;  // quad order: more than four heads
+  if (kStk && nsl <= NSMAX && a.G <= kMaxG / 2)
+    tile_loop<MODE, NSMAX, ACC, FB, GS, kStk>(a, em, sh, bh, lane, L0, Ls, nlist, qa0, qa1, skipm, nsl, ureal);
   else if (nsl <= NSMAX)
     tile_loop<MODE, NSMAX, ACC, FB, GS>(a, em, sh, bh, lane, L0, Ls, nlist, qa0, qa1, skipm, nsl, ureal);
   else

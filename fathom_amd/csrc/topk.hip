@@ -1245,8 +1245,7 @@ struct QuadScores {  // quad_order(G, n) true
         n(n_), G((int)G_), h((int)(blockIdx.x % (uint32_t)G_)) {}
   __device__ __forceinline__ int64_t quad_at(int64_t i) const {  // the quad that holds token i
     const int64_t beta0 = i / kRegTok * (kRegTok / kBlk);
-    const int t = (int)(i - beta0 * kBlk);
-    return quad_score_at(n, G, 0, h, beta0, t / kBlk, (t % kBlk) / 4);
+    return beta0 * (int64_t)(kBlk * G) + quad_off((uint32_t)cdiv(n, kBlk), (uint32_t)G, (uint32_t)h, (uint32_t)beta0, (uint32_t)(i - beta0 * kBlk));
   }
   __device__ __forceinline__ float operator[](int64_t i) const { return p[quad_at(i) + (i & 3)]; }
   __device__ __forceinline__ void group(int64_t t0, float (&v)[kGroupTok]) const {

@@ -88,11 +88,11 @@ inline bool group_select_takes(int64_t n, int64_t kk) {
 // and of 131071 tokens 30.3 padded against 37.1 unpadded.
 __host__ __device__ inline int64_t tile_score_floats(int64_t n) { return cdiv(n, kBlk) * kBlk; }
 __host__ __device__ inline bool quad_order(int64_t G, int64_t n) { return G > 4 && n > kRowSelectMax; }
-// Where the first token of a quad of block beta0 + c (beta0 the tile's first) is.
-__device__ __forceinline__ int64_t quad_score_at(int64_t n, int G, int64_t bh, int h, int64_t beta0, int c, int quad) {
-  const int64_t nblk = cdiv(n, kBlk);
-  const int nbt = (int)(nblk - beta0 < kRegTok / kBlk ? nblk - beta0 : kRegTok / kBlk);
-  return (bh * nblk + beta0) * (int64_t)(kBlk * G) + ((quad * G + h) * nbt + c) * 4;
+// Where the quad of token tt of the tile of blocks beta0 .. is, from the tile's first score.
+__device__ __forceinline__ uint32_t quad_off(uint32_t nblk, uint32_t G, uint32_t h, uint32_t beta0, uint32_t tt) {
+  constexpr uint32_t kTile = (uint32_t)(kRegTok / kBlk);
+  const uint32_t nbt = min(nblk - beta0, kTile);
+  return (((tt % kBlk) / 4u * G + h) * nbt + tt / kBlk) * 4u;
 }
 
 // Candidate counters of a row, one per 256 bytes: every workgroup of a pass
