@@ -234,18 +234,21 @@ struct KeyBins {
 // values placed in bin order).  Bins whose values all rank at or past limit are
 // left out.  Values crowd a bin only where their range is
 // dominated by a few outliers: then (more than kCrowd in one bin) the ranks
-// come from block_rank_desc over the first nlim slots instead.  put(rank, v)
+// come from block_rank_desc over the first nlim slots instead (LINEAR: nothing is
+// ranked and the call returns false).  put(rank, v)
 // is called for every valid value of rank below limit (and some past it).  scratch: LDS of max(E * 1024 + 2048,
 // 2 * nlim) values.
 // The bits of a key grow with the logarithm of the score's magnitude: right for the
 // tail above a threshold, with its outliers, but a whole row's scores, of both
 // signs, crowd into a few dozen bins; those take LINEAR (n = 1000, the selection:
 // 13.8 -> 4.8 us).
-constexpr uint32_t kCrowd = 48;
+// The sort of 8192 allows its bins more before it falls back, to about 80 us of merges
+// (32 rows of 500000 tokens, correlation length 4, k = 6136: 177 -> 102 us).
 template <int E, bool LINEAR = false, typename Put>
-__device__ __forceinline__ void bin_rank_desc(const uint64_t (&v)[E], int cnt, int limit, uint64_t *scratch,
+__device__ __forceinline__ bool bin_rank_desc(const uint64_t (&v)[E], int cnt, int limit, uint64_t *scratch,
                                               RangeShared &sh, int nlim, Put put) {
   static_assert(kBins == 2 * kFinThreads, "two bins per thread");
+  constexpr uint32_t kCrowd = E > 4 ? 192 : 48;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = kFinThreads >> 6;
   uint64_t *placed = scratch;                                           // [E * 1024] values in bin order
   uint32_t *hist = reinterpret_cast<uint32_t *>(scratch + E * 1024);    // [2048] values per bin
@@ -296,11 +299,12 @@ __device__ __forceinline__ void bin_rank_desc(const uint64_t (&v)[E], int cnt, i
   above[kBins - 2 - 2 * t] = ab + c0;
   __syncthreads();
   if (sh.fcnt) {  // uniform
+    if constexpr (LINEAR) return false;
     __syncthreads();  // scratch is rewritten
     block_rank_desc<E>(v, scratch, scratch + nlim, nlim, [&](int rank, uint64_t x) {
       if (rank < cnt) put(rank, x);
     });
-    return;
+    return true;
   }
 #pragma unroll
   for (int e = 0; e < E; ++e)
@@ -314,6 +318,7 @@ __device__ __forceinline__ void bin_rank_desc(const uint64_t (&v)[E], int cnt, i
       for (uint32_t j = 0; j < n; ++j) rank += placed[base + j] > v[e] ? 1u : 0u;
       put((int)rank, v[e]);
     }
+  return true;
 }
 
 // Value sources of the selections.  for_each(f) calls f(ok, v) for every value
@@ -332,24 +337,6 @@ struct ArraySrc {  // values p[0, cnt) (LDS or global memory)
     }
   }
 };
-
-template <typename Get>
-struct IndexSrc {  // values get(0), ..., get(cnt - 1)
-  Get get;
-  int64_t cnt;
-  template <typename F>
-  __device__ __forceinline__ void for_each(F f) const {
-    for (int64_t i0 = 0; i0 < cnt; i0 += blockDim.x) {
-      const int64_t i = i0 + threadIdx.x;
-      const bool ok = i < cnt;
-      f(ok, ok ? get(i) : 0ull);
-    }
-  }
-};
-template <typename Get>
-__device__ __forceinline__ IndexSrc<Get> index_src(Get get, int64_t cnt) {
-  return IndexSrc<Get>{get, cnt};
-}
 
 // A row's candidates in the region layout: region r holds rc[r] values at
 // cand[r * kRegTok, ...).  Each wave takes batches of 64 regions (the next
@@ -889,7 +876,8 @@ __global__ __launch_bounds__(kFinThreads) void finalize_fused_kernel(int64_t m, 
     select_sorted(ArraySrc{cl, (int64_t)cnt}, cnt, kk, m, sink, local, out, cl, ss, sh, s_cnt, false);
   } else {
     select_sorted(src, cnt, kk, m, sink, local, out, cl, ss, sh, s_cnt, false);
-  }  if constexpr (ATTN) row_attention(ra, out, k, in_lds, ranked, cl);
+  }
+  if constexpr (ATTN) row_attention(ra, out, k, in_lds, ranked, cl);
 }
 
 // Wave-wide minimum and maximum of 32-bit values (in every lane): DPP row
@@ -1271,7 +1259,11 @@ __device__ __forceinline__ void rank_cands(uint64_t *cl, uint32_t cnt, RowOut &o
       v[e] = i < cnt ? cl[i] : 0ull;
     }
     __syncthreads();
-    bin_rank_desc<E, LINEAR>(v, (int)cnt, out.got, cl, sh, nlim, [&](int rank, uint64_t x) { out.put(rank, x); });
+    const auto put = [&](int rank, uint64_t x) { out.put(rank, x); };
+    if (!bin_rank_desc<E, LINEAR>(v, (int)cnt, out.got, cl, sh, nlim, put)) {
+      __syncthreads();  // scratch is rewritten
+      bin_rank_desc<E>(v, (int)cnt, out.got, cl, sh, nlim, put);
+    }
   };
   if (WIDE && cnt > (uint32_t)(4 * kFinThreads)) rank_all(std::integral_constant<int, 8>{});
   else if (!WIDE && cnt <= (uint32_t)(2 * kFinThreads)) rank_all(std::integral_constant<int, 2>{});
@@ -1346,68 +1338,187 @@ __device__ __forceinline__ uint32_t place_from_bin(const uint32_t (&key)[E], uin
   return cnt;
 }
 
-// Top kk of cnt distinct values of src where more than one sort takes reach the
-// bound (ties, clustered rows).  kk up to kMaxK by select_sorted; WIDE: up to 8192,
-// from the values in cl (src is cl then) those of the bin that holds the kk-th and
-// above, else the exact kk largest by range selection, gathered in cl, then one
-// sort.  False: the tokens are not in out.ranked.
+// Value sources of the narrowed selection: for_each(f) calls f(ok, key, token) for
+// every value, in loops that are uniform per wave.
+// Keys held in registers, thread t those of tokens t + 1024 e (0: none).
+template <int E>
+struct RegSrc {
+  const uint32_t (&key)[E];
+  template <typename F>
+  __device__ __forceinline__ void for_each(F f) const {
+#pragma unroll
+    for (int e = 0; e < E; ++e) f(key[e] != 0u, key[e], threadIdx.x + (uint32_t)e * kFinThreads);
+  }
+};
+// The unmasked tokens [sink, sink + len) of a row of n.
+struct Unmasked {
+  uint32_t sink, len;
+  __device__ __forceinline__ Unmasked(int64_t n, int64_t s, int64_t lstart)
+      : sink((uint32_t)min(s, n)), len((uint32_t)max(min(lstart, n) - min(s, n), (int64_t)0)) {}
+  __device__ __forceinline__ uint32_t key(float v, uint32_t tok) const {
+    return tok - sink < len ? score_key(v) : kKeyNegInf;
+  }
+};
+// A row's scores, read anew on each pass.
+template <typename Scores>
+struct RowSrc {
+  const Scores &rs;
+  uint32_t n;
+  Unmasked um;
+  template <typename F>
+  __device__ __forceinline__ void for_each(F f) const {
+    constexpr int kU = 8;
+    const uint32_t lane = threadIdx.x & 63;
+    for (uint32_t w0 = threadIdx.x - lane; w0 < n; w0 += kU * kFinThreads) {  // uniform per wave
+      float v[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const uint32_t i = w0 + lane + u * kFinThreads;
+        v[u] = i < n ? rs[i] : 0.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const uint32_t i = w0 + lane + u * kFinThreads;
+        f(i < n, um.key(v[u], i), i);
+      }
+    }
+  }
+};
+// The listed groups of a row: a wave takes 64 of them, 16 lanes each.
+template <typename Scores>
+struct GroupSrc {
+  const Scores &rs;
+  const uint16_t *list;
+  uint32_t ngr, n;
+  Unmasked um;
+  template <typename F>
+  __device__ __forceinline__ void for_each(F f) const {
+    constexpr int kU = 8;
+    const uint32_t lane = threadIdx.x & 63;
+    for (uint32_t e0 = threadIdx.x - lane; e0 < ngr; e0 += kFinThreads) {  // uniform per wave
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        uint32_t tok[kU];
+        float v[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          const uint32_t e = e0 + (uint32_t)(4 * (kU * h + u)) + lane / kGroupTok;
+          tok[u] = e < ngr ? (uint32_t)list[e] * (uint32_t)kGroupTok + lane % kGroupTok : n;
+          v[u] = tok[u] < n ? rs[tok[u]] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) f(tok[u] < n, um.key(v[u], tok[u]), tok[u]);
+      }
+    }
+  }
+};
+
+// A value into a bin of sh.hist: the lanes of a wave that share the first one's
+// bin are added at once (equal scores would serialise on one LDS counter).
+__device__ __forceinline__ void count_bin(bool in, uint32_t b, RangeShared &sh) {
+  const uint64_t m = __ballot(in);
+  if (m == 0ull) return;  // uniform per wave
+  const int first = __ffsll((unsigned long long)m) - 1;
+  const uint32_t b0 = (uint32_t)__builtin_amdgcn_readlane((int)b, first);
+  const uint32_t same = (uint32_t)__popcll(__ballot(in && b == b0));
+  const bool lead = (threadIdx.x & 63) == (uint32_t)first;
+  if (in && (lead || b != b0)) atomicAdd(&sh.hist[b], lead ? same : 1u);
+}
+
+// Where more of src's values with keys in [klo, khi] reach the first bound than one
+// sort takes (ties, groups that hold several top keys): the top kk of them (at least
+// kk, none of a higher key).  Each round counts the range in 2048 bins and keeps the
+// bin that holds the kk-th: of keys, then, once the range is one key, of its tokens;
+// as soon as at most cap >= kk values lie in that bin and above they are gathered in
+// cl (which src does not read below cap) and sorted.  One workgroup works its way
+// through the values at about 25 instructions each and pass, so there are as few
+// passes as can be: two for a row of equal scores.
 template <bool WIDE, typename Src>
-__device__ __forceinline__ bool select_cands(const Src &src, int64_t cnt, RowOut &out, uint64_t *cl, uint64_t *ss,
-                                             RangeShared &sh, uint32_t &s_cnt, bool in_lds) {
-  if constexpr (!WIDE) {
-    select_sorted(src, cnt, out.kk, out.m, out.sink, out.local, out.p, cl, ss, sh, s_cnt, !in_lds);
-    return false;
-  } else {
-    constexpr int kHold = kCandLds / kFinThreads;
-    static_assert(kHold * kFinThreads == kCandLds && 8 * kFinThreads + kBins <= kCandLds, "cl held in registers");
-    const int lane = threadIdx.x & 63;
-    uint64_t v[kHold];
-    if (in_lds) {  // uniform
-      uint32_t key[kHold], lo, hi, off;
-#pragma unroll
-      for (int e = 0; e < kHold; ++e) {
-        const int64_t i = threadIdx.x + (int64_t)e * kFinThreads;
-        v[e] = i < cnt ? cl[i] : 0ull;
-        key[e] = (uint32_t)(v[e] >> 32);
-      }
-      key_range<kHold>(key, lo, hi, sh);
-      const KeyBins bins(lo, hi);
-      const uint32_t b = rank_bin<kHold>(key, (uint32_t)out.kk, bins, sh);
-      const uint32_t kept = place_from_bin<kHold>(key, b, bins, off, sh);
-      if (kept <= 8u * kFinThreads) {  // uniform; every thread has read cl
-#pragma unroll
-        for (int e = 0; e < kHold; ++e)
-          if (key[e] && bins.of(key[e]) >= b) cl[off++] = v[e];
-        __syncthreads();
-        rank_cands<false, true>(cl, kept, out, sh);
-        return out.finish();
-      }
-      __syncthreads();
+__device__ __forceinline__ bool select_narrowed(const Src &src, uint32_t klo, uint32_t khi, int64_t n, uint32_t cap,
+                                                RowOut &out, uint64_t *cl, RangeShared &sh, uint32_t &s_cnt) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t kk = (uint32_t)out.kk;
+  uint32_t above = 0u, tlo = 0u, thi = (uint32_t)(n - 1);  // values above the range; tokens of a range of one key
+  for (;;) {  // uniform; a round takes 11 bits off the range or ends on one key
+    const bool one = klo == khi;
+    const uint32_t R = one ? thi - tlo : khi - klo;
+    const int bl = R ? 32 - __clz((int)R) : 0, s = bl > 11 ? bl - 11 : 0;
+    __syncthreads();  // hist, hsel and hcnt are read
+    sh.hist[tid] = sh.hist[tid + kFinThreads] = 0u;
+    if (tid == 0) sh.hsel = sh.hcnt = sh.need = 0u;
+    __syncthreads();
+    if (one) src.for_each([&](bool ok, uint32_t key, uint32_t tok) {
+      count_bin(ok && key == klo && tok - tlo <= R, kBins - 1 - ((tok - tlo) >> s), sh);
+    });
+    else src.for_each([&](bool ok, uint32_t key, uint32_t) { count_bin(ok && key - klo <= R, (key - klo) >> s, sh); });
+    __syncthreads();
+    // running counts from the top bin down: thread t holds bins 2047 - 2t, 2046 - 2t
+    const uint32_t c0 = sh.hist[kBins - 1 - 2 * tid], c1 = sh.hist[kBins - 2 - 2 * tid], c = c0 + c1;
+    const uint32_t wi = wave_incl_scan_u32(c);
+    if (lane == kWave - 1) sh.wsum[wave] = wi;
+    __syncthreads();
+    uint32_t ab = above + wi - c;
+    for (int w = 0; w < wave; ++w) ab += sh.wsum[w];
+    if (ab < kk && ab + c0 >= kk) {
+      sh.hsel = (uint32_t)(kBins - 1 - 2 * tid);
+      sh.need = ab;
+      sh.hcnt = ab + c0;
+    } else if (ab + c0 < kk && ab + c >= kk) {
+      sh.hsel = (uint32_t)(kBins - 2 - 2 * tid);
+      sh.need = ab + c0;
+      sh.hcnt = ab + c;
     }
-    const uint64_t thr = range_select(src, cnt, (uint32_t)out.kk, sh);
     __syncthreads();
-    if (threadIdx.x == 0) s_cnt = 0u;
-    __syncthreads();
-    if (in_lds) {  // the survivors take the candidates' place
-#pragma unroll
-      for (int e = 0; e < kHold; ++e) lds_append(v[e] >= thr && v[e] != 0ull, v[e], &s_cnt, cl, 8u * kFinThreads, lane);
+    const uint32_t width = (1u << s) - 1u;
+    if (one) {
+      tlo += (uint32_t)(kBins - 1 - sh.hsel) << s;
+      thi = min(thi, tlo + width);
     } else {
-      src.for_each([&](bool ok, uint64_t v) { lds_append(ok && v >= thr, v, &s_cnt, cl, 8u * kFinThreads, lane); });
+      klo += sh.hsel << s;
+      khi = khi - klo > width ? klo + width : khi;
     }
-    __syncthreads();
-    rank_cands<false, true>(cl, min(s_cnt, 8u * kFinThreads), out, sh);
-    return out.finish();
+    if (sh.hcnt <= cap || (one && s == 0)) break;
+    above = sh.need;
+  }
+  if (tid == 0) s_cnt = 0u;
+  __syncthreads();
+  src.for_each([&](bool ok, uint32_t key, uint32_t tok) {
+    lds_append(ok && (key > klo || (key == klo && tok <= thi)), k64_of(key, tok), &s_cnt, cl, cap, lane);
+  });
+  __syncthreads();
+  rank_cands<false, WIDE>(cl, min(s_cnt, cap), out, sh);
+  return out.finish();
+}
+// The range of src's keys.
+template <typename Src>
+__device__ __forceinline__ void key_span(const Src &src, uint32_t &mn, uint32_t &mx, RangeShared &sh) {
+  mn = ~0u;
+  mx = 0u;
+  src.for_each([&](bool ok, uint32_t key, uint32_t) {
+    mn = ok ? min(mn, key) : mn;
+    mx = ok ? max(mx, key) : mx;
+  });
+  wave_minmax_u32(mn, mx);
+  __syncthreads();  // wmin and wmax are read
+  if ((threadIdx.x & 63) == 0) {
+    sh.wmin[threadIdx.x >> 6] = mn;
+    sh.wmax[threadIdx.x >> 6] = mx;
+  }
+  __syncthreads();
+  for (int w = 0; w < kFinThreads / kWave; ++w) {
+    mn = min(mn, (uint32_t)sh.wmin[w]);
+    mx = max(mx, (uint32_t)sh.wmax[w]);
   }
 }
 
 // Exact top kk of a short row, read whole: up to 4096 tokens are ranked at once
 // (E values per thread); longer rows first keep the scores of the bin that
 // holds the kk-th largest and above, 2048 linear bins over the finite scores'
-// range (kk and a few of them for spread scores; rows whose kept scores
-// outgrow the sort are selected by range).
+// range (kk and a few of them for spread scores; where they outgrow the sort, or the
+// bins of a row of up to 4096 crowd, the bound is narrowed).
 template <int E, bool WIDE, typename Scores>
-__device__ __forceinline__ bool rowrank_row(const Scores &rs, int64_t n, RowOut &out, uint64_t *cl, uint64_t *ss,
-                                            RangeShared &sh, uint32_t &s_cnt) {
+__device__ __forceinline__ bool rowrank_row(const Scores &rs, int64_t n, RowOut &out, uint64_t *cl, RangeShared &sh,
+                                            uint32_t &s_cnt) {
   const int tid = threadIdx.x;
   const int64_t kk = out.kk, sink = out.sink;
   const int64_t lstart = (out.m - out.local) > 0 ? (out.m - out.local) : 0;
@@ -1425,7 +1536,13 @@ __device__ __forceinline__ bool rowrank_row(const Scores &rs, int64_t n, RowOut 
     int nlim = kWave;
     while (nlim < (int)n) nlim <<= 1;
     out.got = (int)kk;
-    bin_rank_desc<E, true>(v, (int)n, out.got, cl, sh, nlim, [&](int rank, uint64_t x) { out.put(rank, x); });
+    if (!bin_rank_desc<E, true>(v, (int)n, out.got, cl, sh, nlim, [&](int rank, uint64_t x) { out.put(rank, x); })) {
+      uint32_t cap = kFinThreads / 2;  // many equal scores: the fewer are sorted the better
+      while (cap < (uint32_t)kk) cap <<= 1;
+      uint32_t klo, khi;
+      key_span(RegSrc<E>{key}, klo, khi, sh);
+      return select_narrowed<false>(RegSrc<E>{key}, klo, khi, n, cap, out, cl, sh, s_cnt);
+    }
     return out.finish();
   }
   uint32_t lo, hi;
@@ -1434,9 +1551,12 @@ __device__ __forceinline__ bool rowrank_row(const Scores &rs, int64_t n, RowOut 
   const uint32_t b = rank_bin<E>(key, (uint32_t)kk, bins, sh);  // n >= kk keys are counted
   uint32_t off;
   const uint32_t cnt = place_from_bin<E>(key, b, bins, off, sh);
-  if (cnt > (uint32_t)((WIDE ? 8 : 4) * kFinThreads)) {  // uniform: ties, or a range that outliers stretch
-    const auto src = index_src([&](int64_t i) { return k64_of(masked_key(rs, i, sink, lstart), i); }, n);
-    return select_cands<WIDE>(src, n, out, cl, ss, sh, s_cnt, false);
+  constexpr uint32_t kSort = (WIDE ? 8 : 4) * kFinThreads;
+  if (cnt > kSort) {  // uniform: ties, or a range that outliers stretch
+    const RowSrc<Scores> src{rs, (uint32_t)n, Unmasked(n, sink, lstart)};
+    uint32_t klo, khi;
+    key_span(src, klo, khi, sh);
+    return select_narrowed<WIDE>(src, klo, khi, n, kSort, out, cl, sh, s_cnt);
   }
 #pragma unroll
   for (int e = 0; e < E; ++e)
@@ -1463,19 +1583,72 @@ inline bool rowrank_takes(int64_t n, int64_t kk) {
 // row's kk-th largest key from below (kk groups each hold a key >= T), and
 // every key >= T lies in a group whose maximum is >= T: only those groups'
 // scores are read, and their keys >= T are the candidates (a little over kk
-// for spread scores).  Up to 2048 candidates are ranked by one sort; more are
-// selected first; rows whose candidates outgrow the LDS list (ties around T)
-// are selected from the whole row.
-constexpr int kGroupList = (int)(sizeof(uint64_t) * kMaxK / sizeof(uint16_t));  // listed groups (in ss)
-static_assert(kGmaxSelectMax / kGroupTok <= 65536, "group numbers fit 16 bits");
-// ranked (LDS of k int32, past the sort's scratch in cl; null: none): rows of
-// at most 2048 candidates also leave their k output tokens there, and the
-// call returns true.
+// for spread scores).  Up to 4096 (WIDE: 8192) candidates are ranked by one sort;
+// more are first cut to those of the key bin that holds the kk-th and above.  Where
+// neighbouring tokens score alike a group holds several top keys and T falls, to
+// 16 kk candidates at worst, and ties reach T in any number: more than the LDS list
+// holds narrow T over the listed groups, a few passes over them; where no key is
+// past T, the first kk tokens of that key are the answer.  sink_local_topk of 32
+// rows, us, with the whole row selected in those cases and now: scores of
+// correlation length 64 tokens, n = 131072, k = 2048 191; 51, 300007, 4096 734; 90, all
+// equal, 131072, 512 489; 24.  Scan + top-k of 8 x 4 heads of 131072 with one query
+// row of zeros, k = 512: 485; 33.
+constexpr int kGroupList = (int)(sizeof(uint64_t) * kMaxK / sizeof(uint16_t));  // groups listed in ss
+constexpr int kGroupListAll = kCandLds / 2 * (int)(sizeof(uint64_t) / sizeof(uint16_t));  // in cl's upper half
+static_assert(kGmaxSelectMax / kGroupTok <= kGroupList && kGmaxWideMax / kGroupTok <= kGroupListAll &&
+                  kGmaxWideMax / kGroupTok <= 65536,
+              "every group can be listed, in 16 bits");
+// The top kk of a row whose largest key is T and whose groups reach it at least kk
+// times: the first kk tokens of that key, from the row's start on until they are found.
+template <typename Scores>
+__device__ __forceinline__ bool take_first(const Scores &rs, const uint32_t *__restrict__ gm, uint32_t n, const Unmasked &um,
+                                           uint32_t T, RowOut &out, RangeShared &sh) {
+  constexpr int kU = 16;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = kFinThreads >> 6;
+  const uint32_t kk = (uint32_t)out.kk, ngrp = (uint32_t)cdiv(n, kGroupTok);
+  out.got = (int)kk;
+  uint32_t got = 0u;
+  for (uint32_t c0 = 0; c0 < n && got < kk; c0 += kU * kFinThreads) {  // uniform
+    const uint32_t w0 = c0 + (uint32_t)wave * (kU * kWave), g = w0 / kGroupTok + lane;
+    uint64_t m[kU] = {};
+    uint32_t hits = 0u;
+    if (__ballot(g < ngrp && gm[min(g, ngrp - 1u)] >= T) != 0ull) {  // uniform per wave
+      float v[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) v[u] = w0 + u * kWave + lane < n ? rs[w0 + u * kWave + lane] : 0.0f;
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const uint32_t tok = w0 + u * kWave + lane;
+        m[u] = __ballot(tok < n && um.key(v[u], tok) == T);
+        hits += (uint32_t)__popcll(m[u]);
+      }
+    }
+    if (lane == 0) sh.wsum[wave] = hits;
+    __syncthreads();
+    uint32_t off = got;
+    for (int w = 0; w < nw; ++w) {
+      const uint32_t ws = sh.wsum[w];
+      off += w < wave ? ws : 0u;
+      got += ws;
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const uint32_t tok = w0 + u * kWave + lane;
+      if ((m[u] >> lane) & 1ull) out.put((int)min(off + (uint32_t)__popcll(m[u] & ((1ull << lane) - 1ull)), kk), k64_of(T, tok));
+      off += (uint32_t)__popcll(m[u]);
+    }
+    __syncthreads();  // sh.wsum is rewritten
+  }
+  out.got = (int)min(got, kk);
+  return out.finish();
+}
+
+// The row's k output tokens are left in out.ranked too, where it is given.
 template <int kPer, bool WIDE, typename Scores>
 __device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint32_t *__restrict__ gmax, int64_t n,
                                                    RowOut &out, uint64_t *cl, uint64_t *ss, RangeShared &sh,
                                                    uint32_t &s_cnt) {
-  uint16_t *glist = reinterpret_cast<uint16_t *>(ss);  // ss holds the survivors only after the groups are read
+  uint16_t *glist = reinterpret_cast<uint16_t *>(ss), *glist_all = reinterpret_cast<uint16_t *>(cl + kCandLds / 2);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = kFinThreads >> 6;
   const int64_t row = blockIdx.x;
   const int64_t kk = out.kk, sink = out.sink;
@@ -1488,7 +1661,7 @@ __device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint3
     gm[u] = g < ngrp ? gmax[row * ngrp + g] : 0u;
   }
   const uint32_t T = ngrp > kk ? kth_bound<kPer>(gm, ngrp, (uint32_t)kk, sh) : 0u;
-  // the groups reaching T, listed in order
+  // the groups reaching T, listed by thread (groups tid + 1024 u)
   uint32_t ngr = 0u;
   {
     uint32_t c = 0u;
@@ -1503,24 +1676,24 @@ __device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint3
       off += w < wave ? ws : 0u;
       ngr += ws;
     }
+    uint16_t *list = WIDE && ngr > (uint32_t)kGroupList ? glist_all : glist;  // uniform
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
       const int g = tid + u * kFinThreads;
-      if (g < ngrp && gm[u] >= T) {
-        if (off < (uint32_t)kGroupList) glist[off] = (uint16_t)g;
-        ++off;
-      }
+      if (g < ngrp && gm[u] >= T) list[off++] = (uint16_t)g;
     }
     __syncthreads();
   }
-  if (ngr > (uint32_t)kGroupList) {  // uniform: ties around T
-    const auto src = index_src([&](int64_t i) { return k64_of(masked_key(rs, i, sink, lstart), i); }, n);
-    return select_cands<WIDE>(src, n, out, cl, ss, sh, s_cnt, false);
-  }
+  constexpr uint32_t kSort = (WIDE ? 8 : 4) * kFinThreads;
+  static_assert(kSort <= kCandLds / 2 && kSort <= kGroupList, "gathered below the list in cl");
+  static_assert(((int64_t)kCandLds + kGroupTok * 2 * kFinThreads) * kGroupListAll < ((int64_t)1 << 32) &&
+                    (int64_t)kCandLds * (kGroupList + 2 * kFinThreads) < ((int64_t)1 << 32),
+                "the estimate of the candidates in 32 bits");
   // their keys >= T, kU groups per thread and round, placed by a workgroup prefix sum
   constexpr int kU = WIDE ? 2 : 1;
-  uint32_t cnt = 0u;
-  for (uint32_t e0 = 0; e0 < ngr; e0 += kU * kFinThreads) {  // uniform
+  uint32_t cnt = ngr <= kSort ? 0u : kCandLds + 1;  // each group has one: more groups than the sort takes are narrowed
+  uint32_t e0 = 0;  // read on while the candidates seem to fit (a thread's groups lie 1024 apart: a round is a fair sample)
+  for (; e0 < ngr && cnt * ngr <= (uint32_t)kCandLds * e0; e0 += kU * kFinThreads) {  // uniform
     int64_t t0[kU];
     float v[kU][kGroupTok] = {};
 #pragma unroll
@@ -1560,12 +1733,42 @@ __device__ __forceinline__ bool rowselect_gmax_row(const Scores &rs, const uint3
       }
     __syncthreads();  // sh.wsum is rewritten by the next step
   }
-  if (cnt > (uint32_t)kCandLds) {  // uniform: ties around T
-    const auto src = index_src([&](int64_t i) { return k64_of(masked_key(rs, i, sink, lstart), i); }, n);
-    return select_cands<WIDE>(src, n, out, cl, ss, sh, s_cnt, false);
+  if (e0 < ngr) cnt = kCandLds + 1;
+  if (cnt > kSort && cnt <= (uint32_t)kCandLds) {  // uniform: the candidates in registers, cut by key bins
+    constexpr int kHold = kCandLds / kFinThreads;
+    static_assert(kHold * kFinThreads == kCandLds, "cl held in registers");
+    uint64_t v[kHold];
+    uint32_t key[kHold], lo, hi, off;
+#pragma unroll
+    for (int e = 0; e < kHold; ++e) {
+      const uint32_t i = tid + (uint32_t)e * kFinThreads;
+      v[e] = i < cnt ? cl[i] : 0ull;
+      key[e] = (uint32_t)(v[e] >> 32);
+    }
+    key_range<kHold>(key, lo, hi, sh);
+    const KeyBins bins(lo, hi);
+    const uint32_t b = rank_bin<kHold>(key, (uint32_t)kk, bins, sh);
+    const uint32_t kept = place_from_bin<kHold>(key, b, bins, off, sh);
+    cnt = kept <= kSort ? kept : kCandLds + 1;
+    if (kept <= kSort) {  // uniform; every thread has read cl
+#pragma unroll
+      for (int e = 0; e < kHold; ++e)
+        if (key[e] && bins.of(key[e]) >= b) cl[off++] = v[e];
+    }
+    __syncthreads();
   }
-  if (cnt > (uint32_t)((WIDE ? 8 : 4) * kFinThreads))
-    return select_cands<WIDE>(ArraySrc{cl, (int64_t)cnt}, cnt, out, cl, ss, sh, s_cnt, true);
+  if (cnt > kSort) {  // uniform: keys from T to the largest group maximum
+    uint32_t bot = ~0u, top = 0u;
+    for (int g = tid; g < ngrp; g += kFinThreads) top = max(top, gmax[row * ngrp + g]);
+    wave_minmax_u32(bot, top);
+    if (lane == 0) sh.wmax[wave] = top;
+    __syncthreads();
+    for (int w = 0; w < nw; ++w) top = max(top, (uint32_t)sh.wmax[w]);
+    if (top == T) return take_first(rs, gmax + row * ngrp, (uint32_t)n, Unmasked(n, sink, lstart), T, out, sh);
+    const GroupSrc<Scores> src{rs, WIDE && ngr > (uint32_t)kGroupList ? glist_all : glist, ngr, (uint32_t)n,
+                               Unmasked(n, sink, lstart)};
+    return select_narrowed<WIDE>(src, T, top, n, kSort, out, cl, sh, s_cnt);
+  }
   rank_cands<false, WIDE>(cl, cnt, out, sh);  // one sort ranks them
   return out.finish();
 }
@@ -1590,7 +1793,7 @@ __global__ __launch_bounds__(kFinThreads) void rowselect_kernel(const float *__r
   RowOut ro{idx + blockIdx.x * k, k - sink - local, m, sink, local, ranked, 0};
   const Scores rs(scores, n, G);
   bool in_lds;
-  if constexpr (E > 0) in_lds = rowrank_row<E, WIDE>(rs, n, ro, cl, ss, sh, s_cnt);
+  if constexpr (E > 0) in_lds = rowrank_row<E, WIDE>(rs, n, ro, cl, sh, s_cnt);
   else in_lds = rowselect_gmax_row<kPer, WIDE>(rs, gmax, n, ro, cl, ss, sh, s_cnt);
   if constexpr (ATTN) row_attention(ra, idx + blockIdx.x * k, k, in_lds, ranked, cl);
 }

@@ -68,7 +68,10 @@ constexpr int64_t kGroupTok = 16;
 // selection against this one: n = 8192, k = 4096 107; 17.5, 30000, 4096 104; 29, 32768,
 // 8000 136; 37, 100000, 4096 82; 47, 300007, 4096 104; 71, 524288, 4096 91; 72; beyond
 // the limits 1048576, 4096 98; 97 and 300007, 8192 121; 116 (198 on rows whose list
-// does not fit).
+// does not fit).  Those are independent scores; neighbours that score alike (correlation
+// lengths of 16 and 256 tokens) cost both sides more: 100000, 4096 88; 74 and 126; 72,
+// 300007, 4096 99; 94 and 146; 87, 500000, 5000 96; 110 and 157; 102, 500000, 6136 102; 123
+// and 190; 116.
 inline bool group_select_takes(int64_t n, int64_t kk) {
   if (kk <= kSelMaxK) return n <= kGmaxSelectMax;
   if (n <= kRowSelectMax) return kk <= kRankListMax;

@@ -187,6 +187,48 @@ def test_wide_selection_at_every_route(n, k, extra):
         np.testing.assert_array_equal(got, O.sink_local_topk(s, k, 4, 32, m=n + extra), err_msg=kind)
 
 
+@pytest.mark.parametrize("n,k", [(900, 400), (4096, 512), (8192, 600), (30000, 2048), (32768, 512), (32769, 2084), (131072, 1000),
+                                 (131071, 2084), (8193, 4096), (32768, 8228), (131072, 4000), (131073, 2085), (300007, 4096),
+                                 (524288, 6136)])
+def test_more_candidates_than_one_sort_takes(n, k):
+    """Rows whose first bound leaves more scores than one sort (or the LDS list) takes: neighbouring tokens alike, two and
+    three levels of equal scores with the cut inside one, a ramp, and levels whose lowest group of tokens is the row's last."""
+    print(f"[narrowed] n={n} k={k}", flush=True)
+    rng = np.random.default_rng(n + k)
+    t = np.arange(n)
+    knots = -(-n // 256) + 2
+    smooth = np.stack([np.interp(t, np.arange(knots) * 256, rng.standard_normal(knots)) for _ in range(2)])
+    kk = k - 36
+    two = np.where(rng.random((2, n)) < 1.5 * kk / n, 2.0, 1.0)
+    three = np.where(rng.random((2, n)) < 0.3 * kk / n, 5.0, np.where(rng.random((2, n)) < 0.9, 1.0, -3.0))
+    tail = np.where(t >= n - n // 3, 1.0 + t % 7 * 1e-6, -1.0)[None].repeat(2, 0)
+    for s in (smooth + rng.standard_normal((2, n)) * 1e-4, two, three, t[None] * 1e-3 - 5.0, tail):
+        s = np.ascontiguousarray(s, dtype=np.float32)
+        got = bp.sink_local_topk(torch.from_numpy(s).to(DEV), k, 4, 32).cpu().numpy()
+        np.testing.assert_array_equal(got, O.sink_local_topk(s, k, 4, 32))
+
+
+@pytest.mark.parametrize("BH,G,n,k", [(2, 4, 4000, 512), (2, 4, 20000, 512), (2, 3, 131072, 512), (2, 7, 131071, 512),
+                                      (1, 7, 131072, 2048), (1, 4, 300007, 4096)])
+def test_fused_selection_of_clustered_and_equal_rows(BH, G, n, k):
+    """The same in the fused scan's score orders, and the attention over such rows."""
+    print(f"[narrowed fused] {BH}x{G} n={n} k={k}", flush=True)
+    gen = torch.Generator(DEV).manual_seed(n)
+    knots = -(-n // 300) + 1
+    K = torch.randn(BH, knots, 128, device=DEV, generator=gen).repeat_interleave(300, 1)[:, :n]
+    K = (K + 0.05 * torch.randn(BH, n, 128, device=DEV, generator=gen)).to(torch.bfloat16).contiguous()
+    q = torch.randn(BH, G, 128, device=DEV, generator=gen)
+    g = (q ** 2).sum(1)
+    q[-1, -1] = 0.0                               # every score of this head equal
+    st = bp.PlaneStore(K, keep_code=False)
+    plan = bp.make_plan(g, 48.0)
+    want = _oracle_topk(st.scan(q, plan), k, 4, 32, n)
+    assert torch.equal(st.scan_topk(q, plan, k, 4, 32).cpu(), want)
+    idx, out = st.plan_scan_topk_attention(q, g, 48.0, k, K, K, 4, 32)
+    ref, _ = off.gather_attention(q, idx, n, K, K, n)
+    assert torch.equal(idx.cpu(), want) and torch.equal(out, ref)
+
+
 @pytest.mark.parametrize("BH,G,n,k", [(2, 5, 200001, 4096), (1, 4, 40000, 3000), (1, 8, 9000, 8228), (1, 4, 600000, 5000)])
 def test_wide_fused_selection(BH, G, n, k):
     print(f"[wide-select fused] {BH}x{G} n={n} k={k}", flush=True)
