@@ -67,50 +67,55 @@ __global__ __launch_bounds__(kKltThreads) void klt_query_kernel(const float *__r
 
 // float(K) - mu of key rows [BH, n, D], the store build's input to the rotation: one
 // pass where a conversion and a subtraction took two (a conversion's float32 copy
-// written and read again).  V elements per thread.  Bound: HBM, 6 bytes per 16-bit
-// key: 8 x 20011 f16 keys 48 -> 22 us.
+// written and read again).  V elements per thread and step: 8 16-bit or 4 32-bit keys
+// (16-byte loads and stores), 1 where a pointer or D is not aligned to that.  Bound:
+// HBM, 6 bytes per 16-bit key, 8 per 32-bit one: 8 x 20011 f16 keys 47 -> 20.4 us; 8 x
+// 131072 f32 keys 174 us (329 an element at a time, 177 torch's subtraction).
 template <int KDT, int V>
 __global__ __launch_bounds__(256) void klt_center_kernel(const void *__restrict__ K, const float *__restrict__ mu, int64_t n,
                                                          int64_t D, float *__restrict__ out) {
-  const int64_t bh = blockIdx.y, per = n * D;
-  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V; i < per; i += (int64_t)gridDim.x * 256 * V) {
-    float x[V];
-    if constexpr (V == 8) {
-      const uint4 r = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(K) + bh * per + i);
-      const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+  const int64_t bh = blockIdx.y, per = n * D, step = (int64_t)gridDim.x * 256 * V;
+  int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
+  int64_t j = i % D;  // V divides D
+  const int64_t jstep = step % D;
+  const float *m = mu + bh * D;
+  float *o = out + bh * per;
+  for (; i < per; i += step) {
+    if constexpr (V == 1) {
+      o[i] = load_elem<KDT>(K, bh * per + i) - m[j];
+    } else {
+      float x[V];
+      if constexpr (KDT == FATHOM_DT_F32) {
+        const float4 r = *reinterpret_cast<const float4 *>(static_cast<const float *>(K) + bh * per + i);
+        x[0] = r.x, x[1] = r.y, x[2] = r.z, x[3] = r.w;
+      } else {
+        const uint4 r = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(K) + bh * per + i);
+        const uint32_t w[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
-      for (int e = 0; e < V; ++e) {
-        const uint16_t h = (uint16_t)(e & 1 ? w[e / 2] >> 16 : w[e / 2]);
-        x[e] = KDT == FATHOM_DT_BF16 ? bf16_bits_to_float(h) : f16_bits_to_float(h);
+        for (int e = 0; e < V; ++e) {
+          const uint16_t h = (uint16_t)(e & 1 ? w[e / 2] >> 16 : w[e / 2]);
+          x[e] = KDT == FATHOM_DT_BF16 ? bf16_bits_to_float(h) : f16_bits_to_float(h);
+        }
       }
-    } else {
-      x[0] = load_elem<KDT>(K, bh * per + i);
+#pragma unroll
+      for (int e = 0; e < V; e += 4) {
+        const float4 a = *reinterpret_cast<const float4 *>(m + j + e);
+        *reinterpret_cast<float4 *>(o + i + e) = make_float4(x[e] - a.x, x[e + 1] - a.y, x[e + 2] - a.z, x[e + 3] - a.w);
+      }
     }
-    const int64_t j = i % D;  // V divides D
-    float *o = out + bh * per + i;
-    const float *m = mu + bh * D + j;
-    if constexpr (V == 8) {
-      const float4 a = *reinterpret_cast<const float4 *>(m), b = *reinterpret_cast<const float4 *>(m + 4);
-      *reinterpret_cast<float4 *>(o) = make_float4(x[0] - a.x, x[1] - a.y, x[2] - a.z, x[3] - a.w);
-      *reinterpret_cast<float4 *>(o + 4) = make_float4(x[4] - b.x, x[5] - b.y, x[6] - b.z, x[7] - b.w);
-    } else {
-      o[0] = x[0] - m[0];
-    }
+    j += jstep;
+    if (j >= D) j -= D;
   }
 }
 
 template <int KDT>
 void launch_center(const void *K, const float *mu, int64_t BH, int64_t n, int64_t D, float *out, hipStream_t st) {
-  const bool vec = KDT != FATHOM_DT_F32 && D % 8 == 0 &&
+  constexpr int V = KDT == FATHOM_DT_F32 ? 4 : 8;
+  const bool vec = D % V == 0 &&
                    ((reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(mu) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-  const dim3 grid((unsigned)min(cdiv(n * D, vec ? 256 * 8 : 256), (int64_t)65535), (unsigned)BH);
-  if constexpr (KDT != FATHOM_DT_F32) {
-    if (vec) {
-      klt_center_kernel<KDT, 8><<<grid, 256, 0, st>>>(K, mu, n, D, out);
-      return;
-    }
-  }
-  klt_center_kernel<KDT, 1><<<grid, 256, 0, st>>>(K, mu, n, D, out);
+  const dim3 grid((unsigned)min(cdiv(n * D, vec ? 256 * V : 256), (int64_t)65535), (unsigned)BH);
+  if (vec) klt_center_kernel<KDT, V><<<grid, 256, 0, st>>>(K, mu, n, D, out);
+  else klt_center_kernel<KDT, 1><<<grid, 256, 0, st>>>(K, mu, n, D, out);
 }
 
 }  // namespace

@@ -75,3 +75,15 @@ def test_klt_centering_equals_torch(BH, n, cut, dtype):
     mu = torch.randn(BH, 128, generator=torch.Generator().manual_seed(1)).to(DEV)
     assert torch.equal(_centered(K, mu), K.float() - mu[:, None, :])
     assert torch.equal(_centered(K.transpose(0, 1).contiguous().transpose(0, 1), mu), K.float() - mu[:, None, :])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,D", [(33, 1), (1001, 12), (180000, 100), (700001, 24), (560000, 128)])
+def test_klt_centering_of_other_widths(n, D, dtype):
+    """Widths that the vector forms take for some key types only, and rows longer than one step of the grid."""
+    from fathom_amd.klt import _centered
+    print(f"[klt center] n={n} D={D} {dtype}", flush=True)
+    g = torch.Generator(DEV).manual_seed(D)
+    K = torch.randn(2, n, D, device=DEV, generator=g).to(dtype)
+    mu = torch.randn(2, D, device=DEV, generator=g)
+    assert torch.equal(_centered(K, mu), K.float() - mu[:, None, :])
