@@ -651,7 +651,7 @@ __global__ __launch_bounds__(kFilterThreads) void filter_scores_kernel(const flo
   for (int64_t start = (int64_t)blockIdx.x * steps * kFilterStep; start < end; start += kFilterStep) {  // uniform
     const auto at = [&](int u) { return start + (VEC ? 4 * (tid + kFilterThreads * (u >> 2)) + (u & 3) : tid + kFilterThreads * u); };
     float v[kPer];
-  #pragma unroll
+#pragma unroll
     for (int u = 0; u < kPer; u += VEC ? 4 : 1) {
       const int64_t i = at(u);
       if constexpr (VEC) {  // n is a multiple of 4
@@ -665,7 +665,7 @@ __global__ __launch_bounds__(kFilterThreads) void filter_scores_kernel(const flo
         v[u] = i < n ? rs[i] : 0.0f;
       }
     }
-  #pragma unroll
+#pragma unroll
     for (int u = 0; u < kPer; ++u) {
       const int64_t i = at(u);
       const bool in = i < n;
@@ -1919,11 +1919,12 @@ int launch_sample_scores(const float *scores, int64_t rows, int64_t n, int64_t S
   return launch_status("sample_scores_kernel");
 }
 
-// One step of 4096 scores per workgroup, four where the launch is large anyway
-// (fewer counter atomics per row).  sink_local_topk, k = 512, us, before (16384 scores
-// per workgroup, a load per step) and now: 32 rows of 200001 tokens 54.6; 34.5, 4 rows
-// 43.3; 29.2, 32 of 300007 56.2; 38.2, 4 of 1048576 38.4; 30.7, 32 of 1048576 48.5; ZZ (54.6
-// in single steps).
+// One step of 4096 scores per workgroup (16 loads of a thread in flight); launches of
+// 2^24 scores and more take 16 steps of 1024 (4 loads in flight, a quarter of the
+// counter atomics).  sink_local_topk, k = 512, us, 16384 scores per workgroup with a
+// load per step, and now: 32 rows of 200001 tokens 55.2; 37.7, 4 of 140000 40.6; 31.5, 32
+// of 300007 57.8; 40.4, 16 of 1048577 56.3; 43.9, 32 of 1048576 49.9; 49.9 (54.6 in single
+// steps of 4096).
 int launch_filter_scores(const float *scores, int64_t rows, int64_t n, int64_t sink, int64_t lstart, TopkSel s,
                          bool fallback, hipStream_t st) {
   const bool large = rows * n >= (int64_t)1 << 24;
