@@ -75,12 +75,11 @@ template <int KDT, int V>
 __global__ __launch_bounds__(256) void klt_center_kernel(const void *__restrict__ K, const float *__restrict__ mu, int64_t n,
                                                          int64_t D, float *__restrict__ out) {
   const int64_t bh = blockIdx.y, per = n * D, step = (int64_t)gridDim.x * 256 * V;
-  int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
-  int64_t j = i % D;  // V divides D
-  const int64_t jstep = step % D;
+  const bool small = per <= 0xFFFFFFFFll;  // uniform: a 32-bit remainder
   const float *m = mu + bh * D;
   float *o = out + bh * per;
-  for (; i < per; i += step) {
+  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V; i < per; i += step) {
+    const int64_t j = small ? (int64_t)((uint32_t)i % (uint32_t)D) : i % D;  // V divides D
     if constexpr (V == 1) {
       o[i] = load_elem<KDT>(K, bh * per + i) - m[j];
     } else {
@@ -103,8 +102,6 @@ __global__ __launch_bounds__(256) void klt_center_kernel(const void *__restrict_
         *reinterpret_cast<float4 *>(o + i + e) = make_float4(x[e] - a.x, x[e + 1] - a.y, x[e + 2] - a.z, x[e + 3] - a.w);
       }
     }
-    j += jstep;
-    if (j >= D) j -= D;
   }
 }
 
