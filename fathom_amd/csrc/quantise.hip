@@ -433,7 +433,7 @@ int launch128(const QuantArgs &a, int64_t lead, hipStream_t st) {
     quantise_tile_kernel<KDT, CPL, 1><<<dim3((unsigned)cdiv(a.cover, 4), y), 512 / CPL, 0, st>>>(a);
   else if (blocks < 12288 || !a.code || KDT == FATHOM_DT_F32)
     quantise_tile_kernel<KDT, CPL, 2><<<dim3((unsigned)cdiv(a.cover, 8), y), 512 / CPL, 0, st>>>(a);
-  else
+  else if constexpr (KDT != FATHOM_DT_F32)
     quantise_tile_kernel<KDT, CPL, 4><<<dim3((unsigned)cdiv(a.cover, 16), y), 512 / CPL, 0, st>>>(a);
   return launch_status("quantise128");
 }

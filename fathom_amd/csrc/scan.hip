@@ -356,7 +356,7 @@ namespace {
 // make_plan's arrays of plan_scan_topk with nothing to select, past the scan's
 // workspace.
 size_t plan_arrays_ws(int64_t BH, int64_t D, int bmax) {
-  return ws_align((size_t)(BH * D)) + ws_align((size_t)(BH * D * bmax) * 4) + 2 * ws_align((size_t)BH * 4) +
+  return ws_align((size_t)(BH * D * bmax) * 4) + 2 * ws_align((size_t)BH * 4) +
          ws_align((size_t)(BH * D) * 4) + ws_align((size_t)(BH * bmax * D) * 4) + ws_align((size_t)(BH * bmax) * 4);
 }
 }  // namespace
@@ -366,7 +366,7 @@ extern "C" size_t fathom_plan_scan_topk_workspace_bytes(int64_t BH, int64_t G, i
                                                         int64_t sink, int64_t local) {
   const int64_t kk = k - sink - local;
   if (BH < 1 || G < 1 || D < 1 || bmax < 1 || n < 1 || kk < 0) return 0;
-  return scan_topk_ws(BH * G, n, k, kk) + plan_arrays_ws(BH, D, bmax);
+  return scan_topk_ws(BH * G, n, k, kk) + (kk == 0 ? plan_arrays_ws(BH, D, bmax) : 0);
 }
 
 namespace fathom {
@@ -392,7 +392,7 @@ int plan_scan_topk_run(const float *q, const float *g, const float *budget, floa
   if (kk == 0) {
     // only the fixed positions are written; the plan's depths where asked for
     if (t_out) {
-      char *p = static_cast<char *>(workspace) + sws + ws_align((size_t)(BH * D));
+      char *p = static_cast<char *>(workspace) + sws;
       int32_t *pairs = reinterpret_cast<int32_t *>(p);
       p += ws_align((size_t)(BH * D * bmax) * 4);
       int32_t *npairs = reinterpret_cast<int32_t *>(p);

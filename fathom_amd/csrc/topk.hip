@@ -1887,9 +1887,7 @@ int launch_select_keys(const uint32_t *samp, int64_t rows, int64_t samp_cap, int
       select_groups_kernel<4, false><<<g, kSelThreads, 0, st>>>(samp, samp_cap, ukk, urh, s);
     return launch_status("select_groups_kernel");
   }
-  if (samp_cap <= 8 * kSelThreads)
-    select_keys_kernel<8><<<g, kSelThreads, 0, st>>>(samp, samp_cap, ukk, urh, s);
-  else if (samp_cap <= 16 * kSelThreads)
+  if (samp_cap <= 16 * kSelThreads)  // the chains' rows sample 10240 keys or more
     select_keys_kernel<16><<<g, kSelThreads, 0, st>>>(samp, samp_cap, ukk, urh, s);
   else if (samp_cap <= 32 * kSelThreads)
     select_keys_kernel<32><<<g, kSelThreads, 0, st>>>(samp, samp_cap, ukk, urh, s);
@@ -1903,9 +1901,7 @@ int launch_select_groups(const uint32_t *gmax, int64_t rows, int64_t ng, int64_t
   if (ng > 4 * kSelThreads) return fail(FATHOM_ERR_INVALID, "select: %lld group maxima exceed %d", (long long)ng, 4 * kSelThreads);
   const unsigned g = (unsigned)rows;
   const uint32_t ukk = (uint32_t)kk, urh = (uint32_t)r_hi;
-  if (ng <= kSelThreads)
-    select_groups_kernel<1, true><<<g, kSelThreads, 0, st>>>(gmax, ng, ukk, urh, s);
-  else if (ng <= 2 * kSelThreads)
+  if (ng <= 2 * kSelThreads)  // the chain's rows have 1664 sampled maxima or more
     select_groups_kernel<2, true><<<g, kSelThreads, 0, st>>>(gmax, ng, ukk, urh, s);
   else
     select_groups_kernel<4, true><<<g, kSelThreads, 0, st>>>(gmax, ng, ukk, urh, s);
@@ -1967,27 +1963,37 @@ int launch_row_select(const float *scores, int64_t G, const uint32_t *gmax, int6
                     kGmaxWideMax == 32 * kFinThreads * kGroupTok,
                 "groups per thread");
   const int64_t kk = k - sink - local;
-  if (!group_select_takes(n, kk))
+  if (!group_select_takes(n, kk) || (ATTN && kk > kSelMaxK))
     return fail(FATHOM_ERR_INVALID, "row selection: n=%lld kk=%lld not taken", (long long)n, (long long)kk);
   const unsigned g = (unsigned)rows;
   const auto run = [&](auto kernel) { kernel<<<g, kFinThreads, 0, st>>>(scores, G, gmax, n, m, k, sink, local, idx, ra); };
-  const bool whole = rowrank_takes(n, kk);
-  if constexpr (!ATTN) {
-    if (kk > kSelMaxK && n > 4 * kFinThreads) {
-      if (whole && n <= 8 * kFinThreads) run(rowselect_kernel<Scores, false, true, 0, 8>);
-      else if (whole) run(rowselect_kernel<Scores, false, true, 0, 32>);
-      else if (n <= kGmaxSelectMax) run(rowselect_kernel<Scores, false, true, 8, 0>);
-      else run(rowselect_kernel<Scores, false, true, 32, 0>);
-      return launch_status("rowselect_kernel");
+  const bool wide = kk > kSelMaxK && n > 4 * kFinThreads;
+  if (n <= kRowSelectMax) {
+    if constexpr (!std::is_same<Scores, QuadScores>::value) {  // quad order: longer rows only
+      const bool whole = rowrank_takes(n, kk);
+      if (wide) {
+        if constexpr (!ATTN) {
+          if (whole && n <= 8 * kFinThreads) run(rowselect_kernel<Scores, false, true, 0, 8>);
+          else if (whole) run(rowselect_kernel<Scores, false, true, 0, 32>);
+          else run(rowselect_kernel<Scores, false, true, 8, 0>);
+        }
+      } else if (!whole) {
+        run(rowselect_kernel<Scores, ATTN, false, 2, 0>);
+      } else if (n <= kFinThreads) {
+        run(rowselect_kernel<Scores, ATTN, false, 0, 1>);
+      } else if (n <= 4 * kFinThreads) {
+        run(rowselect_kernel<Scores, ATTN, false, 0, 4>);
+      } else if (n <= 8 * kFinThreads) {
+        run(rowselect_kernel<Scores, ATTN, false, 0, 8>);
+      } else {
+        run(rowselect_kernel<Scores, ATTN, false, 0, 32>);
+      }
     }
-  }
-  if (whole) {
-    if (n <= kFinThreads) run(rowselect_kernel<Scores, ATTN, false, 0, 1>);
-    else if (n <= 4 * kFinThreads) run(rowselect_kernel<Scores, ATTN, false, 0, 4>);
-    else if (n <= 8 * kFinThreads) run(rowselect_kernel<Scores, ATTN, false, 0, 8>);
-    else run(rowselect_kernel<Scores, ATTN, false, 0, 32>);
-  } else if (n <= kRowSelectMax) {
-    run(rowselect_kernel<Scores, ATTN, false, 2, 0>);
+  } else if (wide) {
+    if constexpr (!ATTN) {
+      if (n <= kGmaxSelectMax) run(rowselect_kernel<Scores, false, true, 8, 0>);
+      else run(rowselect_kernel<Scores, false, true, 32, 0>);
+    }
   } else {
     run(rowselect_kernel<Scores, ATTN, false, 8, 0>);
   }
