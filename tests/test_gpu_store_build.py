@@ -14,21 +14,45 @@ DEV = torch.device("cuda")
 SDT = {"f16": torch.float16, "f32": torch.float32, "bf16": torch.bfloat16}
 
 
-def _edge_keys(BH, n, dtype, seed):
+def _edge_keys(BH, n, dtype, sdt, seed):
     """Random keys, and per channel the quotient's edges: multiples of the block's scale step and the representable
-    values next to them, both signs."""
+    values next to them, both signs; next to zero the smallest normal of 32-bit keys, whose denormals (a block that
+    holds one divides) come in the second block."""
     g = torch.Generator().manual_seed(seed)
     K = torch.randn(BH, n, 128, generator=g) * torch.exp(2 * torch.randn(BH, 1, 128, generator=g))
     K = K.to(dtype)
-    a = K.float().abs().reshape(BH, n, 128)[:, :64].amax(1)          # the first block's absmax
-    step = a.half().float() / 8
+    a = K.float().abs().reshape(BH, n, 128)[:, :64].amax(1)          # the first block's absmax,
+    K[:, 0] = a.to(dtype)                                            # kept past the rows below
+    step = a.to(SDT[sdt]).float() / 8
     m = torch.arange(-8, 9, dtype=torch.float32)
     at = (m[None, :, None] * step[:, None, :]).to(dtype)
     near = [at, torch.nextafter(at, torch.full_like(at, math.inf)), torch.nextafter(at, torch.full_like(at, -math.inf))]
     rows = torch.cat(near, 1)                                        # [BH, 51, 128]
     rows = torch.where(rows.float().abs() <= a[:, None], rows, torch.zeros((), dtype=dtype))
+    if n >= 128:
+        K[:, 64] = a.to(dtype)
+        K[:, 69:120] = rows                      # with 32-bit denormals
+    if dtype == torch.float32:
+        rows = torch.where((rows != 0) & (rows.abs() < 2.0 ** -126), 2.0 ** -126 * rows.sign(), rows)
     K[:, 5:56] = rows[:, :min(51, n - 5)]
     return K
+
+
+@pytest.mark.parametrize("sdt", ["f16", "bf16"])
+def test_edge_keys_reach_the_division_free_path(sdt):
+    """The first block of 32-bit edge keys has neither denormals nor scales that divide, and its quotients touch every
+    integer from both sides; the second has denormals."""
+    K = _edge_keys(1, 256, torch.float32, sdt, 3)
+    tiny = (K != 0) & (K.abs() < 2.0 ** -126)
+    assert not tiny[:, :64].any() and tiny[:, 64:128].any()
+    s = K[:, :64].abs().amax(1).to(SDT[sdt]).float() / 8
+    assert (8 * s >= 2.0 ** -14).all() and (8 * s <= 65504).all()
+    x, m = K[0, 5:56].double() / s[0].double(), torch.arange(-8.0, 9.0, dtype=torch.float64)
+    inside = (m[:, None] * s[0].double()).abs() < K[0, :64].abs().amax(0).double() * (1 - 2.0 ** -20)
+    for i in range(17):
+        at, up, down = x[i], x[17 + i], x[34 + i]
+        assert ((up > m[i]) | ~inside[i]).all() and ((down < m[i]) | ~inside[i]).all()
+        assert ((at - m[i]).abs()[inside[i]] <= 2.0 ** -22 * 8).all()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
@@ -39,7 +63,7 @@ def test_build_equals_oracle_at_tile_edges(BH, n, sub, sdt, dtype, monkeypatch):
     print(f"[build] {BH}x{n} sub={sub} {sdt} {dtype}", flush=True)
     nb = -(-n // 64)
     monkeypatch.setattr(bp, "SUB", sub or nb)
-    K = _edge_keys(BH, n, dtype, n)
+    K = _edge_keys(BH, n, dtype, sdt, n)
     if n > 500000:                          # the large shapes' rows repeat their head: the oracle is slow
         K[:, 8192:] = K[:, :8192].repeat(1, -(-n // 8192), 1)[:, 8192:n]
     st = bp.PlaneStore(K.to(DEV), scale_dtype=SDT[sdt])
