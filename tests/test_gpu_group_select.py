@@ -128,6 +128,49 @@ def test_staged_scan_of_plans_without_units(n, G, monkeypatch):
     assert torch.equal(got[64][0].cpu(), first.expand(2, G, 512))
 
 
+@pytest.mark.parametrize("n,G,k", [(160000, 4, 512), (160000, 7, 512), (300011, 4, 2084)])
+@pytest.mark.parametrize("sub", [16, 64])
+def test_rescan_of_a_misled_first_pass(n, G, k, sub, monkeypatch):
+    """The sampled tiles hold one high score per 16-token group, the others none: fewer than kk keys reach the first
+    pass's threshold (checked on the scores), and the row is rescanned with the lower one -- after a direct first pass
+    (superblocks of 16) and a staged one (of 64), with the plan given and made in the sample pass."""
+    print(f"[rescan] n={n} G={G} k={k} sub={sub}", flush=True)
+    monkeypatch.setattr(bp, "SUB", sub)
+    kk, tile = k - 36, 1024
+    ntiles = -(-n // tile)
+    want = max(32, -(-2 * k // 64), -(-32 * n // (5 * k * tile)))
+    S = -(-ntiles // min(want, 64))                       # every S-th tile is sampled
+    gen = torch.Generator().manual_seed(n)
+    tok = torch.arange(0, ntiles, S)[:, None] * tile + torch.arange(64) * 16
+    tok = (tok + torch.randint(0, 16, tok.shape, generator=gen)).flatten()
+    tok = tok[(tok >= 4) & (tok < n - 32)]
+    K = torch.randn(2, n, 128, generator=gen) * 0.01
+    sampled = sum(min(tile, n - t * S * tile) for t in range(-(-ntiles // S)))
+    r_hi = min(max(1, (5 * kk * sampled + 2 * n - 1) // (2 * n)), kk)
+    high = (r_hi + kk) // 2                               # high scores: the threshold's rank and more, fewer than kk
+    K[:, tok[torch.randperm(len(tok), generator=gen)[:high]], 0] = 3.0 + torch.rand(2, high, generator=gen)
+    K = K.to(DEV)
+    q = torch.zeros(2, G, 128, device=DEV)
+    q[..., 0], q[:, 1::2, 1] = 1.0, 0.5
+    gain = torch.ones(2, 128, device=DEV)
+    gain[:, 0], gain[:, 1] = 1000.0, 10.0
+    st = bp.PlaneStore(K, keep_code=False)
+    plan = bp.make_plan(gain, 6.0)
+    scores = st.scan(q, plan)
+    sc = scores.clone()
+    sc[..., :4], sc[..., n - 32:] = -math.inf, -math.inf
+    grp = torch.nn.functional.pad(sc, (0, ntiles * tile - n), value=-math.inf).view(2, G, ntiles, 64, 16)[:, :, ::S].amax(-1)
+    t_hi = grp.flatten(2).topk(r_hi, -1).values[..., -1:]
+    assert bool(((sc >= t_hi).sum(-1) < kk).any()) and r_hi < high < kk
+    want_idx = _oracle_topk(scores, k, 4, 32, n)
+    assert torch.equal(st.scan_topk(q, plan, k, 4, 32).cpu(), want_idx)
+    idx, t = st.plan_scan_topk(q, gain, 6.0, k, 4, 32, return_t=True)
+    assert torch.equal(idx.cpu(), want_idx) and torch.equal(t, plan["t"])
+    i2, out = st.plan_scan_topk_attention(q, gain, 6.0, k, K.bfloat16(), K.bfloat16(), 4, 32)
+    ref, _ = off.gather_attention(q, idx, n, K.bfloat16(), K.bfloat16(), n)
+    assert torch.equal(i2, idx) and torch.equal(out, ref)
+
+
 def _score_rows(kind, rows, n, seed):
     rng = np.random.default_rng(seed)
     s = rng.standard_normal((rows, n)).astype(np.float32)

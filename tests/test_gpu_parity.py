@@ -862,9 +862,10 @@ def test_scan_host_resident_paired_tiles(cfg, n, sub, G):
 
 
 def test_scan_topk_fallback_pass_host_paired():
-    """The fallback pass (direct tiles) after a staged first pass: a falling
-    row in a host-mapped store of 64-block superblocks."""
-    BH, d, n = 2, 128, 90000
+    """A falling row in a host-mapped store of 64-block superblocks, past the
+    lengths that are selected from group maxima: a staged first pass, with the
+    plan given and made in the sample pass."""
+    BH, d, n = 2, 128, 160000
     K = torch.zeros(BH, n, d)
     K[:, :, 0] = torch.linspace(1, -1, n)[None] * 3.0
     K[:, :, 1] = torch.randn(BH, n, generator=torch.Generator().manual_seed(5)) * 0.01
@@ -887,14 +888,16 @@ def test_scan_topk_fallback_pass_host_paired():
     try:
         st.planes32, st.scales_k = pl_dev, sc_dev
         got = st.scan_topk(q, plan, 512)
+        own = st.plan_scan_topk(q, g.to(DEV), 6.0, 512)
         torch.cuda.synchronize()
         torch.testing.assert_close(got, ref, rtol=0, atol=0)
+        torch.testing.assert_close(own, ref, rtol=0, atol=0)
     finally:
         off.free_host(hp1)
         off.free_host(hp2)
 
 
-@pytest.mark.parametrize("direction,n,BH,G", [(1.0, 90000, 2, 4), (-1.0, 90000, 2, 4), (1.0, 300000, 2, 4),
+@pytest.mark.parametrize("direction,n,BH,G", [(-1.0, 150000, 2, 8), (-1.0, 140000, 1, 3), (1.0, 150000, 2, 4), (1.0, 90000, 2, 4), (-1.0, 90000, 2, 4), (1.0, 300000, 2, 4),
                                                (-1.0, 200000, 8, 4), (-1.0, 90000, 2, 8), (-1.0, 40000, 1, 3)])
 def test_scan_topk_fallback_pass(direction, n, BH, G):
     """Fused path with scores falling (or rising) along the sequence: a falling
@@ -931,7 +934,7 @@ def test_scan_topk_stages_repeat(fallback):
     time it runs."""
     print(f"[fused-stages] fallback={fallback}", flush=True)
     if fallback:
-        BH, d, n = 2, 128, 90000
+        BH, d, n = 2, 128, 160000
         K = torch.zeros(BH, n, d)
         K[:, :, 0] = torch.linspace(3, -3, n)[None]
         K[:, :, 1] = torch.randn(BH, n, generator=torch.Generator().manual_seed(3)) * 0.01
