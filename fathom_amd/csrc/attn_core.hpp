@@ -208,12 +208,26 @@ __device__ __forceinline__ void attn_stream_block(const float *__restrict__ qg, 
 #pragma unroll
     for (int sh = 1; sh < NW; sh <<= 1) M = fmaxf(M, __shfl_xor(M, sh));
     const float ev = mv == -INFINITY ? 0.0f : expf(mv - M);  // a wave past k adds nothing
-    float L = 0.0f, O = 0.0f;
+    // summed by fours, then pairs: sixteen in a row round more often than the four
+    // merged splits of four waves that a head of 129 to 512 positions once took (mean relative error
+    // against 64 bits, k = 512: 2.58e-7 in a row, 2.49 the merged splits, 2.46 this way)
+    constexpr int kG = NW / 4;
+    float Lg[kG], Og[kG];
 #pragma unroll
-    for (int v = 0; v < NW; ++v) {
-      const float e = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ev), v));
-      L = fmaf(wl[v], e, L);
-      O = fmaf(wo[v][tid], e, O);
+    for (int i = 0; i < kG; ++i) {
+      Lg[i] = Og[i] = 0.0f;
+#pragma unroll
+      for (int v = 4 * i; v < 4 * i + 4; ++v) {
+        const float e = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ev), v));
+        Lg[i] = fmaf(wl[v], e, Lg[i]);
+        Og[i] = fmaf(wo[v][tid], e, Og[i]);
+      }
+    }
+    static_assert(kG == 1 || kG == 4, "waves of a workgroup");
+    float L = Lg[0], O = Og[0];
+    if constexpr (kG == 4) {
+      L = (Lg[0] + Lg[1]) + (Lg[2] + Lg[3]);
+      O = (Og[0] + Og[1]) + (Og[2] + Og[3]);
     }
     if (single) {
       out_row[tid] = O / L;
