@@ -338,8 +338,10 @@ class PlaneStore:
 
     def scan_topk(self, q, plan, k, sink=4, local=32, m=None):
         """Fused scan + sink/local top-k: the same int64 indices [BH, G, k] as
-        sink_local_topk(self.scan(q, plan), k, sink, local, m), without writing the
-        score tensor (the scan keeps only candidates above a sampled threshold)."""
+        sink_local_topk(self.scan(q, plan), k, sink, local, m).  Rows above 131072
+        tokens with k - sink - local up to 2048 are not written out (the scan keeps
+        only candidates above a sampled threshold); the scores of the others stay
+        in the call's workspace."""
         _need_gpu(q)
         BH, G, d = q.shape
         if BH != self.BH:
